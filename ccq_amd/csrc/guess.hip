@@ -13,9 +13,10 @@
 // FP32.  Loss: mean over samples of ((m / sm) r - y)^2 with y = (t_conv - m) / sm.
 //
 // Training (ccq_hip_mlp_train) runs on the GPU: per step a batch of samples
-// drawn by a counter-based hash, one thread per sample for forward and
-// backward (activations kept in a scratch buffer), one thread per parameter
-// summing the batch in a fixed order (deterministic), then an Adam step.
+// drawn by a counter-based hash, forward, backward and the workgroup's share
+// of the gradient in one kernel (one lane per hidden unit), then a kernel
+// that sums the workgroups' shares in a fixed order (deterministic) and does
+// the Adam step.
 // ccq has no counterpart (its guess is T = 0, src/calc_driver.f90:210-211).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -111,37 +112,6 @@ __global__ __launch_bounds__(256) void guess_msq(GuessBlock B, double* __restric
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// forward pass of one sample; weights (BF16-rounded) in LDS.  Returns r; with
-// keep != nullptr stores the rounded input, rounded h1, rounded h2 there.
-__device__ inline float mlp_forward(const float* __restrict__ w, const float (&xin)[F], float* keep) {
-  float x[F];
-#pragma unroll
-  for (int k = 0; k < F; ++k) x[k] = bf16r((xin[k] - w[P_MU + k]) / w[P_SD + k]);
-  float h1[H];
-#pragma unroll 8
-  for (int p = 0; p < H; ++p) {
-    float acc = w[P_B1 + p];
-#pragma unroll
-    for (int k = 0; k < F; ++k) acc += w[P_W1 + k * H + p] * x[k];
-    h1[p] = bf16r(tanhf(acc));
-  }
-  float out = w[P_B3];
-  for (int q = 0; q < H; ++q) {
-    float acc = w[P_B2 + q];
-#pragma unroll 16
-    for (int p = 0; p < H; ++p) acc += w[P_W2 + p * H + q] * h1[p];
-    const float h2 = bf16r(tanhf(acc));
-    if (keep) keep[F + H + q] = h2;
-    out += w[P_W3 + q] * h2;
-  }
-  if (keep) {
-#pragma unroll
-    for (int k = 0; k < F; ++k) keep[k] = x[k];
-    for (int p = 0; p < H; ++p) keep[F + p] = h1[p];
-  }
-  return out;
-}
-
 // weights into LDS, BF16-rounded (mu, sd and biases are kept in FP32)
 __device__ inline void load_weights(float* w, const float* __restrict__ params) {
   for (int k = threadIdx.x; k < kGuessParams; k += blockDim.x) {
@@ -151,10 +121,10 @@ __device__ inline void load_weights(float* w, const float* __restrict__ params) 
   __syncthreads();
 }
 
-// Inference of one sample per thread, the same operations in the same order
-// as mlp_forward, with the first hidden layer in LDS (hs: this thread's
-// column, stride kApplyThreads) instead of a per-thread array, which the
-// run-time indexed loops would otherwise place in scratch memory.
+// Inference of one sample per thread, with the first hidden layer in LDS
+// (hs: this thread's column, stride kApplyThreads) instead of a per-thread
+// array, which the run-time indexed loops would otherwise place in scratch
+// memory.  Every sum runs in index order, as in mlp_step.
 constexpr int kApplyThreads = 128;
 __device__ inline float mlp_infer(const float* __restrict__ w, const float (&xin)[F], float* hs) {
   float x[F];
@@ -260,9 +230,6 @@ hipError_t launch_guess_data(hipStream_t s, const GuessBlock& B, float* X, float
 // ---------------------------------------------------------------------------
 // training
 
-constexpr int KEEP = F + 2 * H;           // rounded x, h1, h2 of a sample
-constexpr int SCR = KEEP + 2 * H + 2;     // + gh1, gh2, g_out, e^2
-
 __device__ inline uint64_t mix64(uint64_t z) {
   z += 0x9E3779B97F4A7C15ull;
   z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -270,96 +237,237 @@ __device__ inline uint64_t mix64(uint64_t z) {
   return z ^ (z >> 31);
 }
 
-// one thread per sample of the batch: forward, loss and the back-propagated
-// signals gh1, gh2, g_out (activations in scr[s][...])
-__global__ __launch_bounds__(256) void mlp_fwd_bwd(const float* __restrict__ params,
-                                                   const float* __restrict__ X,
-                                                   const float* __restrict__ Mv,
-                                                   const float* __restrict__ Yv, int64_t n,
-                                                   int64_t batch, uint64_t seed, int64_t step,
-                                                   int full, float* __restrict__ scr) {
-  __shared__ float w[kGuessParams];
-  load_weights(w, params);
-  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= batch) return;
-  const int64_t idx = full ? s : (int64_t)(mix64(seed ^ mix64((uint64_t)step * 0x100000001ull + s)) %
-                                           (uint64_t)n);
-  float x[F];
-#pragma unroll
-  for (int k = 0; k < F; ++k) x[k] = X[idx * F + k];
-  float* q = scr + s * SCR;
-  const float r = mlp_forward(w, x, q);
-  const float mm = Mv[idx];
-  const float e = mm * r - Yv[idx];
-  const float g = 2.0f * e * mm / (float)batch;
-  q[KEEP + 2 * H] = g;
-  q[KEEP + 2 * H + 1] = e * e;
-  // gh2 = g W3 (1 - h2^2); gh1 = (W2 gh2) (1 - h1^2)
-  float gh2[H];
-  for (int qq = 0; qq < H; ++qq) {
-    const float h2 = q[F + H + qq];
-    gh2[qq] = g * w[P_W3 + qq] * (1.0f - h2 * h2);
-    q[KEEP + H + qq] = gh2[qq];
-  }
-  for (int p = 0; p < H; ++p) {
-    float acc = 0.0f;
-#pragma unroll 16
-    for (int qq = 0; qq < H; ++qq) acc += w[P_W2 + p * H + qq] * gh2[qq];
-    const float h1 = q[F + p];
-    q[KEEP + p] = acc * (1.0f - h1 * h1);
-  }
-}
+// Forward, backward and gradient of kStepTile samples at a time per workgroup.
+// A lane is a hidden unit and a wave carries four samples, so the 64-long sums
+// read the weights once per four samples, the activations stay in LDS, and
+// 4096 samples fill 256 workgroups (a thread per sample filled 16).  The
+// gradient is the outer product of activations and signals: a thread owns a
+// 4 x 4 tile of W2 and up to three of the other entries, in FP64; each
+// workgroup stores its share (partial[block][k]) and mlp_reduce sums them.
+// Bound by the latency of the six phases.  Batch 4096: 275 us (a thread per
+// sample, activations through memory) + 1687 us (a thread per parameter,
+// serial over the batch) before, 22 us + 5.7 us (mlp_reduce) now.
+constexpr int kStepThreads = 256;
+constexpr int kStepTile = 16;       // samples of one pass
+constexpr int kStepBlocks = 256;    // most workgroups (one pass each at batch 4096)
+constexpr int kW2P = H + 1;         // W2 rows and columns both read without bank conflicts
+constexpr int kActP = H + 4;        // row pitch of the samples' activations, 16-byte aligned
+constexpr int kGradN = kGuessParams + 1;   // gradient and loss (mu, sd entries unused)
+constexpr int kExtra = (kGradN - P_W1 - H * H + kStepThreads - 1) / kStepThreads;
 
-// one thread per parameter (and one for the loss): sum over the batch in
-// sample order.  grad[k] for k < kGuessParams (mu / sd get 0), grad[kGuessParams] = loss.
-__global__ __launch_bounds__(256) void mlp_grad(const float* __restrict__ scr, int64_t batch,
-                                                float* __restrict__ grad) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k > kGuessParams) return;
-  double acc = 0.0;
-  if (k == kGuessParams) {
-    for (int64_t s = 0; s < batch; ++s) acc += scr[s * SCR + KEEP + 2 * H + 1];
-    grad[k] = (float)(acc / (double)batch);
-    return;
-  }
-  int a = -1, b = -1;   // gradient = sum_s act[a] * sig[b] (a = -1: sig alone)
-  if (k < P_W1) {
-    grad[k] = 0.0f;
-    return;
-  } else if (k < P_B1) {
-    const int kk = (k - P_W1) / H, p = (k - P_W1) % H;
-    a = kk;                 // rounded input x[kk]
-    b = KEEP + p;           // gh1[p]
+// gradient entry k as sum_s act[s][a] * sig[s][b]; columns of a sample's row:
+// x (F), 1, h1, h2, gh1, gh2, g, e^2
+constexpr int C_X = 0, C_ONE = F, C_H1 = 8, C_H2 = C_H1 + kActP, C_G1 = C_H2 + kActP, C_G2 = C_G1 + kActP,
+              C_G = C_G2 + kActP, C_E = C_G + 1, kRow = C_G + 4;
+__device__ inline void grad_columns(int k, int& a, int& b) {
+  if (k < P_B1) {
+    a = C_X + (k - P_W1) / H;
+    b = C_G1 + (k - P_W1) % H;
   } else if (k < P_W2) {
-    b = KEEP + (k - P_B1);
-  } else if (k < P_B2) {
-    const int p = (k - P_W2) / H, qq = (k - P_W2) % H;
-    a = F + p;              // h1[p]
-    b = KEEP + H + qq;      // gh2[q]
+    a = C_ONE;
+    b = C_G1 + (k - P_B1);
   } else if (k < P_W3) {
-    b = KEEP + H + (k - P_B2);
+    a = C_ONE;
+    b = C_G2 + (k - P_B2);
   } else if (k < P_B3) {
-    a = F + H + (k - P_W3); // h2[q]
-    b = KEEP + 2 * H;       // g_out
+    a = C_H2 + (k - P_W3);
+    b = C_G;
   } else {
-    b = KEEP + 2 * H;
+    a = C_ONE;
+    b = k == P_B3 ? C_G : C_E;
   }
-  for (int64_t s = 0; s < batch; ++s) {
-    const float* q = scr + s * SCR;
-    acc += a >= 0 ? (double)q[a] * (double)q[b] : (double)q[b];
-  }
-  grad[k] = (float)acc;
 }
 
-__global__ __launch_bounds__(256) void mlp_adam(float* __restrict__ params, const float* __restrict__ grad,
-                                                float* __restrict__ m1, float* __restrict__ m2, float lr,
-                                                float c1, float c2) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < P_W1 || k >= kGuessParams) return;
-  const float g = grad[k];
-  m1[k] = 0.9f * m1[k] + 0.1f * g;
-  m2[k] = 0.999f * m2[k] + 0.001f * g * g;
-  params[k] -= lr * (m1[k] / c1) / (sqrtf(m2[k] / c2) + 1e-8f);
+__global__ __launch_bounds__(kStepThreads) void mlp_step(const float* __restrict__ params,
+                                                         const float* __restrict__ X,
+                                                         const float* __restrict__ Mv,
+                                                         const float* __restrict__ Yv, int64_t n,
+                                                         int64_t batch, uint64_t seed, int64_t step, int full,
+                                                         double* __restrict__ partial) {
+  __shared__ __align__(16) float rows[kStepTile * kRow];
+  __shared__ float w2[H * kW2P];
+  __shared__ float w[kGuessParams - H * H];   // the other parameters, in order
+  auto at = [](int k) { return k < P_W2 ? k : k - H * H; };
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int k = tid; k < kGuessParams; k += kStepThreads) {
+    const bool wt = (k >= P_W1 && k < P_B1) || (k >= P_W2 && k < P_B2) || (k >= P_W3 && k < P_B3);
+    const float v = wt ? bf16r(params[k]) : params[k];
+    if (k >= P_W2 && k < P_B2) w2[(k - P_W2) / H * kW2P + (k - P_W2) % H] = v;
+    else w[at(k)] = v;
+  }
+  const int p0 = (tid >> 4) * 4, q0 = (tid & 15) * 4;
+  double acc[4][4], ext[kExtra];
+  int ea[kExtra], eb[kExtra];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
+#pragma unroll
+  for (int x = 0; x < kExtra; ++x) {
+    ext[x] = 0.0;
+    // entry number tid + x kStepThreads of those outside W2
+    const int e = P_W1 + tid + x * kStepThreads;
+    const int k = e < P_W2 ? e : e + H * H;
+    ea[x] = eb[x] = -1;
+    if (k < kGradN) grad_columns(k, ea[x], eb[x]);
+  }
+
+  for (int64_t s0 = (int64_t)blockIdx.x * kStepTile; s0 < batch; s0 += (int64_t)gridDim.x * kStepTile) {
+    auto sample = [&](int s) -> int64_t {
+      return full ? s0 + s : (int64_t)(mix64(seed ^ mix64((uint64_t)step * 0x100000001ull + (uint64_t)(s0 + s))) %
+                                       (uint64_t)n);
+    };
+    __syncthreads();   // the weights are in; the previous pass's rows are read
+    if (tid < kStepTile * F) {
+      const int s = tid / F, k = tid % F;
+      float x = 0.0f;
+      if (s0 + s < batch) x = bf16r((X[sample(s) * F + k] - w[P_MU + k]) / w[P_SD + k]);
+      rows[s * kRow + C_X + k] = x;
+      if (k == 0) rows[s * kRow + C_ONE] = 1.0f;
+    }
+    __syncthreads();
+    float* r0 = rows + wave * 4 * kRow;   // this wave's four samples
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float* r = r0 + i * kRow;
+      float a = w[P_B1 + lane];
+#pragma unroll
+      for (int k = 0; k < F; ++k) a += w[P_W1 + k * H + lane] * r[C_X + k];
+      r[C_H1 + lane] = bf16r(tanhf(a));
+    }
+    __syncthreads();
+    {
+      float a[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = w[at(P_B2) + lane];
+#pragma unroll 4
+      for (int p = 0; p < H; p += 4) {
+        float4 h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = *reinterpret_cast<const float4*>(r0 + i * kRow + C_H1 + p);
+        const float u0 = w2[p * kW2P + lane], u1 = w2[(p + 1) * kW2P + lane], u2 = w2[(p + 2) * kW2P + lane],
+                    u3 = w2[(p + 3) * kW2P + lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a[i] += u0 * h[i].x;
+          a[i] += u1 * h[i].y;
+          a[i] += u2 * h[i].z;
+          a[i] += u3 * h[i].w;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) r0[i * kRow + C_H2 + lane] = bf16r(tanhf(a[i]));
+    }
+    __syncthreads();
+    if (tid < kStepTile) {
+      float* r = rows + tid * kRow;
+      float out = w[at(P_B3)];
+      for (int q = 0; q < H; ++q) out += w[at(P_W3) + q] * r[C_H2 + q];
+      float g = 0.0f, e2 = 0.0f;
+      if (s0 + tid < batch) {
+        const int64_t idx = sample(tid);
+        const float mm = Mv[idx];
+        const float e = mm * out - Yv[idx];
+        g = 2.0f * e * mm / (float)batch;
+        e2 = e * e;
+      }
+      r[C_G] = g;
+      r[C_E] = e2;
+    }
+    __syncthreads();
+    // gh2 = g W3 (1 - h2^2); gh1 = (W2 gh2) (1 - h1^2)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float* r = r0 + i * kRow;
+      const float h2 = r[C_H2 + lane];
+      r[C_G2 + lane] = r[C_G] * w[at(P_W3) + lane] * (1.0f - h2 * h2);
+    }
+    __syncthreads();
+    {
+      float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+      for (int q = 0; q < H; q += 4) {
+        float4 h[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = *reinterpret_cast<const float4*>(r0 + i * kRow + C_G2 + q);
+        const float* u = w2 + lane * kW2P + q;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          a[i] += u[0] * h[i].x;
+          a[i] += u[1] * h[i].y;
+          a[i] += u[2] * h[i].z;
+          a[i] += u[3] * h[i].w;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float* r = r0 + i * kRow;
+        const float h1 = r[C_H1 + lane];
+        r[C_G1 + lane] = a[i] * (1.0f - h1 * h1);
+      }
+    }
+    __syncthreads();
+    for (int s = 0; s < kStepTile; ++s) {
+      const float* r = rows + s * kRow;
+      const float4 h = *reinterpret_cast<const float4*>(r + C_H1 + p0);
+      const float4 g = *reinterpret_cast<const float4*>(r + C_G2 + q0);
+      const double hd[4] = {h.x, h.y, h.z, h.w}, gd[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] += hd[i] * gd[j];
+#pragma unroll
+      for (int x = 0; x < kExtra; ++x)
+        if (ea[x] >= 0) ext[x] += (double)r[ea[x]] * (double)r[eb[x]];
+    }
+  }
+
+  double* out = partial + (int64_t)blockIdx.x * kGradN;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) out[P_W2 + (p0 + i) * H + q0 + j] = acc[i][j];
+#pragma unroll
+  for (int x = 0; x < kExtra; ++x) {
+    const int e = P_W1 + tid + x * kStepThreads;
+    const int k = e < P_W2 ? e : e + H * H;
+    if (k < kGradN) out[k] = ext[x];
+  }
+}
+
+// workgroups of mlp_step for a batch
+static int step_blocks(int64_t batch) {
+  const int64_t b = (batch + kStepTile - 1) / kStepTile;
+  return (int)(b < kStepBlocks ? b : kStepBlocks);
+}
+
+// grad[k] = sum over the workgroups' shares in order (mu / sd get 0),
+// grad[kGuessParams] = loss; with adam set, the Adam step of that gradient.
+// A lane per entry, the shares in four runs (one per wave) added in order.
+__global__ __launch_bounds__(256) void mlp_reduce(const double* __restrict__ partial, int blocks, int64_t batch,
+                                                  float* __restrict__ grad, int adam, float* __restrict__ params,
+                                                  float* __restrict__ m1, float* __restrict__ m2, float lr, float c1,
+                                                  float c2) {
+  __shared__ double red[3][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int k = blockIdx.x * 64 + lane;
+  const int per = (blocks + 3) / 4, lo = wave * per, hi = lo + per < blocks ? lo + per : blocks;
+  double acc = 0.0;
+  if (k >= P_W1 && k < kGradN) {
+#pragma unroll 8
+    for (int b = lo; b < hi; ++b) acc += partial[(int64_t)b * kGradN + k];
+  }
+  if (wave) red[wave - 1][lane] = acc;
+  __syncthreads();
+  if (wave || k >= kGradN) return;
+  acc = ((acc + red[0][lane]) + red[1][lane]) + red[2][lane];
+  const float g = (float)(k == kGuessParams ? acc / (double)batch : acc);
+  grad[k] = g;
+  if (!adam || k < P_W1 || k >= kGuessParams) return;
+  const float a = 0.9f * m1[k] + 0.1f * g, b = 0.999f * m2[k] + 0.001f * g * g;
+  m1[k] = a;
+  m2[k] = b;
+  params[k] -= lr * (a / c1) / (sqrtf(b / c2) + 1e-8f);
 }
 
 }  // namespace ccqk
@@ -390,16 +498,21 @@ struct DevF {
     }                                                                      \
   } while (0)
 
-// loss and gradient over all n samples (device buffers; scr holds n * SCR
-// floats, grad kGuessParams + 1), on the null stream
-hipError_t launch_full_grad(const float* P, const float* X, const float* M, const float* Y,
-                            int64_t n, float* scr, float* grad) {
+// loss and gradient of one batch (device buffers; partial holds
+// step_blocks(batch) * kGradN doubles, grad kGradN floats), on the null stream;
+// full: the batch is samples 0 .. batch - 1, else drawn by (seed, step).  With
+// m1, the Adam step of that gradient follows (bias corrections c1, c2).
+hipError_t launch_step(float* P, const float* X, const float* M, const float* Y, int64_t n, int64_t batch,
+                       uint64_t seed, int64_t step, int full, double* partial, float* grad, float* m1 = nullptr,
+                       float* m2 = nullptr, float lr = 0.0f, float c1 = 1.0f, float c2 = 1.0f) {
   using namespace ccqk;
-  hipLaunchKernelGGL(mlp_fwd_bwd, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, 0, P, X, M, Y,
-                     n, n, (uint64_t)0, (int64_t)0, 1, scr);
+  const int blocks = step_blocks(batch);
+  hipLaunchKernelGGL(mlp_step, dim3(blocks), dim3(kStepThreads), 0, 0, P, X, M, Y, n, batch, seed, step, full,
+                     partial);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(mlp_grad, dim3((kGuessParams + 1 + 255) / 256), dim3(256), 0, 0, scr, n, grad);
+  hipLaunchKernelGGL(mlp_reduce, dim3((kGradN + 63) / 64), dim3(256), 0, 0, partial, blocks, batch, grad,
+                     m1 ? 1 : 0, P, m1, m2, lr, c1, c2);
   return hipGetLastError();
 }
 
@@ -415,8 +528,9 @@ int run_training(const float* X, const float* M, const float* Y, int64_t n, floa
     g_guess_err = "bad sample / batch count";
     return 2;
   }
-  DevF dX(n * F), dM(n), dY(n), dP(kGuessParams), dG(kGuessParams + 1), dm1(kGuessParams),
-      dm2(kGuessParams), dS(batch * SCR);
+  DevF dX(n * F), dM(n), dY(n), dP(kGuessParams), dG(kGradN), dm1(kGuessParams), dm2(kGuessParams),
+      dS((int64_t)2 * step_blocks(batch) * kGradN);
+  double* part = reinterpret_cast<double*>(dS.p);
   if (!dX.p || !dM.p || !dY.p || !dP.p || !dG.p || !dm1.p || !dm2.p || !dS.p) {
     g_guess_err = "out of device memory";
     return 1;
@@ -427,24 +541,16 @@ int run_training(const float* X, const float* M, const float* Y, int64_t n, floa
   GCHK(hipMemcpy(dP.p, params, sizeof(float) * kGuessParams, hipMemcpyHostToDevice));
   GCHK(hipMemset(dm1.p, 0, sizeof(float) * kGuessParams));
   GCHK(hipMemset(dm2.p, 0, sizeof(float) * kGuessParams));
-  const dim3 gp((kGuessParams + 1 + 255) / 256);
   if (grad_out) {
-    GCHK(launch_full_grad(dP.p, dX.p, dM.p, dY.p, n, dS.p, dG.p));
+    GCHK(launch_step(dP.p, dX.p, dM.p, dY.p, n, n, 0, 0, 1, part, dG.p));
     steps = 0;
   }
-  const dim3 gb((unsigned)((batch + 255) / 256));
   double b1 = 1.0, b2 = 1.0;
   for (int64_t st = 0; st < steps; ++st) {
-    hipLaunchKernelGGL(mlp_fwd_bwd, gb, dim3(256), 0, 0, dP.p, dX.p, dM.p, dY.p, n, batch, seed, st,
-                       0, dS.p);
-    GCHK(hipGetLastError());
-    hipLaunchKernelGGL(mlp_grad, gp, dim3(256), 0, 0, dS.p, batch, dG.p);
-    GCHK(hipGetLastError());
     b1 *= 0.9;
     b2 *= 0.999;
-    hipLaunchKernelGGL(mlp_adam, gp, dim3(256), 0, 0, dP.p, dG.p, dm1.p, dm2.p, (float)lr,
-                       (float)(1.0 - b1), (float)(1.0 - b2));
-    GCHK(hipGetLastError());
+    GCHK(launch_step(dP.p, dX.p, dM.p, dY.p, n, batch, seed, st, 0, part, dG.p, dm1.p, dm2.p, (float)lr,
+                     (float)(1.0 - b1), (float)(1.0 - b2)));
   }
   float loss = 0.0f;
   GCHK(hipMemcpy(&loss, dG.p + kGuessParams, sizeof(float), hipMemcpyDeviceToHost));
@@ -457,8 +563,8 @@ int run_training(const float* X, const float* M, const float* Y, int64_t n, floa
 
 // ---------------------------------------------------------------------------
 // Gradient without device allocation: every device buffer of the gradient
-// (the staged samples and parameters, the per-sample activations and
-// signals, the gradient and loss) lives in one file-scope array.  Each GPU
+// (the staged samples and parameters, the workgroups' shares, the gradient
+// and loss) lives in one file-scope array.  Each GPU
 // holds its own copy until the process ends; its address is looked up once
 // per device and used for every kernel argument and copy.
 
@@ -468,8 +574,8 @@ constexpr int64_t kNaM = kNaX + kNaMax * ccqk::F;             // M[n]
 constexpr int64_t kNaY = kNaM + kNaMax;                       // Y[n]
 constexpr int64_t kNaP = kNaY + kNaMax;                       // params
 constexpr int64_t kNaG = kNaP + 64 * ((ccqk::kGuessParams + 63) / 64);        // grad + loss
-constexpr int64_t kNaS = kNaG + 64 * ((ccqk::kGuessParams + 1 + 63) / 64);    // scr[n][SCR]
-constexpr int64_t kNaFloats = kNaS + kNaMax * ccqk::SCR;
+constexpr int64_t kNaS = kNaG + 64 * ((ccqk::kGradN + 63) / 64);              // shares (doubles)
+constexpr int64_t kNaFloats = kNaS + 2 * (int64_t)ccqk::kStepBlocks * ccqk::kGradN;
 
 constexpr int kNaDevices = 64;
 std::mutex g_na_mu;
@@ -528,7 +634,8 @@ int ccq_hip_mlp_grad_noalloc(const float* X, const float* M, const float* Y, int
   GCHK(hipMemcpy(s + kNaM, M, sizeof(float) * n, hipMemcpyHostToDevice));
   GCHK(hipMemcpy(s + kNaY, Y, sizeof(float) * n, hipMemcpyHostToDevice));
   GCHK(hipMemcpy(s + kNaP, params, sizeof(float) * kGuessParams, hipMemcpyHostToDevice));
-  GCHK(launch_full_grad(s + kNaP, s + kNaX, s + kNaM, s + kNaY, n, s + kNaS, s + kNaG));
+  GCHK(launch_step(s + kNaP, s + kNaX, s + kNaM, s + kNaY, n, n, 0, 0, 1, reinterpret_cast<double*>(s + kNaS),
+                   s + kNaG));
   float l = 0.0f;
   GCHK(hipMemcpy(&l, s + kNaG + kGuessParams, sizeof(float), hipMemcpyDeviceToHost));
   GCHK(hipMemcpy(grad, s + kNaG, sizeof(float) * kGuessParams, hipMemcpyDeviceToHost));

@@ -213,7 +213,7 @@ int ccq_hip_mlp_grad(const float* X, const float* M, const float* Y, int64_t n,
  * for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments, kernels and results as ccq_hip_mlp_grad; every device buffer
- * is a static per-GPU array of about 9 MB held until the process ends, so
+ * is a static per-GPU array of about 10 MB held until the process ends, so
  * n is limited to CCQ_HIP_MLP_NOALLOC_MAX_SAMPLES (larger n returns 2 and
  * leaves the GPU untouched).  Calls that overlap on one GPU race (they share
  * that array). */

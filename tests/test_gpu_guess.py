@@ -170,3 +170,19 @@ def test_learned_guess_gains_over_mp2(n, o, seed):
     assert it_ml < it_mp2
     assert abs(e_ml - e_conv) < 1e-9 and abs(e_mp2 - e_conv) < 1e-9
     eng.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 4095, 4097])
+def test_gradient_at_workgroup_edges(n):
+    """Sample counts around the 16-sample passes and the 256-workgroup limit.
+    An FP32 sum may round one activation to the other BF16 neighbour (2^-8 of
+    it), which moves a gradient entry by at most that much: 2^-6 leaves room
+    for a few of them in the single-sample case."""
+    _say(f"case gradient of {n} samples")
+    X, M, Y = _data(21, n)
+    p = GS.init_params(_data(22)[0], seed=23)
+    loss, g = GS.grad(X, M, Y, p)
+    lw, gw = mlp.loss_grad(p.astype(np.float64), X, M, Y, rounding=True)
+    assert abs(loss - lw) <= 2.0 ** -6 * lw
+    assert np.abs(g - gw).max() <= 2.0 ** -6 * np.abs(gw).max()
+    assert not g[:10].any()
