@@ -1170,6 +1170,17 @@ struct ccq_hip_ctx {
     return s;
   }
 
+  // largest offset of an operand's rows and summed indices, with a slab (at
+  // most 32 indices) past the end, which the tile loader's offsets may name
+  static int64_t reach(const std::vector<int64_t>& rows, const std::vector<int64_t>& ks, int64_t aff) {
+    auto top = [](const std::vector<int64_t>& t) { return t.empty() ? 0 : *std::max_element(t.begin(), t.end()); };
+    return top(rows) + top(ks) + 32 * std::max<int64_t>(aff, 1);
+  }
+  // operands whose last element lies at 4 GiB or beyond need 64-bit addresses
+  // in the tile kernel (CCQ_HIP_WIDE=1: all of them do)
+  static constexpr int64_t kWideElems = ((int64_t)1 << 32) / (int64_t)sizeof(double);
+  bool wide_all = false;
+
   static std::string plan_tag(const ccqk::GemmArgs& g) {
     std::string t;
     if (g.kind == 1)
@@ -1544,6 +1555,7 @@ struct ccq_hip_ctx {
                       : (!ns.empty() && stride_of(B, op.lb, ns.back()) == 1 ? 0 : 1));
           g.kA_aff = affine_stride(kAp);
           g.kB_aff = affine_stride(kBp);
+          g.wide = wide_all || reach(rA, kAp, g.kA_aff) >= kWideElems || reach(cB, kBp, g.kB_aff) >= kWideElems;
           // C contiguous along m (n): its fastest m (n) label has stride 1,
           // so consecutive rows (columns) are adjacent in runs of that extent
           g.c_mfast = !ms.empty() && stride_of(C, op.lc, ms.back()) == 1 ? 1 : 0;
@@ -1586,7 +1598,7 @@ struct ccq_hip_ctx {
               gp.ksplit = 1;
               gp.bm = mmax >= 96 ? 64 : 32;
               gp.bn = nmax >= 96 ? 64 : 32;
-              gp.bk = 32;
+              gp.bk = ccqk::tile_bk(gp.bm, gp.bn);
               gp.nsplit = 1;
               gp.kchunk = gp.K;
               planned[q].gplan = gp;
@@ -1786,7 +1798,7 @@ struct ccq_hip_ctx {
         if (!ops[i].fused) live.push_back(i);
       for (size_t p = 0; p < live.size();) {
         const Op& h = ops[live[p]];
-        if (!eligible(live[p]) || h.plan.nsplit < 2) {
+        if (!eligible(live[p]) || (h.plan.nsplit < 2 && ccqk::gemm_tiles(h.plan) >= kGroupTiles)) {
           ++p;
           continue;
         }
@@ -1817,12 +1829,11 @@ struct ccq_hip_ctx {
         cp.K = ktot;
         cp.kA_aff = cp.kB_aff = -1;
         ccqk::gemm_plan(cp, kWsCap);
-        // (the chain kernel spills registers with tiles above 64 x 64)
-        if (cp.kind != 0 || cp.bm * cp.bn > 64 * 64) {
+        if (cp.kind != 0) {
           ++p;
           continue;
         }
-        cp.bk = 32;
+        cp.bk = ccqk::tile_bk(cp.bm, cp.bn);
         cp.ksplit = 1;
         ws_need = std::max<int64_t>(ws_need, ccqk::gemm_ws_need(cp));
         const int c = (int)sec.chains.size();
@@ -1842,12 +1853,12 @@ struct ccq_hip_ctx {
     const Op& h = sec.ops[mem[0]];
     std::string t = "gemm:" + std::to_string(mem.size()) + "*" + std::to_string(h.M) + "x" +
                     std::to_string(h.N) + "x" + std::to_string(cp.K / (int64_t)mem.size());
-    return t + "/" + std::to_string(cp.bm) + "x" + std::to_string(cp.bn) + "k32s" +
+    return t + "/" + std::to_string(cp.bm) + "x" + std::to_string(cp.bn) + "k" + std::to_string(cp.bk) + "s" +
            std::to_string(cp.nsplit) + (cp.trans ? "t" : "") + "c";
   }
 
   // entries of a chain, oriented like its first member run with trans
-  // (1: the whole chain transposed), tile bm x bn, BK 32
+  // (1: the whole chain transposed), tile bm x bn
   void chain_entries(const Section& sec, int c, int trans, int bm, int bn, ccqk::GemmArgs* es) const {
     const auto& mem = sec.chains[c];
     for (size_t k = 0; k < mem.size(); ++k) {
@@ -1855,7 +1866,7 @@ struct ccq_hip_ctx {
       es[k].kind = 0;
       es[k].bm = bm;
       es[k].bn = bn;
-      es[k].bk = 32;
+      es[k].bk = ccqk::tile_bk(bm, bn);
       es[k].ksplit = 1;
       es[k].nsplit = 1;
       es[k].kchunk = es[k].K;
@@ -1899,6 +1910,9 @@ struct ccq_hip_ctx {
   int part_count = 0;
   bool dump_schedule = false;   // CCQ_HIP_SCHEDULE=1: levels and launches to stderr
   static constexpr int64_t kGroupTiles = 512;   // below this a GEMM joins groups
+  // a member runs its whole K: longer ones are faster split (8100 x 100 x 8100
+  // with two 900 x 100 x 8100: 553 us grouped, 480 us as split launches)
+  static constexpr int64_t kGroupMaxK = 4096;
   // products with K >= group_min_k join groups; small register-direct
   // products (K <= 2048, M N <= 65536) join as 32 x 32 tile members
   // (CCQ_HIP_GROUP_MINK, CCQ_HIP_GROUP_REG=0; both cut launches of the
@@ -1915,8 +1929,7 @@ struct ccq_hip_ctx {
     return {b, b + sizeof(double) * (uintptr_t)std::max<int64_t>(n, 1)};
   }
 
-  // the op's plan as a member of a grouped launch: its tile, full K in
-  // 32-deep slabs, no split
+  // the op's plan as a member of a grouped launch: its tile, full K, no split
   static ccqk::GemmArgs group_plan(const Op& op) {
     if (op.has_gplan) return op.gplan;
     ccqk::GemmArgs g = op.plan;
@@ -1929,7 +1942,7 @@ struct ccq_hip_ctx {
     }
     g.nsplit = 1;
     g.kchunk = g.K;
-    if (g.kind == 0 && g.ksplit == 1) g.bk = 32;
+    if (g.kind == 0 && g.ksplit == 1) g.bk = ccqk::tile_bk(g.bm, g.bn);
     return g;
   }
 
@@ -2021,7 +2034,7 @@ struct ccq_hip_ctx {
         for (int i : here) {
           const Op& op = sec.ops[i];
           if (grouped.count(i)) continue;
-          if (!op.gemm || op.chain >= 0 || op.K < group_min_k) continue;
+          if (!op.gemm || op.chain >= 0 || op.K < group_min_k || op.K > kGroupMaxK) continue;
           if (op.plan.kind != 0 && !(group_reg && op.K <= 2048 && op.M * op.N <= 65536)) continue;
           const ccqk::GemmArgs g = group_plan(op);
           if (ccqk::gemm_tiles(g) >= kGroupTiles) continue;
@@ -3113,6 +3126,7 @@ int ccq_hip_create(const ccq_hip_dims* dims, const ccq_hip_opts* opts, ccq_hip_c
     if (const char* g = std::getenv("CCQ_HIP_TUNE32")) ctx->tune32 = std::string(g) != "0";
     if (const char* g = std::getenv("CCQ_HIP_GROUP_MINK")) ctx->group_min_k = std::max(1, std::atoi(g));
     if (const char* g = std::getenv("CCQ_HIP_GROUP_REG")) ctx->group_reg = std::string(g) != "0";
+    if (const char* g = std::getenv("CCQ_HIP_WIDE")) ctx->wide_all = std::string(g) == "1";
     if (const char* g = std::getenv("CCQ_HIP_MERGE")) ctx->merge_sections = std::string(g) != "0";
     if (const char* g = std::getenv("CCQ_HIP_STREAMS"))
       ctx->nstreams = std::max(1, std::min(ccq_hip_ctx::kMaxStreams, std::atoi(g)));

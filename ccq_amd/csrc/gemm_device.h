@@ -138,72 +138,135 @@ __device__ __forceinline__ void store_partial(const GemmArgs& g, int z, int64_t 
   g.ws[((int64_t)z * g.M + m) * g.N + n] = v;
 }
 
-// LDS tile of an operand: R x BK values of type T.  KF (k-fastest in global
-// memory): stored row-major [R][BK+P] so a 16-lane group writing consecutive
-// k and the MFMA fragment read (16 consecutive rows, one k) are bank-conflict
-// free; otherwise stored k-major [BK][R+Q].  FP64: P = 1, Q = 2.  FP32 (four
-// k per fragment read by the four 16-lane groups): P = 4 makes the row pitch
-// 4 mod 16 words apart and Q = 16 puts the four k rows 16 banks apart, so the
-// 64 lanes of one fragment read hit 64 distinct banks.
-template <typename T, int R, bool KF, int BK>
+// LDS tile of an operand: R rows of BK values of type T, pitch BK + P, whatever
+// the operand's layout in memory.  P keeps rows on pairs of values (the
+// loader writes and the fragments read two consecutive k at a time) and
+// spreads the 16 rows of a fragment read over all 64 banks: FP64 pitch
+// 18 / 34 pairs of words 4 apart mod 64, FP32 pitch 20 / 36.
+template <typename T, int R, int BK>
 struct LdsTile {
-  static constexpr int P = sizeof(T) == 8 ? 1 : 4;
-  static constexpr int Q = sizeof(T) == 8 ? 2 : 16;
-  static constexpr int size = KF ? R * (BK + P) : BK * (R + Q);
-  __device__ static int at(int row, int k) { return KF ? row * (BK + P) + k : k * (R + Q) + row; }
+  static constexpr int pitch = BK + (sizeof(T) == 8 ? 2 : 4);
+  static constexpr int size = R * pitch;
 };
 
-// Per-thread loader of one operand slab (R rows x BK k-values per slab).
-// KF: thread owns k = tid % BK and rows tid / BK + j * (256 / BK);
-// else: thread owns row tid % R and k = tid / R + j * (256 / R).
-template <int R, bool KF, int BK>
-struct Loader {
+// How an operand's summed indices lie in memory: Vec, contiguous (k-contiguous
+// operand, stride 1): two k per load; Aff, any constant stride; Tab, a table.
+// All three address it with 32-bit byte offsets; Wide is Tab with 64-bit
+// addresses, for operands that reach 4 GiB (GemmArgs::wide).
+enum class KMode { Vec, Aff, Tab, Wide };
+
+// Offsets of the summed indices of a Tab or Wide operand's K range, in LDS (bytes;
+// Wide: elements), for at most kKCache indices; longer ranges are walked in runs
+// of kKCache.
+constexpr int kKCache = 1024;
+
+// One operand's slabs (R rows x BK k-values), global memory -> registers ->
+// LDS, 256 threads.  A thread owns L values: Vec: L / 2 rows, two consecutive
+// k; else one k of L rows (kfast: neighbouring threads own neighbouring k) or L
+// k of one row (neighbouring threads own neighbouring rows).  FP64 MFMAs share
+// the vector ALUs with everything else (a pure loop of them runs at 77 TF/s,
+// and every other vector instruction takes its time from it), so the loop over
+// whole slabs has none of its own: Vec and Aff addresses are a scalar base that
+// moves by a slab plus a 32-bit offset that does not, rows past the end are
+// clamped to the last one (their products are never stored), and only the last
+// slab is masked.
+// The registers hold the stored type IO: a conversion right after the load
+// would wait for it there.
+template <typename T, typename IO, int R, int BK, KMode MODE>
+struct Feed {
+  static constexpr bool vec = MODE == KMode::Vec;
+  static constexpr bool tab = MODE == KMode::Tab || MODE == KMode::Wide;
+  // unit of off[] and of the offset table
+  static constexpr uint32_t unit = MODE == KMode::Wide ? 1 : (uint32_t)sizeof(IO);
   static constexpr int L = R * BK / 256;
-  int row_off[L];        // table offset of each owned row (or -1)
-  int kk[L];             // owned k within slab
-  int rr[L];             // owned row within tile
-  __device__ void init(const int* __restrict__ rowtab, int64_t r0, int64_t R_total, int tid) {
+  static constexpr int NJ = vec ? L / 2 : L;
+  static constexpr int pitch = LdsTile<T, R, BK>::pitch;
+  typedef IO io2 __attribute__((ext_vector_type(2), aligned(sizeof(IO))));
+  typedef T t2 __attribute__((ext_vector_type(2)));
+  struct Slab {
+    IO v[L];
+  };
+  const char* base;   // the operand, at the first summed index of the range (Vec, Aff)
+  int64_t aff;
+  uint32_t off[NJ];   // offset of each row (Vec, Aff: plus that of the value's k in the slab)
+  int k0, ks;         // k of item j in a slab: k0 + j ks
+  int lds0, ldss;     // its place in the LDS tile: lds0 + j ldss
+
+  __device__ __forceinline__ void init(const double* X, const int* __restrict__ rowtab, int64_t r0, int64_t rows,
+                                       int kfast, int64_t kaff, int64_t kr, int tid) {
+    int r, rs;
+    if constexpr (vec) {
+      r = tid / (BK / 2), rs = 512 / BK;
+      k0 = 2 * (tid % (BK / 2)), ks = 0;
+    } else {
+      r = kfast ? tid / BK : tid % R, rs = kfast ? 256 / BK : 0;
+      k0 = kfast ? tid % BK : tid / R, ks = kfast ? 0 : 256 / R;
+    }
+    lds0 = r * pitch + k0;
+    ldss = rs * pitch + ks;
+    aff = tab ? 0 : kaff;
+    base = reinterpret_cast<const char*>(X) + kr * aff * (int64_t)sizeof(IO);
 #pragma unroll
-    for (int j = 0; j < L; ++j) {
-      int row, k;
-      if (KF) { k = tid % BK; row = tid / BK + j * (256 / BK); }
-      else { row = tid % R; k = tid / R + j * (256 / R); }
-      kk[j] = k;
-      rr[j] = row;
-      const int64_t g = r0 + row;
-      row_off[j] = g < R_total ? rowtab[g] : -1;
+    for (int j = 0; j < NJ; ++j) {
+      const int64_t gr = r0 + r + j * rs;
+      off[j] = (uint32_t)rowtab[gr < rows ? gr : rows - 1] * unit;
+      if (!tab) off[j] += (uint32_t)((k0 + j * ks) * aff) * unit;
     }
   }
-  // K offsets: k * kaff when affine, else the workgroup's copy of the table
-  // in LDS (lk[k - kbase]) when use_l, else the table in global memory.
-  // The registers hold the stored type IO: a conversion right after the
-  // load would wait for it there and expose its latency to the MFMA loop.
-  template <typename IO>
-  __device__ void fetch(IO (&reg)[L], const double* __restrict__ Xd, const int* __restrict__ ktab,
-                        int64_t kaff, const int* lk, bool use_l, int64_t kbase, int64_t k0,
-                        int64_t kend) const {
-    const IO* __restrict__ X = reinterpret_cast<const IO*>(Xd);
-    auto ko = [&](int64_t gk) -> int64_t {
-      return kaff >= 0 ? gk * kaff : (use_l ? (int64_t)lk[gk - kbase] : (int64_t)ktab[gk]);
-    };
-    if (KF) {
-      const int64_t gk = k0 + kk[0];
-      const bool kin = gk < kend;
-      const int64_t o = kin ? ko(gk) : 0;
+  __device__ __forceinline__ IO at(uint32_t row, uint32_t k) const {
+    if constexpr (MODE == KMode::Wide) return reinterpret_cast<const IO*>(base)[(uint64_t)row + k];
+    else return *reinterpret_cast<const IO*>(base + (row + k));
+  }
+  // whole slab at index i of the range; ko: the range's offset table (Tab, Wide)
+  __device__ __forceinline__ void fetch(Slab& s, int i, const uint32_t* ko) const {
+    const char* p = base + i * aff * (int64_t)sizeof(IO);
 #pragma unroll
-      for (int j = 0; j < L; ++j) reg[j] = (kin && row_off[j] >= 0) ? X[(int64_t)row_off[j] + o] : IO(0);
-    } else {
-#pragma unroll
-      for (int j = 0; j < L; ++j) {
-        const int64_t gk = k0 + kk[j];
-        reg[j] = (gk < kend && row_off[j] >= 0) ? X[(int64_t)row_off[j] + ko(gk)] : IO(0);
+    for (int j = 0; j < NJ; ++j) {
+      if constexpr (vec) {
+        const io2 x = *reinterpret_cast<const io2*>(p + off[j]);
+        s.v[2 * j] = x.x;
+        s.v[2 * j + 1] = x.y;
+      } else if constexpr (MODE == KMode::Aff) {
+        s.v[j] = *reinterpret_cast<const IO*>(p + off[j]);
+      } else {
+        s.v[j] = at(off[j], ko[i + k0 + j * ks]);
       }
     }
   }
-  template <typename T, typename IO>
-  __device__ void stash(T* lds, const IO (&reg)[L]) const {
+  // the slab at index i with k past the end (klen) clamped to the last one
+  __device__ __forceinline__ void fetch_tail(Slab& s, int i, int klen, const uint32_t* ko) const {
 #pragma unroll
-    for (int j = 0; j < L; ++j) lds[LdsTile<T, R, KF, BK>::at(rr[j], kk[j])] = (T)reg[j];
+    for (int j = 0; j < L; ++j) {
+      const int q = vec ? j / 2 : j;
+      const int kq = k0 + q * ks;
+      const int k = i + (vec ? k0 + (j & 1) : kq);
+      const int kc = k < klen ? k : klen - 1;
+      if constexpr (tab)
+        s.v[j] = at(off[q], ko[kc]);
+      else
+        s.v[j] = *reinterpret_cast<const IO*>(base + off[q] + (int64_t)(kc - kq) * aff * (int64_t)sizeof(IO));
+    }
+  }
+  __device__ __forceinline__ void stash(T* to, const Slab& s) const {
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      if constexpr (vec) {
+        t2 x;
+        x.x = (T)s.v[2 * j];
+        x.y = (T)s.v[2 * j + 1];
+        *reinterpret_cast<t2*>(to + lds0 + j * ldss) = x;
+      } else {
+        to[lds0 + j * ldss] = (T)s.v[j];
+      }
+    }
+  }
+  // left: summed indices from the slab's first k to the end of the range
+  __device__ __forceinline__ void stash_tail(T* to, const Slab& s, int left) const {
+#pragma unroll
+    for (int j = 0; j < L; ++j) {
+      const int q = vec ? j / 2 : j, e = vec ? j & 1 : 0;
+      to[lds0 + q * ldss + e] = k0 + q * ks + e < left ? (T)s.v[j] : T(0);
+    }
   }
 };
 
@@ -235,11 +298,14 @@ struct Mma<float> {
 // both output extents large (MFMA bound).  256 threads = 4 waves in a 2 x 2
 // grid; each wave owns a (BM/2) x (BN/2) sub-tile of 16x16 MFMA tiles.
 // Operands are gathered in their stored type IO (FP64; FP32 in the
-// FP32-storage sweeps) through int32 offset tables (rowA/kA, kB/colB) and
-// staged into LDS as T; the next K slab is fetched into
-// registers while the current one is multiplied out of LDS.  T = double runs
-// on v_mfma_f64_16x16x4f64; T = float rounds the operands to FP32 and
-// accumulates in FP32 on v_mfma_f32_16x16x4f32 (the mixed-precision form).
+// FP32-storage sweeps) through int32 row offset tables (rowA, colB) and their
+// summed indices' stride or table (kA, kB), and staged into LDS as T.  T =
+// double runs on v_mfma_f64_16x16x4f64; T = float rounds the operands to FP32
+// and accumulates in FP32 on v_mfma_f32_16x16x4f32 (the mixed-precision form).
+// FP64, against one slab of look-ahead with two barriers a slab, predicated
+// loads and single-k fragment reads: 1225 x 4375 x 1225 303 -> 244 us (54 TF/s),
+// 900^3 58.6 -> 42 us, 8100 x 100 x 8100 448 -> 328 us, 4096 x 4096 x 2048
+// 53 -> 65 TF/s; without the loads and LDS writes the same loop runs at 73.
 // blockIdx.z owns K range [z*kchunk, (z+1)*kchunk) (split-K, completed by
 // gemm_splitk_reduce).  KS = 2 doubles the workgroup: two groups of 4 waves
 // take alternate K slabs of the same tile (each with its own LDS slab) and
@@ -322,108 +388,165 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, int64_t m0, int64_
   }
 }
 
-// LDS bytes of one tile-kernel variant
-template <typename T, int BM, int BN, int BK, bool AKF, bool BKF, int KS>
+// Waves per SIMD the tile kernels are compiled for: three 64 x 64 workgroups a CU
+// measured 8 % faster than two on operands that are not k-contiguous
+// (1225 x 4375 x 1225: 287 -> 265 us).
+template <int KS>
+constexpr int kTileWaves = KS > 1 ? 1 : 3;
+
+// LDS bytes of one tile-kernel variant (two slabs per group)
+template <typename T, int BM, int BN, int BK, int KS>
 struct TabLds {
-  static constexpr int tile = KS * (LdsTile<T, BM, AKF, BK>::size + LdsTile<T, BN, BKF, BK>::size) * (int)sizeof(T);
+  static constexpr int slab = LdsTile<T, BM, BK>::size + LdsTile<T, BN, BK>::size;
+  static constexpr int tile = 2 * KS * slab * (int)sizeof(T);
   static constexpr int red = (KS - 1) * 256 * (BM / 32) * (BN / 32) * 4 * (int)sizeof(T);
-  static constexpr int bytes = tile > red ? tile : red;
+  static constexpr int kts = (tile > red ? tile : red);   // offset of the K offsets
+  static constexpr int bytes = kts + 2 * kKCache * (int)sizeof(int);
 };
-
-// K-offset tables of a workgroup's K range are copied into LDS when the range
-// has at most kKCache entries (the non-k-contiguous loader reads L offsets
-// per slab; from global memory each is a dependent load before the data)
-constexpr int kKCache = 2048;
-
-template <typename T, typename IO, int BM, int BN, int BK, bool AKF, bool BKF, int KS>
-__device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty, int tz, unsigned char* smem,
-                                              int* kts);
-
-template <typename T, typename IO, int BM, int BN, int BK, bool AKF, bool BKF, int KS>
-__global__ __launch_bounds__(256 * KS, (KS == 1 && !(sizeof(T) == 8 && BM * BN >= 128 * 128)) ? 2 : 1)
-void gemm_tab(GemmArgs g) {
-  __shared__ __align__(16) unsigned char smem[TabLds<T, BM, BN, BK, AKF, BKF, KS>::bytes];
-  __shared__ int kts[2 * kKCache];
-  int tx, ty, tz;
-  tile_coords(g.group, tx, ty, tz);
-  gemm_tab_tile<T, IO, BM, BN, BK, AKF, BKF, KS>(g, tx, ty, tz, smem, kts);
-}
 
 // The K-slab loop of the tile kernel: acc += A(m0.., kbeg..kend) B(kbeg..kend, n0..)
 // (the caller zeroes acc; group grp of KS takes slabs grp, grp + KS, ...).
-template <typename T, typename IO, int BM, int BN, int BK, bool AKF, bool BKF, int KS>
-__device__ __forceinline__ void tile_mma(const GemmArgs& g, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
-                                         unsigned char* smem, int* kts,
-                                         typename Mma<T>::acc_t (&acc)[BM / 32][BN / 32]) {
+// Slab s is multiplied out of one LDS buffer while slab s + 1 is written to
+// the other and slabs s + 2, s + 3 are in flight to registers: one barrier a
+// slab, and a load has two slabs' time to arrive.  A fragment read takes two
+// consecutive k (the four 16-lane groups of an MFMA then hold k, k + 2, k + 4,
+// k + 6: the same products, summed in another order).
+template <typename T, typename IO, int BM, int BN, int BK, int KS, KMode MA, KMode MB>
+__device__ __forceinline__ void tile_run(const GemmArgs& g, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
+                                         unsigned char* smem, typename Mma<T>::acc_t (&acc)[BM / 32][BN / 32]) {
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int TM = WM / 16, TN = WN / 16;
-  using TA = LdsTile<T, BM, AKF, BK>;
-  using TB = LdsTile<T, BN, BKF, BK>;
+  using FA = Feed<T, IO, BM, BK, MA>;
+  using FB = Feed<T, IO, BN, BK, MB>;
   using MM = Mma<T>;
-  const int grp = threadIdx.x >> 8;
-  T* As = reinterpret_cast<T*>(smem) + grp * (TA::size + TB::size);
-  T* Bs = As + TA::size;
+  typedef T t2 __attribute__((ext_vector_type(2)));
+  constexpr int slab = TabLds<T, BM, BN, BK, KS>::slab;
+  constexpr bool tab = FA::tab || FB::tab;
+  const int grp = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  T* lds = reinterpret_cast<T*>(smem) + grp * 2 * slab;
+  uint32_t* kts = reinterpret_cast<uint32_t*>(smem + TabLds<T, BM, BN, BK, KS>::kts);
   const int tid = threadIdx.x & 255;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = (wave & 1) * WM;
-  const int wn = (wave >> 1) * WN;
+  const T* fa = lds + ((wave & 1) * WM + (lane & 15)) * FA::pitch + 2 * (lane >> 4);
+  const T* fb = lds + LdsTile<T, BM, BK>::size + ((wave >> 1) * WN + (lane & 15)) * FB::pitch + 2 * (lane >> 4);
 
-  Loader<BM, AKF, BK> la;
-  Loader<BN, BKF, BK> lb;
-  la.init(g.rowA, m0, g.M, tid);
-  lb.init(g.colB, n0, g.N, tid);
-  IO ra[Loader<BM, AKF, BK>::L], rb[Loader<BN, BKF, BK>::L];
-
-  // non-affine K tables of this K range into LDS (uniform condition)
-  const int64_t klen = kend > kbeg ? kend - kbeg : 0;
-  const bool a_l = g.kA_aff < 0 && klen <= kKCache;
-  const bool b_l = g.kB_aff < 0 && klen <= kKCache;
-  if (a_l || b_l) {
-    for (int i = (int)threadIdx.x; i < (int)klen; i += (int)blockDim.x) {
-      if (a_l) kts[i] = g.kA[kbeg + i];
-      if (b_l) kts[kKCache + i] = g.kB[kbeg + i];
-    }
-    __syncthreads();
-  }
-
-  // (a slab past the end loads zeros, so both groups run the same barriers)
-  const int64_t nslabs = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
-  const int64_t nsteps = (nslabs + KS - 1) / KS;
-  if (nsteps > 0) {
-    la.template fetch<IO>(ra, g.A, g.kA, g.kA_aff, kts, a_l, kbeg, kbeg + grp * BK, kend);
-    lb.template fetch<IO>(rb, g.B, g.kB, g.kB_aff, kts + kKCache, b_l, kbeg, kbeg + grp * BK, kend);
-  }
-  for (int64_t s = 0; s < nsteps; ++s) {
-    __syncthreads();
-    la.stash(As, ra);
-    lb.stash(Bs, rb);
-    __syncthreads();
-    if (s + 1 < nsteps) {
-      const int64_t k0 = kbeg + ((s + 1) * KS + grp) * BK;
-      la.template fetch<IO>(ra, g.A, g.kA, g.kA_aff, kts, a_l, kbeg, k0, kend);
-      lb.template fetch<IO>(rb, g.B, g.kB, g.kB_aff, kts + kKCache, b_l, kbeg, k0, kend);
-    }
+  auto mma = [&](int b) {
 #pragma unroll
-    for (int ks = 0; ks < BK; ks += 4) {
-      const int kr = ks + (lane >> 4);
-      const int rr = lane & 15;
-      T af[TM], bf[TN];
+    for (int ks = 0; ks < BK; ks += 8) {
+      t2 af[TM], bf[TN];
 #pragma unroll
-      for (int i = 0; i < TM; ++i) af[i] = As[TA::at(wm + 16 * i + rr, kr)];
+      for (int i = 0; i < TM; ++i) af[i] = *reinterpret_cast<const t2*>(fa + b * slab + 16 * i * FA::pitch + ks);
 #pragma unroll
-      for (int j = 0; j < TN; ++j) bf[j] = Bs[TB::at(wn + 16 * j + rr, kr)];
+      for (int j = 0; j < TN; ++j) bf[j] = *reinterpret_cast<const t2*>(fb + b * slab + 16 * j * FB::pitch + ks);
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = MM::step(af[i], bf[j], acc[i][j]);
+        for (int j = 0; j < TN; ++j) acc[i][j] = MM::step(af[i].x, bf[j].x, acc[i][j]);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = MM::step(af[i].y, bf[j].y, acc[i][j]);
     }
+  };
+  const int64_t run = tab ? (int64_t)kKCache : kend - kbeg;
+  for (int64_t kr = kbeg; kr < kend; kr += run) {
+    const int klen = (int)(kend - kr < run ? kend - kr : run);
+    const int nfull = klen / BK;   // whole slabs
+    const int nsteps = ((klen + BK - 1) / BK + KS - 1) / KS;
+    FA la;
+    FB lb;
+    la.init(g.A, g.rowA, m0, g.M, g.a_kfast, g.kA_aff, kr, tid);
+    lb.init(g.B, g.colB, n0, g.N, g.b_kfast, g.kB_aff, kr, tid);
+    typename FA::Slab ra[2];
+    typename FB::Slab rb[2];
+    if (tab) {
+      if (kr > kbeg) __syncthreads();
+      for (int i = (int)threadIdx.x; i < klen; i += 256 * KS) {
+        if (FA::tab) kts[i] = (uint32_t)(g.kA_aff >= 0 ? (kr + i) * g.kA_aff : (int64_t)g.kA[kr + i]) * FA::unit;
+        if (FB::tab)
+          kts[kKCache + i] = (uint32_t)(g.kB_aff >= 0 ? (kr + i) * g.kB_aff : (int64_t)g.kB[kr + i]) * FB::unit;
+      }
+      __syncthreads();
+    }
+    auto first = [&](int s) { return (s * KS + grp) * BK; };
+    // values of slab s to register set x, and from there to LDS buffer x; whole
+    // slabs, and any slab (past the end: zeros, so both groups run the same barriers)
+    auto fetch = [&](int x, int s) {
+      la.fetch(ra[x], first(s), kts);
+      lb.fetch(rb[x], first(s), kts + kKCache);
+    };
+    auto fetch_any = [&](int x, int s) {
+      if (s * KS + grp < nfull) {
+        fetch(x, s);
+      } else {
+        la.fetch_tail(ra[x], first(s), klen, kts);
+        lb.fetch_tail(rb[x], first(s), klen, kts + kKCache);
+      }
+    };
+    auto stash = [&](int x) {
+      la.stash(lds + x * slab, ra[x]);
+      lb.stash(lds + x * slab + LdsTile<T, BM, BK>::size, rb[x]);
+    };
+    auto stash_any = [&](int x, int s) {
+      if (s * KS + grp < nfull) {
+        stash(x);
+      } else {
+        la.stash_tail(lds + x * slab, ra[x], klen - first(s));
+        lb.stash_tail(lds + x * slab + LdsTile<T, BM, BK>::size, rb[x], klen - first(s));
+      }
+    };
+    // step s: slab s is in buffer x = s & 1; register set 1 - x holds slab s + 1
+    auto step = [&](int x, int s) {
+      __syncthreads();
+      stash(1 - x);
+      fetch(1 - x, s + 3);
+      mma(x);
+    };
+    auto step_any = [&](int x, int s) {
+      __syncthreads();
+      if (s + 1 < nsteps) stash_any(1 - x, s + 1);
+      if (s + 3 < nsteps) fetch_any(1 - x, s + 3);
+      mma(x);
+    };
+    fetch_any(0, 0);
+    if (nsteps > 1) fetch_any(1, 1);
+    stash_any(0, 0);
+    if (nsteps > 2) fetch_any(0, 2);
+    int s = 0;
+    for (; s + 4 < nfull / KS; s += 2) {
+      step(0, s);
+      step(1, s + 1);
+    }
+    for (; s + 2 <= nsteps; s += 2) {
+      step_any(0, s);
+      step_any(1, s + 1);
+    }
+    if (s < nsteps) step_any(0, s);
   }
 }
 
-template <typename T, typename IO, int BM, int BN, int BK, bool AKF, bool BKF, int KS>
-__device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty, int tz, unsigned char* smem,
-                                              int* kts) {
+template <typename T, typename IO, int BM, int BN, int BK, int KS>
+__device__ __forceinline__ void tile_mma(const GemmArgs& g, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
+                                         unsigned char* smem, typename Mma<T>::acc_t (&acc)[BM / 32][BN / 32]) {
+  const int ma = g.kA_aff < 0 ? 2 : (g.a_kfast && g.kA_aff == 1 ? 0 : 1);
+  const int mb = g.kB_aff < 0 ? 2 : (g.b_kfast && g.kB_aff == 1 ? 0 : 1);
+#define CCQ_RUN(a, b) tile_run<T, IO, BM, BN, BK, KS, KMode::a, KMode::b>(g, m0, n0, kbeg, kend, smem, acc)
+  switch (g.wide ? 9 : 3 * ma + mb) {
+    case 0: CCQ_RUN(Vec, Vec); break;
+    case 1: CCQ_RUN(Vec, Aff); break;
+    case 3: CCQ_RUN(Aff, Vec); break;
+    case 4: CCQ_RUN(Aff, Aff); break;
+    case 2: CCQ_RUN(Vec, Tab); break;
+    case 6: CCQ_RUN(Tab, Vec); break;
+    case 9: CCQ_RUN(Wide, Wide); break;
+    default: CCQ_RUN(Tab, Tab); break;
+  }
+#undef CCQ_RUN
+}
+
+template <typename T, typename IO, int BM, int BN, int BK, int KS>
+__device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty, int tz, unsigned char* smem) {
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int TM = WM / 16, TN = WN / 16;
   using MM = Mma<T>;
@@ -443,7 +566,7 @@ __device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty,
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
-  tile_mma<T, IO, BM, BN, BK, AKF, BKF, KS>(g, m0, n0, kbeg, kend, smem, kts, acc);
+  tile_mma<T, IO, BM, BN, BK, KS>(g, m0, n0, kbeg, kend, smem, acc);
 
   if (KS > 1) {
     // group 1 hands its accumulators to group 0 (slab order: group 0's sum
@@ -487,15 +610,23 @@ __device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty,
   }
 }
 
+template <typename T, typename IO, int BM, int BN, int BK, int KS>
+__global__ __launch_bounds__(256 * KS, kTileWaves<KS>) void gemm_tab(GemmArgs g) {
+  __shared__ __align__(16) unsigned char smem[TabLds<T, BM, BN, BK, KS>::bytes];
+  int tx, ty, tz;
+  tile_coords(g.group, tx, ty, tz);
+  gemm_tab_tile<T, IO, BM, BN, BK, KS>(g, tx, ty, tz, smem);
+}
+
 // Entries e0 <= e < e1 of a chain accumulating into one output tile (tx, ty):
 // the workgroup walks the concatenated K range [kbeg, kend) (kend < 0: all of
 // it) entry by entry, each with its own operands and layouts, adds alpha_e
 // times the entry's partial product to an FP64 sum, and stores once with the
 // first entry's output arguments (split z of a split-K launch: into the
 // workspace).
-template <typename T, typename IO, int BM, int BN, int BK, bool AKF, bool BKF>
+template <typename T, typename IO, int BM, int BN, int BK>
 __device__ __forceinline__ void tile_entries(const GemmArgs* es, int e0, int e1, int tx, int ty, int tz,
-                                             int64_t kbeg, int64_t kend, unsigned char* smem, int* kts) {
+                                             int64_t kbeg, int64_t kend, unsigned char* smem) {
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int TM = WM / 16, TN = WN / 16;
   using MM = Mma<T>;
@@ -527,7 +658,7 @@ __device__ __forceinline__ void tile_entries(const GemmArgs* es, int e0, int e1,
       for (int j = 0; j < TN; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
     // the previous entry's waves are past their last LDS reads
     if (e > e0) __syncthreads();
-    tile_mma<T, IO, BM, BN, BK, AKF, BKF, 1>(g, m0, n0, a, b, smem, kts, acc);
+    tile_mma<T, IO, BM, BN, BK, 1>(g, m0, n0, a, b, smem, acc);
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -555,53 +686,29 @@ __device__ __forceinline__ void tile_entries(const GemmArgs* es, int e0, int e1,
   }
 }
 
-// LDS of the kernels that switch between operand layouts per entry
-template <typename T, int BM, int BN, int BK>
-struct AnyLds {
-  static constexpr int b11 = TabLds<T, BM, BN, BK, true, true, 1>::bytes;
-  static constexpr int b10 = TabLds<T, BM, BN, BK, true, false, 1>::bytes;
-  static constexpr int b01 = TabLds<T, BM, BN, BK, false, true, 1>::bytes;
-  static constexpr int b00 = TabLds<T, BM, BN, BK, false, false, 1>::bytes;
-  static constexpr int m1 = b11 > b10 ? b11 : b10, m2 = b01 > b00 ? b01 : b00;
-  static constexpr int bytes = m1 > m2 ? m1 : m2;
-};
-
 // A chain of GEMMs accumulating into one output with the same tile mapping
 // and operand layouts (C (+)= sum_e alpha_e A_e B_e (+ dcoef D)), as one
 // product over the concatenated K ranges, split along the concatenated K
 // (split z of tile (tx, ty) covers [z kchunk, (z + 1) kchunk)).
-template <typename T, typename IO, int BM, int BN, int BK, bool AKF, bool BKF>
-__global__ __launch_bounds__(256, !(sizeof(T) == 8 && BM * BN >= 128 * 128) ? 2 : 1)
-void gemm_tab_chain(GemmChain ch) {
-  __shared__ __align__(16) unsigned char smem[TabLds<T, BM, BN, BK, AKF, BKF, 1>::bytes];
-  __shared__ int kts[2 * kKCache];
+template <typename T, typename IO, int BM, int BN, int BK>
+__global__ __launch_bounds__(256, kTileWaves<1>) void gemm_tab_chain(GemmChain ch) {
+  __shared__ __align__(16) unsigned char smem[TabLds<T, BM, BN, BK, 1>::bytes];
   int tx, ty, tz;
   tile_coords(ch.e[0].group, tx, ty, tz);
   const int64_t ktot = ch.koff[ch.n];
   const int64_t kbeg = (int64_t)tz * ch.e[0].kchunk;
   const int64_t kend = (kbeg + ch.e[0].kchunk < ktot) ? kbeg + ch.e[0].kchunk : ktot;
-  tile_entries<T, IO, BM, BN, BK, AKF, BKF>(ch.e, 0, ch.n, tx, ty, tz, kbeg, kend, smem, kts);
+  tile_entries<T, IO, BM, BN, BK>(ch.e, 0, ch.n, tx, ty, tz, kbeg, kend, smem);
 }
 
 // The same tile kernel over the tiles of a group of independent GEMMs (full K
-// each).  The operand layouts (k-contiguous or not) may differ between
-// members: the workgroup branches once, uniformly, to the body of its
-// member's layouts.
+// each).
 template <typename T, typename IO, int BM, int BN, int BK>
-__global__ __launch_bounds__(256, !(sizeof(T) == 8 && BM * BN >= 128 * 128) ? 2 : 1)
-void gemm_tab_group(GemmGroup gg) {
-  __shared__ __align__(16) unsigned char smem[AnyLds<T, BM, BN, BK>::bytes];
-  __shared__ int kts[2 * kKCache];
+__global__ __launch_bounds__(256, kTileWaves<1>) void gemm_tab_group(GemmGroup gg) {
+  __shared__ __align__(16) unsigned char smem[TabLds<T, BM, BN, BK, 1>::bytes];
   int tx, ty;
   const int mem = group_tile<BM, BN>(gg, tx, ty);
-  const GemmArgs& g = gg.g[mem];
-  if (g.a_kfast) {
-    if (g.b_kfast) gemm_tab_tile<T, IO, BM, BN, BK, true, true, 1>(g, tx, ty, 0, smem, kts);
-    else gemm_tab_tile<T, IO, BM, BN, BK, true, false, 1>(g, tx, ty, 0, smem, kts);
-  } else {
-    if (g.b_kfast) gemm_tab_tile<T, IO, BM, BN, BK, false, true, 1>(g, tx, ty, 0, smem, kts);
-    else gemm_tab_tile<T, IO, BM, BN, BK, false, false, 1>(g, tx, ty, 0, smem, kts);
-  }
+  gemm_tab_tile<T, IO, BM, BN, BK, 1>(gg.g[mem], tx, ty, 0, smem);
 }
 
 // Register-direct GEMM for skinny and dot-shaped products (an output extent

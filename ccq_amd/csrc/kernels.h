@@ -32,6 +32,8 @@ struct GemmArgs {
   int c_mfast = 0, c_nfast = 0;
   // kA[k] == k * kA_aff for every k when kA_aff >= 0 (same for B)
   int64_t kA_aff = -1, kB_aff = -1;
+  // A or B reaches 4 GiB: the tile kernel addresses both with 64 bits
+  int wide = 0;
   // launch plan (gemm_plan)
   int kind = 0;            // 0: LDS-tiled kernel, 1: register-direct kernel
   int trans = 0;           // run as C^T = B^T A^T (register-direct kernel)
@@ -43,8 +45,8 @@ struct GemmArgs {
   // arithmetic of the LDS-tiled kernel: 0 FP64 MFMA; 1 FP32 MFMA (operands
   // rounded to FP32 when staged into LDS, FP32 accumulation, FP64 epilogue)
   int prec = 0;
-  // LDS-tiled kernel: 2 = two 4-wave groups share a tile and split its K
-  // slabs (tiles up to 64x64), 1 = one group
+  // LDS-tiled kernel: 2 = two 4-wave groups share a 32x32 tile and split its K
+  // slabs, 1 = one group
   int ksplit = 1;
   // split-K workspace of at least gemm_ws_need doubles
   double* ws = nullptr;
@@ -131,6 +133,11 @@ struct Coeffs {
   double c[kMaxDiis];
 };
 
+// K depth of a tile kernel's slab: 16 keeps three 64 x 64 workgroups on a CU (45 KB
+// of LDS each; 252 us against 270 us with 32 on 1225 x 4375 x 1225), 32 halves
+// the slabs of the small tiles, which run short summed ranges.
+constexpr int tile_bk(int bm, int bn) { return bm * bn > 32 * 32 ? 16 : 32; }
+
 // Choose kernel, tile shape and split-K for a GEMM; ws_cap bounds the
 // split-K workspace (doubles).
 void gemm_plan(GemmArgs& g, int64_t ws_cap);
@@ -161,7 +168,7 @@ hipError_t launch_gemm_group(hipStream_t s, const GemmArgs* gs, int n);
 
 // A chain of GEMMs accumulating into one output with the same tile mapping
 // and the same operand layouts (k-contiguous or not, after transposition),
-// run as one product over the concatenated K ranges (LDS-tiled kernel, BK 32,
+// run as one product over the concatenated K ranges (LDS-tiled kernel,
 // split-K over the concatenated K).  Entry i contributes alpha_i A_i B_i
 // (its trans flag: run transposed to match the output orientation); the
 // output arguments (C, its tables, accumulate, the folded addend) and the

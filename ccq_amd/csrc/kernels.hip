@@ -769,47 +769,45 @@ void gemm_plan_ranked(GemmArgs& g, int64_t ws_cap, std::vector<std::pair<double,
   };
 
   // LDS-tiled kernel.  A WG of 4 waves keeps each SIMD busy for
-  // (BM/32)(BN/32)*BK/4 MFMAs per K slab; resident WGs per CU (VGPR/LDS):
-  // 2 for 128x128, 3 for 128x64 / 64x128, 4 for 64x64, 6 for 64x32 / 32x64,
-  // 8 for 32x32.  A CU holding a single WG cannot hide the global-load
-  // latency of a slab (~1500 cycles); every slab costs two barriers and the
-  // LDS round trip (~300 cycles).  The small tiles pay off for products with
-  // a short side of a few MFMA tiles or a short K (more WGs, no split-K).
+  // (BM/32)(BN/32)*BK/4 MFMAs per K slab; three WGs are resident per CU.  A
+  // slab costs about 200 cycles beside its MFMAs, and a CU holding a single
+  // WG waits for its barriers and loads (512^3 in 64x64 tiles, one a CU: 1800
+  // cycles a slab against 1024 of MFMAs; in 32x32 tiles 1500 against 512).
+  // The small tiles pay off for products with a short side of a few MFMA
+  // tiles or a short K (more WGs, no split-K).
   struct Shape { int bm, bn, occ; };
-  // resident WGs per CU (128x128 uses more than 256 VGPRs: one)
-  const Shape shapes[7] = {{128, 128, 1}, {128, 64, 3}, {64, 128, 3}, {64, 64, 4},
-                           {64, 32, 6},   {32, 64, 6},  {32, 32, 8}};
+  const Shape shapes[4] = {{64, 64, 3}, {64, 32, 3}, {32, 64, 3}, {32, 32, 3}};
   // the epilogue stores 16 consecutive columns per 16 lanes: when C is
   // contiguous along m only, run the product transposed (C^T = B^T A^T)
   const int ttile = (g.c_mfast && !g.c_nfast) ? 1 : 0;
   const int64_t TM_ = ttile ? g.N : g.M, TN_ = ttile ? g.M : g.N;
-  for (int bk : {16, 32}) {
+  for (const Shape& sh : shapes) {
+    const int bk = tile_bk(sh.bm, sh.bn);
     const int64_t ksteps = cdiv(g.K, bk);
-    for (const Shape& sh : shapes) {
-      // small tiles only for a short side (measured: no gain, or a loss, on
-      // square-ish products such as the 900^3 ring)
-      if (sh.bm * sh.bn < 64 * 64 && std::min(g.M, g.N) > 128) continue;
-      // no tiles for dot-like products with a tiny side and a long K (the
-      // register-direct kernel with split-K measured faster)
-      if (std::min(g.M, g.N) < 16 && g.K >= 4096) continue;
-      const int64_t tiles = cdiv(TM_, sh.bm) * cdiv(TN_, sh.bn);
-      const double slab = (sh.bm / 32.0) * (sh.bn / 32.0) * (bk / 4.0) * 64.0;
-      const int64_t maxsplit = std::max<int64_t>(1, std::min<int64_t>(ksteps / 2, 512));
-      for (int ksp = 1; ksp <= 2; ++ksp)
+    // no tiles for dot-like products with a tiny side and a long K (the
+    // register-direct kernel with split-K measured faster)
+    if (std::min(g.M, g.N) < 16 && g.K >= 4096) continue;
+    // square-ish products take 64x64 (a 64x32 tile loads 1.5 times as much per
+    // MFMA: 900^3 68 - 80 us in the sweep against 53), except where those
+    // would leave half the chip idle (512^3: 24 us, 10 us in 32x32)
+    if (sh.bm * sh.bn < 64 * 64 && std::min(g.M, g.N) > 128 &&
+        (sh.bm * sh.bn > 32 * 32 || cdiv(g.M, 64) * cdiv(g.N, 64) >= cus / 2))
+      continue;
+    const int64_t tiles = cdiv(TM_, sh.bm) * cdiv(TN_, sh.bn);
+    const double slab = (sh.bm / 32.0) * (sh.bn / 32.0) * (bk / 4.0) * 64.0;
+    const int64_t maxsplit = std::max<int64_t>(1, std::min<int64_t>(ksteps / 2, 512));
+    for (int ksp = 1; ksp <= 2; ++ksp)
       for (int64_t split = 1; split <= maxsplit; split *= 2) {
-        if (ksp == 2 && sh.bm * sh.bn > 64 * 64) break;
         // measured inside the sweep: the doubled workgroup pays off only for
-        // matrix-vector products (a side of 1 or 2); on the 900^3 ring it
-        // beats split-K with hot operands (58 vs 61 us) but loses with the
-        // sweep's cold ones (94 vs 82 us)
-        if (ksp == 2 && std::min(g.M, g.N) > 2) break;
+        // matrix-vector products (a side of 1 or 2)
+        if (ksp == 2 && (sh.bm * sh.bn > 32 * 32 || std::min(g.M, g.N) > 2)) break;
         if (split > 1 && split * g.M * g.N > ws_cap) break;
         // ksp = 2: a doubled workgroup whose two groups take alternate slabs
         const int64_t steps = cdiv(ksteps, split * ksp);
         const double per_cu = std::ceil((double)tiles * split / cus);
         const double resident = std::min<double>(per_cu, std::max(1, sh.occ / ksp)) * ksp;
-        double cyc = per_cu * (steps + 2) * (ksp * slab + 300.0);
-        if (resident < 2) cyc += per_cu * steps * 1500.0;
+        double cyc = per_cu * (steps + 2) * (ksp * slab + 200.0);
+        if (resident < 2) cyc += per_cu * steps * 700.0;
         if (std::min(g.M, g.N) <= 128) {
           // skinny: at least one streaming pass over the operands and C
           const double bytes = 8.0 * ((double)g.M * g.K + (double)g.K * g.N + (double)g.M * g.N);
@@ -821,7 +819,6 @@ void gemm_plan_ranked(GemmArgs& g, int64_t ws_cap, std::vector<std::pair<double,
         take(cyc, 0, ttile, sh.bm, sh.bn, bk, nullptr, split, steps * ksp * bk, ksp);
         if (best < before) g.ksplit = ksp;
       }
-    }
   }
 
   // Register-direct kernel for products with a skinny output side (N, or M
@@ -950,7 +947,7 @@ hipError_t launch_gemm_chain(hipStream_t s, const GemmArgs* es, int n) {
   }
   const GemmArgs& o = ch.e[0];
   if (o.M <= 0 || o.N <= 0) return hipSuccess;
-  if (o.kind != 0 || o.bk != 32 || o.ksplit != 1 || o.nsplit < 1 || (o.nsplit > 1 && !o.ws))
+  if (o.kind != 0 || o.bk != tile_bk(o.bm, o.bn) || o.ksplit != 1 || o.nsplit < 1 || (o.nsplit > 1 && !o.ws))
     return hipErrorInvalidValue;
   for (int i = 1; i < n; ++i)
     if (ch.e[i].M != o.M || ch.e[i].N != o.N || ch.e[i].prec != o.prec ||
@@ -968,10 +965,10 @@ hipError_t launch_gemm_chain(hipStream_t s, const GemmArgs* es, int n) {
   return launch_reduce(s, r);
 }
 
-// Grouped launches run the KS = 1, BK = 32 tile kernel; members share the
+// Grouped launches run the KS = 1 tile kernel; members share the
 // tile shape (after transposition) and the arithmetic.
 int64_t gemm_group_key(const GemmArgs& g0) {
-  if (g0.kind != 0 || g0.nsplit != 1 || g0.ksplit != 1 || g0.bk != 32) return -1;
+  if (g0.kind != 0 || g0.nsplit != 1 || g0.ksplit != 1 || g0.bk != tile_bk(g0.bm, g0.bn)) return -1;
   const GemmArgs g = g0.trans ? transposed(g0) : g0;
   return ((int64_t)g.bm * 1000 + g.bn) * 2 + g.prec;
 }

@@ -404,3 +404,25 @@ def test_fp32_storage_autotuned_plans(method, n, o, ob, rhf, monkeypatch):
     step = np.abs(t64 - vec).max()
     assert np.abs(t32 - t32m).max() <= 1e-6 * scale
     assert 1e-13 < np.abs(t32 - t64).max() < 1e-5 * step
+
+
+@pytest.mark.parametrize("method,n,o,ob,prec", [("CCSD", 19, 4, 3, 0), ("CCSD", 41, 6, 6, 0), ("CCSD", 41, 6, 6, 2),
+                                                ("CCSDT", 11, 3, 2, 0)])
+def test_wide_addresses_equal_narrow(method, n, o, ob, prec, monkeypatch):
+    """The tile kernel's 64-bit addressing (operands that reach 4 GiB; forced
+    with CCQ_HIP_WIDE=1) reads the same elements in the same order as its
+    32-bit forms: sweeps equal bit for bit."""
+    _say(f"case wide addresses {method} n={n} o={o} ob={ob} precision {prec}")
+    c = Case(n, o, 2 * n, 43, occ_b=ob)
+    vec = _state(c, method, 9)
+    out = []
+    for wide in ("0", "1"):
+        eng = _engine_env(c, method, monkeypatch, {"CCQ_HIP_WIDE": wide}, shift=0.02)
+        eng.set_t(vec)
+        eng.set_precision(prec)
+        for _ in range(2):
+            eng.update()
+        out.append((eng.energy(), eng.get_t()))
+        eng.close()
+    assert out[0][0] == out[1][0]
+    np.testing.assert_array_equal(out[1][1], out[0][1])
