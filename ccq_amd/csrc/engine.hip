@@ -23,6 +23,7 @@
 
 #include "../../include/ccq_hip.h"
 #include "kernels.h"
+#include "levels.h"
 #include "restart_io.h"
 
 #include "ir_ccsd_rhf.inc"
@@ -181,7 +182,6 @@ struct Section {
   // order, one launch each.
   std::vector<std::vector<int>> launches;
   std::vector<std::string> launch_cls;
-  std::vector<int> launch_level;   // dependency level of each launch (non-decreasing)
   // chains: member op indices (program order), their orientation against the
   // first member (1: transposed) and the launch plan over the concatenated K
   std::vector<std::vector<int>> chains;
@@ -242,17 +242,8 @@ struct ccq_hip_ctx {
   std::vector<std::unique_ptr<DevBuf>> view_buf;
   struct Gather { int t; int64_t rows, cols, t_src_row, t_src_col, t_dst_row, t_dst_col; };
   std::vector<Gather> gathers;
-  DevBuf ws;                 // split-K workspace (main stream)
-  // launches of one dependency level run concurrently on up to nstreams
-  // streams (the main one and side[0..nstreams-2], default priority), each
-  // with its own split-K workspace; CCQ_HIP_STREAMS=1 runs everything on the
-  // main stream
-  static constexpr int kMaxStreams = 4;
-  int nstreams = kMaxStreams;
-  hipStream_t side[kMaxStreams - 1] = {};
-  DevBuf ws_side[kMaxStreams - 1];
-  hipEvent_t fork_ev = nullptr, join_ev[kMaxStreams - 1] = {};
-  double* cur_ws = nullptr;  // workspace of the stream being launched on
+  DevBuf ws;                 // split-K workspace
+  double* cur_ws = nullptr;  // workspace of the launches (the autotuner's while it measures)
   int* itab = nullptr;
   double* dtab = nullptr;
   // program
@@ -297,6 +288,11 @@ struct ccq_hip_ctx {
 
   ~ccq_hip_ctx() {
     for (auto& kv : graphs) drop_graph(kv.second);
+    for (auto& kv : level_progs) {
+      if (kv.second.items) (void)hipFree(kv.second.items);
+      for (auto* t : kv.second.tasks)
+        if (t) (void)hipFree(t);
+    }
     for (float* p : f32_bufs) (void)hipFree(p);
     if (guess_params) (void)hipFree(guess_params);
     if (d3tab) (void)hipFree(d3tab);
@@ -305,11 +301,6 @@ struct ccq_hip_ctx {
     if (gather_tab) (void)hipFree(gather_tab);
     if (itab) (void)hipFree(itab);
     if (dtab) (void)hipFree(dtab);
-    for (auto& e : join_ev)
-      if (e) (void)hipEventDestroy(e);
-    if (fork_ev) (void)hipEventDestroy(fork_ev);
-    for (auto& st : side)
-      if (st) (void)hipStreamDestroy(st);
     if (stream) (void)hipStreamDestroy(stream);
   }
 
@@ -1671,19 +1662,10 @@ struct ccq_hip_ctx {
     for (auto& sec : sections) {
       sec.launches.clear();
       sec.launch_cls.clear();
-      sec.launch_level.clear();
     }
     group_gemms(dump_schedule);
     ws.alloc(std::max<int64_t>(ws_need, 1));
     cur_ws = ws.p;
-    if (nstreams > 1) {
-      HIPCHK(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming));
-      for (int k = 0; k < nstreams - 1; ++k) {
-        HIPCHK(hipStreamCreateWithFlags(&side[k], hipStreamNonBlocking));
-        HIPCHK(hipEventCreateWithFlags(&join_ev[k], hipEventDisableTiming));
-        ws_side[k].alloc(std::max<int64_t>(ws_need, 1));
-      }
-    }
     if (lsq_n) lsq.alloc(lsq_n);
     HIPCHK(hipMalloc(&tables32, sizeof(int) * std::max<size_t>(host32.size(), 1)));
     if (!host32.empty())
@@ -1693,6 +1675,12 @@ struct ccq_hip_ctx {
     HIPCHK(hipMalloc(&dtab, sizeof(double) * std::max<size_t>(dh.size(), 1)));
     if (!dh.empty())
       HIPCHK(hipMemcpy(dtab, dh.data(), sizeof(double) * dh.size(), hipMemcpyHostToDevice));
+    if (use_levels()) {
+      std::set<std::string> progs;
+      for (const auto& sec : sections) progs.insert(sec.prog);
+      for (const auto& prog : progs) build_levels(prog);
+      lv_ws.alloc(std::max<int64_t>(lv_ws_need, 1));
+    }
   }
 
   // Fold an add op (C (+)= c A) into the GEMM that next updates C, when that
@@ -1957,7 +1945,6 @@ struct ccq_hip_ctx {
         for (int i : idx) {
           sec.launches.push_back({i});
           sec.launch_cls.push_back(sec.ops[i].chain >= 0 ? chain_cls(sec, sec.ops[i].chain) : sec.ops[i].cls);
-          sec.launch_level.push_back((int)sec.launch_level.size());
         }
         continue;
       }
@@ -2119,11 +2106,9 @@ struct ccq_hip_ctx {
             sec.launch_cls.push_back(sec.ops[i].gemm ? group_cls(sec, it->second)
                                      : (sec.ops[i].part_of >= 0 || !sec.ops[i].flat ? "add:perm*" : "add:flat*") +
                                            std::to_string(it->second.size()));
-            sec.launch_level.push_back(lv);
           } else if (!grouped.count(i)) {
             sec.launches.push_back({i});
             sec.launch_cls.push_back(sec.ops[i].chain >= 0 ? chain_cls(sec, sec.ops[i].chain) : sec.ops[i].cls);
-            sec.launch_level.push_back(lv);
           }
         }
       }
@@ -2302,18 +2287,19 @@ struct ccq_hip_ctx {
       HIPCHK(ccqk::launch_gemm(stream, gemm_args(op)));
     } else {
       if (amp_in_fp64(1, [&](size_t) { return op.out; }, [&] { run_op(op); })) return;
-      const int io32 = run_prec == 2;
-      const double* A = sp(op.a);
-      double* C = sp(op.out);
-      // the float form has no alignment condition
-      const bool aligned =
-          io32 || ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(C)) & 15) == 0;
-      if (op.flat && aligned)
-        HIPCHK(ccqk::launch_axpy_flat(stream, op.M * op.N, A, C, op.coef, acc, io32));
-      else
-        HIPCHK(ccqk::launch_perm_add(stream, op.M, op.N, A, tables32 + op.t_rowA, tables32 + op.t_kA, C,
-                                     tables32 + op.t_rowC, tables32 + op.t_colC, op.coef, acc, io32));
+      run_add(op, sp(op.a), sp(op.out), acc);
     }
+  }
+
+  void run_add(const Op& op, const double* A, double* C, int acc) {
+    const int io32 = run_prec == 2;
+    // the float form has no alignment condition
+    const bool aligned = io32 || ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(C)) & 15) == 0;
+    if (op.flat && aligned)
+      HIPCHK(ccqk::launch_axpy_flat(stream, op.M * op.N, A, C, op.coef, acc, io32));
+    else
+      HIPCHK(ccqk::launch_perm_add(stream, op.M, op.N, A, tables32 + op.t_rowA, tables32 + op.t_kA, C,
+                                   tables32 + op.t_rowC, tables32 + op.t_colC, op.coef, acc, io32));
   }
 
   ccqk::UpdateParams update_params(const UpdateStep& u) const {
@@ -2426,6 +2412,7 @@ struct ccq_hip_ctx {
 
   void run_graphed(const std::string& prog, double key = 0.0) {
     if (prog == "sweep" && prec == 2) prep_sweep32();
+    if (use_levels() && !profile) prep_levels(prog);
     if (!use_graph || profile) {
       run_program(prog);
       return;
@@ -2457,68 +2444,511 @@ struct ccq_hip_ctx {
     run_program("sweep", nsec);
   }
 
-  std::string cur_sec;   // section being run (profile attribution)
+  // ---- level launches --------------------------------------------------------
+  // A program's sections as dependency levels over the whole program
+  // (levels.h), each level one launch of the level kernel (products as tiles,
+  // adds, split-K completions, sums of partial accumulators) after the
+  // operations that keep a launch of their own: amplitude updates and copies,
+  // large adds, and products that the register-direct kernel streams faster.
+  // One stream, so the captured graph is a chain: a graph with parallel
+  // branches costs about 4 us of host time a node when it is launched (CCSD 24
+  // orbitals: 870 us for 176 nodes, as long as the sweep itself), a chain 0.4.
+  // Profiling and CCQ_HIP_GROUP=0 run the sections' own launches.
+  struct LevelStep {
+    std::vector<std::pair<int, int>> own;   // (section, op or -1: the whole section)
+    std::vector<int> own_task;              // for an op: its task (arguments), else -1
+    int64_t item0 = 0;
+    int nitems = 0;
+  };
+  struct SlotBuf {
+    int tensor = -1, slot = 0;
+    DevBuf buf;
+    float* p32 = nullptr;
+  };
+  // what a task is built from, for either storage
+  struct TaskSrc {
+    int kind = 0;
+    int sec = -1, op = -1;            // products and adds
+    int tensor = -1, slot = 0;        // destination
+    int nslots = 0;                   // kLvSum
+    bool overwrite = false;
+    ccqk::GemmArgs plan{};            // products: tile, split (kLvReduce: of its product)
+    int64_t ws_off = -1;              // split-K partials in lv_ws
+    int chunk = 0, pshift = 0;
+  };
+  struct LevelProg {
+    std::vector<LevelStep> steps;
+    std::vector<TaskSrc> src;
+    ccqk::LevelItem* items = nullptr;
+    ccqk::LevelTask* tasks[2] = {nullptr, nullptr};   // FP64 storage, FP32 storage
+    std::vector<ccqk::LevelTask> host[2];             // the same, for the operations with a launch of their own
+  };
+  std::map<std::string, LevelProg> level_progs;
+  std::map<std::pair<int, int>, std::unique_ptr<SlotBuf>> slot_bufs;   // (canonical tensor, slot)
+  DevBuf lv_ws;
+  int64_t lv_ws_need = 0;
+  bool use_levels() const { return group; }
 
-  // rough launch time (s) of launch k of a section: MFMA or HBM bound plus a
-  // fixed cost
-  double launch_cost(const Section& sec, size_t k) const {
-    double fl = 0, by = 0;
-    const auto& L = sec.launches[k];
-    std::vector<int> mem = L;
-    if (L.size() == 1 && sec.ops[L[0]].chain >= 0) mem = sec.chains[sec.ops[L[0]].chain];
-    for (int i : mem) fl += sec.ops[i].flops, by += sec.ops[i].bytes;
-    return std::max(fl / 40e12, by / 3e12) + 4e-6;
+  int64_t tensor_size(int t) const {
+    int64_t n = 1;
+    for (int i = 0; i < tensors[t].rank; ++i) n *= tensors[t].dims[i];
+    return std::max<int64_t>(n, 1);
+  }
+  ccqlv::Key key_of(int t) const { return reinterpret_cast<ccqlv::Key>(tensors[t].ptr); }
+
+  // cycles of one workgroup on a tile of the product, its MFMAs alone, and
+  // the tiles: a slab costs about 150 cycles beside its MFMAs, the first
+  // operands and the epilogue about 4000
+  struct TileCost {
+    double item, mfma;
+    int64_t tiles;
+  };
+  static TileCost tile_cost(int64_t M, int64_t N, int64_t K, int bm, int bn) {
+    const int bk = ccqk::tile_bk(bm, bn);
+    const double slabs = (double)((K + bk - 1) / bk);
+    const double slab = (bm / 32.0) * (bn / 32.0) * (bk / 4.0) * 64.0;
+    // a workgroup alone on its CU waits about 700 cycles a slab (gemm_plan_ranked)
+    return {slabs * std::max(slab + 150.0, 1200.0) + 4000.0 + bm * bn / 2.0, slabs * slab,
+            ((M + bm - 1) / bm) * ((N + bn - 1) / bn)};
   }
 
-  // The launches [a, b) of one dependency level (independent of each other:
-  // no two write the same tensor or read what another writes) on up to
-  // nstreams streams: longest first, each to the least loaded stream.  The
-  // side streams wait for the main stream's work so far and the main stream
-  // waits for theirs at the end, so the next level starts after all of this
-  // one (also under graph capture, where this becomes a fork / join).
-  template <typename F>
-  void run_level(const Section& sec, size_t a, size_t b, F&& run_launch) {
-    const int ns = std::min<int>(nstreams, (int)(b - a));
-    std::vector<size_t> order;
-    for (size_t k = a; k < b; ++k) order.push_back(k);
-    std::vector<double> cost(b - a);
-    for (size_t k = a; k < b; ++k) cost[k - a] = launch_cost(sec, k);
-    std::stable_sort(order.begin(), order.end(),
-                     [&](size_t x, size_t y) { return cost[x - a] > cost[y - a]; });
-    std::vector<double> load(ns, 0.0);
-    std::vector<int> where(b - a, 0);
-    for (size_t k : order) {
-      const int s = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-      where[k - a] = s;
-      load[s] += cost[k - a];
-    }
-    HIPCHK(hipEventRecord(fork_ev, stream));
-    for (int s = 1; s < ns; ++s) HIPCHK(hipStreamWaitEvent(side[s - 1], fork_ev, 0));
-    hipStream_t main = stream;
-    for (size_t k = a; k < b; ++k) {
-      const int s = where[k - a];
-      stream = s ? side[s - 1] : main;
-      cur_ws = s ? ws_side[s - 1].p : ws.p;
-      try {
-        run_launch(k);
-      } catch (...) {
-        stream = main;
-        cur_ws = ws.p;
-        throw;
+  // tile of a product in a level launch: the shape with the least time if it
+  // had the chip to itself plus its share of the chip's time
+  ccqk::GemmArgs level_plan(const Op& op) const {
+    ccqk::GemmArgs g = op.plan;
+    g.kind = 0;
+    g.ksplit = 1;
+    g.nsplit = 1;
+    g.trans = (g.c_mfast && !g.c_nfast) ? 1 : 0;
+    const int64_t M = g.trans ? op.N : op.M, N = g.trans ? op.M : op.N;
+    double best = 1e300;
+    const bool f64 = op.plan.kind == 1;   // register-direct products are FP64 in every precision mode
+    for (int bm : {64, 32})
+      for (int bn : {64, 32}) {
+        if (f64 && (bm != 32 || bn != 32)) continue;
+        const TileCost c = tile_cost(M, N, op.K, bm, bn);
+        const double share = c.tiles * std::max(c.mfma, c.item / 3.0) / 256.0;
+        const double t = std::max(share, c.item) + share;
+        if (t < best) {
+          best = t;
+          g.bm = bm;
+          g.bn = bn;
+        }
+      }
+    g.bk = ccqk::tile_bk(g.bm, g.bn);
+    g.kchunk = (op.K + g.bk - 1) / g.bk * g.bk;
+    return g;
+  }
+  // the chip's time the product takes (cycles)
+  static double level_share(const Op& op, const ccqk::GemmArgs& g) {
+    const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, g.bm, g.bn);
+    return c.tiles * std::max(c.mfma, c.item / 3.0) / 256.0;
+  }
+
+  // operations that keep their own launch
+  bool own_launch(const Op& op) const {
+    if (!op.gemm) return tensors[op.out].kind == TKind::Amp || (op.M * op.N >= kOwnAdd && op.part_of < 0);
+    // a short summed range and one long side: store bound, and the
+    // register-direct kernel streams it (5 x 1071875 x 5: 2.2 TB/s)
+    return op.plan.kind == 1 && op.K <= 64 && op.M * op.N >= kOwnStream;
+  }
+  static constexpr int64_t kOwnAdd = 1 << 21, kOwnStream = 1 << 19;
+
+  void build_levels(const std::string& prog) {
+    LevelProg& lp = level_progs[prog];
+    // units in program order; parts of one op form one unit
+    struct Src {
+      int sec;
+      std::vector<int> ops;   // empty: the whole section
+    };
+    std::vector<Src> us;
+    std::vector<ccqlv::Unit> units;
+    auto amp_key = [&](const std::string& b, bool left) {
+      return reinterpret_cast<ccqlv::Key>((left ? lvec.p : tvec.p) + blk_off.at(dimkey(b)));
+    };
+    for (int si = 0; si < (int)sections.size(); ++si) {
+      const Section& sec = sections[si];
+      if (sec.prog != prog) continue;
+      if (sec.kind == Section::Compute) {
+        for (int i = 0; i < (int)sec.ops.size(); ++i) {
+          const Op& op = sec.ops[i];
+          if (op.fused) continue;
+          if (op.part_of >= 0 && !us.empty() && us.back().sec == si && !us.back().ops.empty() &&
+              sec.ops[us.back().ops[0]].part_of == op.part_of) {
+            us.back().ops.push_back(i);
+            continue;
+          }
+          ccqlv::Unit u;
+          u.reads.push_back(key_of(op.a));
+          if (op.gemm) u.reads.push_back(key_of(op.b));
+          if (op.fuse_a >= 0) u.reads.push_back(key_of(op.fuse_a));
+          u.writes.push_back(key_of(op.out));
+          u.term = true;
+          u.assign = op.assign;
+          u.full = !op.restricted && op.t_rowC2 < 0 && op.t_colC2 < 0;
+          u.size = tensor_size(op.out);
+          // the amplitudes hold no partial accumulators
+          if (tensors[op.out].kind == TKind::Amp) u.term = false;
+          us.push_back({si, {i}});
+          units.push_back(u);
+        }
+      } else {
+        ccqlv::Unit u;
+        if (sec.kind == Section::Update) {
+          u.reads = {key_of(sec.upd.resid), amp_key(sec.upd.block, sec.upd.left)};
+          u.writes = {amp_key(sec.upd.block, sec.upd.left)};
+        } else if (sec.kind == Section::Copy) {
+          u.reads = {amp_key(sec.src, false)};
+          u.writes = {amp_key(sec.dst, false)};
+        } else {
+          u.barrier = true;
+        }
+        us.push_back({si, {}});
+        units.push_back(u);
       }
     }
-    stream = main;
-    cur_ws = ws.p;
-    for (int s = 1; s < ns; ++s) {
-      HIPCHK(hipEventRecord(join_ev[s - 1], side[s - 1]));
-      HIPCHK(hipStreamWaitEvent(stream, join_ev[s - 1], 0));
+    // a term with an output part that no first term writes (an assigning op
+    // over irrep blocks or P-space rectangles) is never a slot's overwrite:
+    // full is false there, so its slot starts from zeros
+    auto schedule = [&](std::vector<ccqlv::Unit>& v) {
+      ccqlv::Scheduler sch;
+      sch.run(v);
+      return sch;
+    };
+    // first pass: levels without K splits, and the chip time of each
+    std::vector<std::vector<ccqk::GemmArgs>> plans(units.size());
+    for (size_t u = 0; u < units.size(); ++u)
+      for (int i : us[u].ops) {
+        const Op& op = sections[us[u].sec].ops[i];
+        plans[u].push_back(op.gemm ? level_plan(op) : ccqk::GemmArgs{});
+      }
+    std::vector<ccqlv::Unit> first = units;
+    ccqlv::Scheduler s1 = schedule(first);
+    std::vector<double> load(s1.levels + 1, 0.0);
+    for (size_t u = 0; u < units.size(); ++u)
+      for (size_t k = 0; k < us[u].ops.size(); ++k) {
+        const Op& op = sections[us[u].sec].ops[us[u].ops[k]];
+        if (op.gemm && !own_launch(op)) load[first[u].level] += level_share(op, plans[u][k]);
+      }
+    // a product whose single workgroups would outlast their level by more than
+    // the extra level of a split is split along K
+    std::vector<int64_t> partials(s1.levels + 1, 0);
+    for (size_t u = 0; u < units.size(); ++u)
+      for (size_t k = 0; k < us[u].ops.size(); ++k) {
+        const Op& op = sections[us[u].sec].ops[us[u].ops[k]];
+        if (!op.gemm || own_launch(op) || op.K == 0) continue;
+        ccqk::GemmArgs& g = plans[u][k];
+        const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, g.bm, g.bn);
+        const double span = std::max(load[first[u].level], kSplitSpan);
+        if (c.item < span + kSplitGain) continue;
+        const int64_t slabs = (op.K + g.bk - 1) / g.bk;
+        int64_t split = (int64_t)std::ceil((c.item - 4000.0) / std::max(span - 4000.0, 4000.0));
+        split = std::min({split, slabs / 4, (int64_t)256, std::max<int64_t>(1, kSplitMax / (op.M * op.N))});
+        if (split < 2) continue;
+        if ((partials[first[u].level] += split * op.M * op.N) > kLevelPartials) continue;
+        const int64_t per = (slabs + split - 1) / split;
+        g.nsplit = (int)((slabs + per - 1) / per);
+        g.kchunk = per * g.bk;
+        if (g.nsplit > 1) units[u].lat = 2;
+      }
+    ccqlv::Scheduler sch = schedule(units);
+    lp.steps.assign((size_t)sch.levels, {});
+
+    // tasks and items
+    struct Pending {
+      int task;
+      int64_t n;
+      double cost;
+    };
+    std::vector<std::vector<Pending>> at((size_t)sch.levels);
+    std::vector<int64_t> ws_used((size_t)sch.levels, 0);   // partials written on each level
+    std::map<ccqlv::Key, int> canon;   // a tensor of every accumulator
+    for (size_t u = 0; u < units.size(); ++u)
+      for (int i : us[u].ops) {
+        const int t = sections[us[u].sec].ops[i].out;
+        canon.emplace(key_of(t), t);
+      }
+    auto tensor_of = [&](ccqlv::Key k) { return canon.at(k); };
+    auto slot_of_tensor = [&](int t, int s) {
+      if (!s) return;
+      auto& b = slot_bufs[{t, s}];
+      if (b) return;
+      b.reset(new SlotBuf);
+      b->tensor = t;
+      b->slot = s;
+      b->buf.alloc(tensor_size(t));
+    };
+    auto items_of = [&](int64_t total, int chunk) { return (total + chunk - 1) / chunk; };
+    for (size_t u = 0; u < units.size(); ++u) {
+      const ccqlv::Unit& un = units[u];
+      const int si = us[u].sec;
+      if (us[u].ops.empty()) {
+        lp.steps[un.level].own.emplace_back(si, -1);
+        lp.steps[un.level].own_task.push_back(-1);
+        continue;
+      }
+      for (size_t k = 0; k < us[u].ops.size(); ++k) {
+        const int oi = us[u].ops[k];
+        const Op& op = sections[si].ops[oi];
+        if (op.M <= 0 || op.N <= 0) continue;
+        if (tensors[op.out].kind == TKind::Amp) {
+          lp.steps[un.level].own.emplace_back(si, oi);
+          lp.steps[un.level].own_task.push_back(-1);
+          continue;
+        }
+        TaskSrc ts;
+        ts.sec = si;
+        ts.op = oi;
+        ts.tensor = tensor_of(key_of(op.out));
+        ts.slot = un.slot;
+        ts.overwrite = un.overwrite;
+        slot_of_tensor(ts.tensor, ts.slot);
+        int64_t n;
+        double cost;
+        if (op.gemm) {
+          ts.plan = plans[u][k];
+          if (own_launch(op)) {
+            ts.plan = op.plan;
+            lp.steps[un.level].own.emplace_back(si, oi);
+            lp.steps[un.level].own_task.push_back((int)lp.src.size());
+            lp.src.push_back(ts);
+            continue;
+          }
+          const ccqk::GemmArgs& g = ts.plan;
+          const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, g.bm, g.bn);
+          ts.kind = op.plan.kind == 1 ? ccqk::kLvTileF64
+                                      : g.bm == 64 ? (g.bn == 64 ? ccqk::kLvTile6464 : ccqk::kLvTile6432)
+                                                   : (g.bn == 64 ? ccqk::kLvTile3264 : ccqk::kLvTile3232);
+          n = c.tiles * g.nsplit;
+          cost = c.item / g.nsplit;
+          if (g.nsplit > 1) {
+            ts.ws_off = ws_used[un.level];
+            ws_used[un.level] += g.nsplit * op.M * op.N;
+            TaskSrc r = ts;
+            r.kind = ccqk::kLvReduce;
+            while ((1 << r.pshift) < g.nsplit && r.pshift < 5 && op.M * op.N * (2 << r.pshift) <= 262144) ++r.pshift;
+            r.chunk = 256 >> r.pshift;
+            at[un.level + 1].push_back({(int)lp.src.size(), items_of(op.M * op.N, r.chunk), 3000.0});
+            lp.src.push_back(r);
+          }
+        } else {
+          if (own_launch(op)) {
+            lp.steps[un.level].own.emplace_back(si, oi);
+            lp.steps[un.level].own_task.push_back((int)lp.src.size());
+            lp.src.push_back(ts);
+            continue;
+          }
+          ts.kind = op.flat ? ccqk::kLvFlat : ccqk::kLvPerm;
+          ts.chunk = 1024;
+          n = items_of(op.M * op.N, ts.chunk);
+          cost = 3000.0;
+        }
+        at[un.level].push_back({(int)lp.src.size(), n, cost});
+        lp.src.push_back(ts);
+      }
+    }
+    for (const auto& sm : sch.sums) {
+      TaskSrc ts;
+      ts.kind = ccqk::kLvSum;
+      ts.tensor = tensor_of(sm.out);
+      ts.nslots = sm.nslots;
+      ts.chunk = 1024;
+      at[sm.level].push_back({(int)lp.src.size(), items_of(tensor_size(ts.tensor), ts.chunk), 3000.0});
+      lp.src.push_back(ts);
+    }
+    for (const auto& z : sch.zeros) {
+      TaskSrc ts;
+      ts.kind = ccqk::kLvZero;
+      ts.tensor = tensor_of(z.out);
+      ts.slot = z.slot;
+      ts.chunk = 4096;
+      slot_of_tensor(ts.tensor, ts.slot);
+      at[z.level].push_back({(int)lp.src.size(), items_of(tensor_size(ts.tensor), ts.chunk), 1000.0});
+      lp.src.push_back(ts);
+    }
+    // the partials of one level are reduced on the next: two halves by parity
+    int64_t half = 0;
+    for (int64_t w : ws_used) half = std::max(half, w);
+    lv_ws_need = std::max(lv_ws_need, 2 * half);
+    for (size_t l = 0; l < at.size(); ++l)
+      for (const Pending& p : at[l]) {
+        TaskSrc& ts = lp.src[p.task];
+        if (ts.ws_off < 0) continue;
+        const size_t made = ts.kind == ccqk::kLvReduce ? l - 1 : l;   // level the partials are written on
+        if (made & 1) ts.ws_off += half;
+      }
+    // items: longest first; consecutive workgroups go to the eight XCDs in
+    // turn, so every operation's tiles are dealt in eight contiguous runs
+    std::vector<ccqk::LevelItem> items;
+    for (size_t l = 0; l < at.size(); ++l) {
+      auto& v = at[l];
+      std::stable_sort(v.begin(), v.end(), [](const Pending& a, const Pending& b) { return a.cost > b.cost; });
+      std::vector<ccqk::LevelItem> q[8];
+      int turn = 0;
+      for (const Pending& p : v) {
+        if (p.n > 0x7fffffffLL) throw Fail("level task too large");
+        const int64_t base = p.n / 8, rem = p.n % 8;
+        int64_t i = 0;
+        for (int x = 0; x < 8; ++x) {
+          const int64_t c = base + (x < rem ? 1 : 0);
+          auto& dst = q[(turn + x) & 7];
+          for (int64_t e = 0; e < c; ++e) dst.push_back({p.task, (int)i++});
+        }
+        turn = (turn + (int)rem) & 7;
+      }
+      size_t longest = 0;
+      for (auto& x : q) longest = std::max(longest, x.size());
+      lp.steps[l].item0 = (int64_t)items.size();
+      for (size_t i = 0; i < longest; ++i)
+        for (auto& x : q) items.push_back(i < x.size() ? x[i] : ccqk::LevelItem{-1, 0});
+      lp.steps[l].nitems = (int)((int64_t)items.size() - lp.steps[l].item0);
+    }
+    HIPCHK(hipMalloc(&lp.items, sizeof(ccqk::LevelItem) * std::max<size_t>(items.size(), 1)));
+    if (!items.empty())
+      HIPCHK(hipMemcpy(lp.items, items.data(), sizeof(ccqk::LevelItem) * items.size(), hipMemcpyHostToDevice));
+    if (dump_schedule)
+      for (size_t l = 0; l < at.size(); ++l) {
+        std::fprintf(stderr, "[levels] %s level %zu: %d items, %zu own launches\n", prog.c_str(), l, lp.steps[l].nitems,
+                     lp.steps[l].own.size());
+        for (const Pending& p : at[l]) {
+          const TaskSrc& ts = lp.src[p.task];
+          std::fprintf(stderr, "[levels]   kind %d %s -> %s slot %d items %lld cost %.0f split %d\n", ts.kind,
+                       ts.op >= 0 ? sections[ts.sec].ops[ts.op].cls.c_str() : "", tensors[ts.tensor].id.c_str(), ts.slot,
+                       (long long)p.n, p.cost, ts.plan.nsplit);
+        }
+        for (auto& o : lp.steps[l].own)
+          std::fprintf(stderr, "[levels]   own %s %s\n", sections[o.first].name.c_str(),
+                       o.second >= 0 ? sections[o.first].ops[o.second].cls.c_str() : "");
+      }
+  }
+
+  // device task table of a program for the storage of run_prec
+  void bind_levels(LevelProg& lp, int st) {
+    if (lp.tasks[st]) return;
+    auto dst = [&](int t, int s) -> double* {
+      if (!s) return sp(t);
+      SlotBuf& b = *slot_bufs.at({t, s});
+      return st ? reinterpret_cast<double*>(b.p32) : b.buf.p;
+    };
+    std::vector<ccqk::LevelTask>& v = lp.host[st];
+    v.assign(lp.src.size(), ccqk::LevelTask{});
+    for (size_t i = 0; i < lp.src.size(); ++i) {
+      const TaskSrc& ts = lp.src[i];
+      ccqk::LevelTask& t = v[i];
+      t.kind = ts.kind;
+      t.chunk = ts.chunk;
+      t.pshift = ts.pshift;
+      ccqk::GemmArgs& g = t.g;
+      if (ts.kind == ccqk::kLvSum || ts.kind == ccqk::kLvZero) {
+        g.M = tensor_size(ts.tensor);
+        g.N = 1;
+        g.C = dst(ts.tensor, ts.kind == ccqk::kLvSum ? 0 : ts.slot);
+        t.nsrc = ts.kind == ccqk::kLvSum ? ts.nslots - 1 : 0;
+        for (int k = 0; k < t.nsrc; ++k) t.src[k] = dst(ts.tensor, k + 1);
+        continue;
+      }
+      const Op& op = sections[ts.sec].ops[ts.op];
+      if (op.gemm) {
+        g = gemm_args(op);
+        if (ts.kind != 0) {
+          copy_plan(g, ts.plan);
+          g.group = 1;
+          const int64_t tm = ((g.trans ? op.N : op.M) + g.bm - 1) / g.bm;
+          const int64_t tiles = tm * (((g.trans ? op.M : op.N) + g.bn - 1) / g.bn);
+          g.group = (int)std::max<int64_t>(1, std::min<int64_t>(tm, std::lround(std::sqrt((double)tiles * g.nsplit / 8.0))));
+          g = ccqk::gemm_oriented(g);
+          if (ts.ws_off >= 0) g.ws = lv_ws.p + ts.ws_off;
+        }
+      } else {
+        g.M = op.M;
+        g.N = op.N;
+        g.A = sp(op.a);
+        g.rowA = tables32 + op.t_rowA;
+        g.kA = tables32 + op.t_kA;
+        g.rowC = tables32 + op.t_rowC;
+        g.colC = tables32 + op.t_colC;
+        g.alpha = op.coef;
+        if (op.M * op.N > 0x7fffffffLL) throw Fail("level add too large");
+      }
+      g.C = dst(ts.tensor, ts.slot);
+      g.accumulate = ts.overwrite ? 0 : 1;
+    }
+    HIPCHK(hipMalloc(&lp.tasks[st], sizeof(ccqk::LevelTask) * std::max<size_t>(v.size(), 1)));
+    if (!v.empty())
+      HIPCHK(hipMemcpy(lp.tasks[st], v.data(), sizeof(ccqk::LevelTask) * v.size(), hipMemcpyHostToDevice));
+  }
+
+  // outside any capture: the schedule of a program and its tables
+  void prep_levels(const std::string& prog) {
+    const int st = (prog == "sweep" ? prec : std::min(prec, 1)) == 2;
+    if (!level_progs.count(prog)) throw Fail("no level schedule of program " + prog);
+    LevelProg& lp = level_progs.at(prog);
+    if (lp.tasks[st]) return;
+    if (st)
+      for (auto& kv : slot_bufs) {
+        SlotBuf& b = *kv.second;
+        if (b.p32) continue;
+        HIPCHK(hipMalloc(&b.p32, sizeof(float) * tensor_size(b.tensor)));
+        f32_bufs.push_back(b.p32);
+      }
+    const int keep = run_prec;
+    run_prec = st ? 2 : 0;
+    try {
+      bind_levels(lp, st);
+    } catch (...) {
+      run_prec = keep;
+      throw;
+    }
+    run_prec = keep;
+  }
+
+  void run_levels(const std::string& prog) {
+    LevelProg& lp = level_progs.at(prog);
+    const int st = run_prec == 2;
+    for (const LevelStep& step : lp.steps) {
+      for (size_t k = 0; k < step.own.size(); ++k) {
+        const Section& sec = sections[step.own[k].first];
+        const int oi = step.own[k].second;
+        cur_sec = sec.name;
+        if (oi < 0) {
+          if (sec.kind == Section::Update) run_update(sec.upd);
+          else if (sec.kind == Section::Copy) run_copy(sec.dst, sec.src);
+          else run_cct3(sec.upd);
+          continue;
+        }
+        const Op& op = sec.ops[oi];
+        if (step.own_task[k] < 0) {
+          run_op(op);
+          continue;
+        }
+        ccqk::GemmArgs g = lp.host[st][step.own_task[k]].g;
+        if (op.gemm) {
+          g.prec = run_prec;
+          g.ws = cur_ws;
+          HIPCHK(ccqk::launch_gemm(stream, g));
+        } else {
+          run_add(op, g.A, g.C, g.accumulate);
+        }
+      }
+      HIPCHK(ccqk::launch_level(stream, run_prec, lp.tasks[st], lp.items + step.item0, step.nitems));
     }
   }
+  // a single workgroup's cycles below which splitting never pays, and what the
+  // extra level costs
+  static constexpr double kSplitSpan = 12000.0, kSplitGain = 10000.0;
+  // partials of one product and of one level (doubles)
+  static constexpr int64_t kSplitMax = 4 << 20, kLevelPartials = 32 << 20;
+
+  std::string cur_sec;   // section being run (profile attribution)
 
   void run_program(const std::string& prog, int64_t nsec = -1) {
     if (!ints_ready) throw Fail("integrals not uploaded");
     run_prec = prog == "sweep" ? prec : std::min(prec, 1);
     if (run_prec == 2 && (!f32_ready || views32_stale)) throw Fail("FP32 shadows not prepared");
+    if (use_levels() && !profile && nsec < 0) {
+      run_levels(prog);
+      return;
+    }
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (profile) {
       HIPCHK(hipEventCreate(&e0));
@@ -2582,16 +3012,7 @@ struct ccq_hip_ctx {
             else
               timed(sec.launch_cls[k], fl, by, [&] { run_add_group(sec, L); });
           };
-          for (size_t a = 0; a < sec.launches.size();) {
-            size_t b = a + 1;
-            while (b < sec.launches.size() && sec.launch_level[b] == sec.launch_level[a]) ++b;
-            if (b - a == 1 || nstreams == 1 || profile) {
-              for (size_t k = a; k < b; ++k) run_launch(k);
-            } else {
-              run_level(sec, a, b, run_launch);
-            }
-            a = b;
-          }
+          for (size_t k = 0; k < sec.launches.size(); ++k) run_launch(k);
         }
       } else if (sec.kind == Section::Update) {
         const Tensor& R = tensors[sec.upd.resid];
@@ -2712,6 +3133,7 @@ struct ccq_hip_ctx {
   // hbar2 + add_twobody_hbar (src/hbar.f90:10-720) from the current T1, T2
   void hbar() {
     if (!tail) throw Fail("H-bar needs the CC(t;3) program (level 6)");
+    if (use_levels() && !profile) prep_levels("hbar");
     run_program("hbar");
     auto diag = [&](const char* src, int64_t n, double* dst) {
       HIPCHK(ccqk::launch_diag(stream, tens(src).ptr, n, n, dst));
@@ -2907,6 +3329,7 @@ struct ccq_hip_ctx {
       HIPCHK(ccqk::launch_hadamard_sum(stream, h.M, h.K, h.X, d3tab + h.xr, d3tab + h.xk, h.Y,
                                        d3tab + h.yr, d3tab + h.yk, tensors[h.out].ptr, h.scale));
     HIPCHK(hipMemsetAsync(cpart.p, 0, sizeof(double) * cpart.n, stream));
+    if (use_levels() && !profile) prep_levels("cct3");
     run_program("cct3");
     host_partial.resize((size_t)cpart.n);
     HIPCHK(hipMemcpyAsync(host_partial.data(), cpart.p, sizeof(double) * cpart.n,
@@ -3128,8 +3551,6 @@ int ccq_hip_create(const ccq_hip_dims* dims, const ccq_hip_opts* opts, ccq_hip_c
     if (const char* g = std::getenv("CCQ_HIP_GROUP_REG")) ctx->group_reg = std::string(g) != "0";
     if (const char* g = std::getenv("CCQ_HIP_WIDE")) ctx->wide_all = std::string(g) == "1";
     if (const char* g = std::getenv("CCQ_HIP_MERGE")) ctx->merge_sections = std::string(g) != "0";
-    if (const char* g = std::getenv("CCQ_HIP_STREAMS"))
-      ctx->nstreams = std::max(1, std::min(ccq_hip_ctx::kMaxStreams, std::atoi(g)));
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     ctx->layout();

@@ -91,6 +91,16 @@ __device__ __forceinline__ int xcd_logical(int lin, int total) {
   return xcd < r ? xcd * (q + 1) + slot : r * (q + 1) + (xcd - r) * q + slot;
 }
 
+// tile pid of tm x tn in groups of `group` tile rows
+__device__ __forceinline__ void tile_in_group(int pid, int tm, int tn, int group, int& tx, int& ty) {
+  const int gsize = group * tn;
+  const int first = (pid / gsize) * group;
+  const int gm = tm - first < group ? tm - first : group;
+  const int in = pid - (pid / gsize) * gsize;
+  tx = first + in % gm;
+  ty = in / gm;
+}
+
 __device__ __forceinline__ void tile_coords(int group, int& tx, int& ty, int& tz) {
   const int tm = gridDim.x, tn = gridDim.y;
   const int total = tm * tn * (int)gridDim.z;
@@ -98,13 +108,7 @@ __device__ __forceinline__ void tile_coords(int group, int& tx, int& ty, int& tz
   const int logical = xcd_logical(lin, total);
   const int per_z = tm * tn;
   tz = logical / per_z;
-  const int pid = logical - tz * per_z;
-  const int gsize = group * tn;
-  const int first = (pid / gsize) * group;
-  const int gm = tm - first < group ? tm - first : group;
-  const int in = pid - (pid / gsize) * gsize;
-  tx = first + in % gm;
-  ty = in / gm;
+  tile_in_group(logical - tz * per_z, tm, tn, group, tx, ty);
 }
 
 // Grouped launch (1-D grid over the tiles of every member): the member owning
@@ -120,14 +124,7 @@ __device__ __forceinline__ int group_tile(const GemmGroup& gg, int& tx, int& ty)
     if (i < gg.n && logical >= gg.start[i]) mem = i;
   const GemmArgs& g = gg.g[mem];
   const int tm = (int)((g.M + BM - 1) / BM), tn = (int)((g.N + BN - 1) / BN);
-  const int pid = logical - gg.start[mem];
-  const int group = g.group;
-  const int gsize = group * tn;
-  const int first = (pid / gsize) * group;
-  const int gm = tm - first < group ? tm - first : group;
-  const int in = pid - (pid / gsize) * gsize;
-  tx = first + in % gm;
-  ty = in / gm;
+  tile_in_group(logical - gg.start[mem], tm, tn, g.group, tx, ty);
   return mem;
 }
 
@@ -711,6 +708,126 @@ __global__ __launch_bounds__(256, kTileWaves<1>) void gemm_tab_group(GemmGroup g
   gemm_tab_tile<T, IO, BM, BN, BK, 1>(gg.g[mem], tx, ty, 0, smem);
 }
 
+// One dependency level (launch_level).  Bodies of every task kind in one kernel:
+// the operations of a level are a few microseconds each, most of it latency
+// (descriptor, tables, operands), so a launch per operation costs 3 - 4 us of
+// GPU time, or 4 us of host time each in a graph with parallel branches; side
+// by side in one launch they share that latency.  CCSD 24 orbitals: 919 us a
+// sweep as 176 launches, 185 us in 27 levels.
+// The descriptors are read through the constant address space: nothing
+// writes them while the kernel runs, so they stay scalar loads.
+template <typename IO>
+__device__ __forceinline__ void level_add(const LevelTask& t, int idx) {
+  const GemmArgs& g = t.g;
+  const uint32_t N = (uint32_t)g.N, total = (uint32_t)(g.M * g.N);
+  const uint32_t e0 = (uint32_t)idx * (uint32_t)t.chunk;
+  const uint32_t e1 = total - e0 < (uint32_t)t.chunk ? total : e0 + (uint32_t)t.chunk;
+  const bool flat = t.kind == kLvFlat;
+  for (uint32_t b = e0 + threadIdx.x; b < e1; b += 1024) {
+    int64_t ia[4], ic[4];
+    double v[4], c[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t e = b + 256u * j < e1 ? b + 256u * j : b;
+      if (flat) {
+        ia[j] = ic[j] = e;
+      } else {
+        const uint32_t r = e / N, n = e - r * N;
+        ia[j] = (int64_t)g.rowA[r] + g.kA[n];
+        ic[j] = (int64_t)g.rowC[r] + g.colC[n];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[j] = ldg<IO>(g.A, ia[j]);
+      c[j] = g.accumulate ? ldg<IO>(g.C, ic[j]) : 0.0;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (b + 256u * j < e1) stg<IO>(g.C, ic[j], g.accumulate ? c[j] + g.alpha * v[j] : g.alpha * v[j]);
+  }
+}
+
+template <typename IO>
+__device__ __forceinline__ void level_sum(const LevelTask& t, int idx) {
+  const int64_t total = t.g.M, e0 = (int64_t)idx * t.chunk;
+  const int64_t e1 = e0 + t.chunk < total ? e0 + t.chunk : total;
+  for (int64_t e = e0 + threadIdx.x; e < e1; e += 256) {
+    double v[kMaxLevelSrc];
+#pragma unroll
+    for (int k = 0; k < kMaxLevelSrc; ++k) v[k] = k < t.nsrc ? ldg<IO>(t.src[k], e) : 0.0;
+    double s = ldg<IO>(t.g.C, e);
+#pragma unroll
+    for (int k = 0; k < kMaxLevelSrc; ++k)
+      if (k < t.nsrc) s += v[k];
+    stg<IO>(t.g.C, e, s);
+  }
+}
+
+// P = 2^pshift threads share an element (splits p, p + P, ...), combined in p order
+template <typename IO>
+__device__ __forceinline__ void level_reduce(const LevelTask& t, int idx, double* red) {
+  const GemmArgs& g = t.g;
+  const int P = 1 << t.pshift, p = threadIdx.x & (P - 1);
+  const uint32_t total = (uint32_t)(g.M * g.N), N = (uint32_t)g.N;
+  const uint32_t e = (uint32_t)idx * (uint32_t)t.chunk + (threadIdx.x >> t.pshift);
+  double s = 0.0;
+  if (e < total) s = sum_strided(g.ws + (int64_t)p * total + e, (int64_t)P * total, (g.nsplit - p + P - 1) >> t.pshift);
+  if (P > 1) {
+    red[threadIdx.x] = s;
+    __syncthreads();
+    if (p == 0)
+      for (int x = 1; x < P; ++x) s += red[threadIdx.x + x];
+  }
+  if (e < total && p == 0) store_c<IO>(g, e / N, e % N, s);
+}
+
+template <typename T, typename IO>
+__global__ __launch_bounds__(256, kTileWaves<1>) void level_kernel(const LevelTask* __restrict__ tasks,
+                                                                   const LevelItem* __restrict__ items) {
+  constexpr int b1 = TabLds<T, 64, 64, tile_bk(64, 64), 1>::bytes, b2 = TabLds<double, 32, 32, tile_bk(32, 32), 1>::bytes;
+  __shared__ __align__(16) unsigned char smem[b1 > b2 ? b1 : b2];
+  typedef const __attribute__((address_space(4))) LevelTask* ConstTask;
+  typedef const __attribute__((address_space(4))) LevelItem* ConstItem;
+  const LevelItem& it = *(const LevelItem*)((ConstItem)items + blockIdx.x);
+  if (it.task < 0) return;
+  const LevelTask& t = *(const LevelTask*)((ConstTask)tasks + it.task);
+  const int idx = it.idx;
+  if (t.kind >= kLvPerm) {
+    switch (t.kind) {
+      case kLvPerm:
+      case kLvFlat: level_add<IO>(t, idx); break;
+      case kLvReduce: level_reduce<IO>(t, idx, reinterpret_cast<double*>(smem)); break;
+      case kLvSum: level_sum<IO>(t, idx); break;
+      default: {
+        const int64_t e0 = (int64_t)idx * t.chunk;
+        const int64_t e1 = e0 + t.chunk < t.g.M ? e0 + t.chunk : t.g.M;
+        for (int64_t e = e0 + threadIdx.x; e < e1; e += 256) stg<IO>(t.g.C, e, 0.0);
+      }
+    }
+    return;
+  }
+  const GemmArgs& g = t.g;
+  const int tm = (int)((g.M + g.bm - 1) / g.bm), tn = (int)((g.N + g.bn - 1) / g.bn);
+  const int per_z = tm * tn;
+  const int tz = idx / per_z;
+  int tx, ty;
+  tile_in_group(idx - tz * per_z, tm, tn, g.group, tx, ty);
+#define CCQ_LV(A, BM, BN) gemm_tab_tile<A, IO, BM, BN, tile_bk(BM, BN), 1>(g, tx, ty, tz, smem)
+  switch (t.kind) {
+    case kLvTile6464: CCQ_LV(T, 64, 64); break;
+    case kLvTile6432: CCQ_LV(T, 64, 32); break;
+    case kLvTile3264: CCQ_LV(T, 32, 64); break;
+    case kLvTileF64:
+      if constexpr (sizeof(T) == 4) {
+        CCQ_LV(double, 32, 32);
+        break;
+      }
+    default: CCQ_LV(T, 32, 32); break;
+  }
+#undef CCQ_LV
+}
+
 // Register-direct GEMM for skinny and dot-shaped products (an output extent
 // of at most a few MFMA tiles; HBM / latency bound).  No LDS staging: in a
 // 16-deep k step, lane l loads row l%16 of each 16-row block at
@@ -867,6 +984,9 @@ bool launch_chain_f32io(hipStream_t s, dim3 grid, const GemmChain& ch);
 bool launch_group_f64(hipStream_t s, dim3 grid, const GemmGroup& gg);
 bool launch_group_f32(hipStream_t s, dim3 grid, const GemmGroup& gg);
 bool launch_group_f32io(hipStream_t s, dim3 grid, const GemmGroup& gg);
+void launch_level_f64(hipStream_t s, const LevelTask* tasks, const LevelItem* items, int n);
+void launch_level_f32(hipStream_t s, const LevelTask* tasks, const LevelItem* items, int n);
+void launch_level_f32io(hipStream_t s, const LevelTask* tasks, const LevelItem* items, int n);
 bool launch_reg_f64(hipStream_t s, dim3 grid, const GemmArgs& g);
 bool launch_reg_f32io(hipStream_t s, dim3 grid, const GemmArgs& g);
 

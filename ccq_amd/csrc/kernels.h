@@ -182,6 +182,37 @@ struct GemmChain {
 };
 hipError_t launch_gemm_chain(hipStream_t s, const GemmArgs* es, int n);
 
+// One dependency level of a program in one launch: a task is an operation (or
+// a piece of the schedule), an item the part of it that one workgroup runs.
+enum LevelKind {
+  kLvTile6464 = 1,   // LDS-tiled GEMM, tile by kind (g after transposition)
+  kLvTile6432,
+  kLvTile3264,
+  kLvTile3232,
+  kLvTileF64,        // 32 x 32 in FP64 arithmetic whatever the precision mode
+  kLvPerm,           // C(perm) (+)= alpha A(perm): rowA / kA, rowC / colC
+  kLvFlat,           // C (+)= alpha A, identical layouts
+  kLvReduce,         // split-K completion of a GEMM of the previous level
+  kLvSum,            // C += sum of src
+  kLvZero            // C = 0
+};
+constexpr int kMaxLevelSrc = 8;
+struct LevelTask {
+  int kind;
+  int chunk;     // elements of an item (kLvPerm on: of the M x N elements)
+  int pshift;    // kLvReduce: 2^pshift threads share an element
+  int nsrc;
+  GemmArgs g;
+  const double* src[kMaxLevelSrc];
+};
+struct LevelItem {
+  int task, idx;   // task < 0: nothing
+};
+// prec as GemmArgs::prec (storage of the arrays and arithmetic of the tiles)
+hipError_t launch_level(hipStream_t s, int prec, const LevelTask* tasks, const LevelItem* items, int n);
+// the operand roles of a plan that runs transposed, swapped
+GemmArgs gemm_oriented(const GemmArgs& g);
+
 // Independent dense block copies / accumulations C_i (+)= alpha_i A_i over
 // identical layouts, in one launch (the small adds of one dependency level).
 constexpr int kMaxAddGroup = 16;

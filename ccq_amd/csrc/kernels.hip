@@ -936,6 +936,16 @@ hipError_t launch_gemm(hipStream_t s, const GemmArgs& g0) {
   return launch_reduce(s, g);
 }
 
+GemmArgs gemm_oriented(const GemmArgs& g) { return g.trans ? transposed(g) : g; }
+
+hipError_t launch_level(hipStream_t s, int prec, const LevelTask* tasks, const LevelItem* items, int n) {
+  if (n <= 0) return hipSuccess;
+  if (prec == 2) launch_level_f32io(s, tasks, items, n);
+  else if (prec == 1) launch_level_f32(s, tasks, items, n);
+  else launch_level_f64(s, tasks, items, n);
+  return hipGetLastError();
+}
+
 hipError_t launch_gemm_chain(hipStream_t s, const GemmArgs* es, int n) {
   if (n < 1 || n > kMaxChain) return hipErrorInvalidValue;
   GemmChain ch{};
