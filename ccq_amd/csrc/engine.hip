@@ -105,6 +105,10 @@ struct Tensor {
   float* p32 = nullptr;      // float shadow of the FP32-storage sweeps
   std::string base;          // View: base array; Amp/Resid: block name
   std::string spec[8];       // View: per-index "oa", "vb", ...
+  // storage order (choose_orders): index i is the declared index perm[i]
+  // (dims, spec and the operations' labels are permuted with it)
+  int perm[8] = {0, 1, 2, 3, 4, 5, 6, 7};
+  std::string spec0[8];      // spec in declared order
   // View: where the block lives inside the full-range base array; the view is
   // gathered into a dense C-order copy (ptr/strides) after every upload
   double* src = nullptr;
@@ -671,6 +675,203 @@ struct ccq_hip_ctx {
   // -------------------------------------------------------------------------
   // planning
 
+  // ---- storage orders ----------------------------------------------------
+  // The index order of an intermediate's or a view's storage is free: every
+  // access goes through offset tables.  A product reads an operand well when its
+  // fastest index is summed and last among the summed indices (k-contiguous
+  // loads), or an output index and last among the rows; otherwise every 8-byte
+  // load touches a cache line of its own (Wr[m,b,e,j] summed over (m,e): a ring
+  // product of the 100-orbital CCSD took 53 us instead of 34).  choose_orders
+  // permutes the indices of each free tensor, with the labels of every operation
+  // on it, so that the modelled cost of its operations is least.
+  struct OrderedOp {
+    int sec, op;
+    double time = 0;              // when its accesses are contiguous (s)
+    double nA = 0, nB = 0, nC = 0;
+    int64_t ext[128] = {};        // extent of each label
+  };
+  OrderedOp ordered_op(int si, int i) const {
+    const Op& op = sections[si].ops[i];
+    OrderedOp o;
+    o.sec = si;
+    o.op = i;
+    auto elems = [&](int t, const std::string& l) {
+      double n = 1;
+      for (int d = 0; d < tensors[t].rank; ++d) {
+        n *= (double)tensors[t].dims[d];
+        o.ext[l[d] & 127] = tensors[t].dims[d];
+      }
+      return n;
+    };
+    o.nA = elems(op.a, op.la);
+    o.nC = elems(op.out, op.lc);
+    if (!op.gemm) {
+      o.time = 8.0 * (o.nA + 2 * o.nC) / 3e12;
+      return o;
+    }
+    o.nB = elems(op.b, op.lb);
+    double k = 1;
+    for (char c : summed(op.la, op.lb, op.lc)) k *= (double)o.ext[c & 127];
+    o.time = std::max(2.0 * o.nC * k / 50e12, 8.0 * (o.nA + o.nB + 2 * o.nC) / 3e12);
+    return o;
+  }
+  // the summed labels in the order the product enumerates them: the order of
+  // the operand that is contiguous in one of them (A first)
+  static std::string summed(const std::string& la, const std::string& lb, const std::string& lc) {
+    const bool in_a = !la.empty() && lc.find(la.back()) == std::string::npos;
+    const bool in_b = !lb.empty() && lc.find(lb.back()) == std::string::npos;
+    std::string s;
+    for (char c : !in_a && in_b ? lb : la)
+      if (lc.find(c) == std::string::npos) s += c;
+    return s;
+  }
+  // cost factor of reading an operand with labels l in a product (1: contiguous)
+  static double operand_factor(const OrderedOp& o, const std::string& l, const std::string& lc, const std::string& ks) {
+    if (l.empty()) return 1.0;
+    std::string rows;   // the operand's output labels in C's order
+    for (char c : lc)
+      if (l.find(c) != std::string::npos) rows += c;
+    const bool k = lc.find(l.back()) == std::string::npos;
+    const std::string& g = k ? ks : rows;
+    int64_t run = 1;
+    size_t n = 0;
+    while (n < l.size() && n < g.size() && l[l.size() - 1 - n] == g[g.size() - 1 - n]) {
+      run *= o.ext[l[l.size() - 1 - n] & 127];
+      ++n;
+    }
+    if (n == 0) return 8.0;
+    // two k per load where pairs never straddle a run, a table where they do
+    const double form = !k ? 1.15 : n == g.size() ? 1.0 : run % 2 == 0 ? 1.05 : 1.2;
+    return form + 6.0 / (double)run;
+  }
+  static double op_cost(const OrderedOp& o, bool gemm, const std::string& la, const std::string& lb, const std::string& lc) {
+    // C(perm) += A: flat, or the same fastest index, or one side uncoalesced
+    if (!gemm) return o.time * (la == lc ? 1.0 : la.empty() || la.back() == lc.back() ? 1.3 : 4.0);
+    const std::string ks = summed(la, lb, lc);
+    const double fA = operand_factor(o, la, lc, ks), fB = operand_factor(o, lb, lc, ks);
+    // the output's fastest run: its trailing labels that belong to one operand
+    int64_t run = 1;
+    if (!lc.empty()) {
+      const bool from_a = la.find(lc.back()) != std::string::npos;
+      for (size_t i = lc.size(); i-- > 0;) {
+        if ((la.find(lc[i]) != std::string::npos) != from_a) break;
+        run *= o.ext[lc[i] & 127];
+      }
+    }
+    const double fC = 1.0 + 6.0 / (double)run;
+    return o.time * (fA * o.nA + fB * o.nB + fC * 2 * o.nC) / (o.nA + o.nB + 2 * o.nC);
+  }
+  static std::string permuted(const std::string& l, const std::vector<int>& p) {
+    std::string out;
+    for (int i : p) out += l[i];
+    return out;
+  }
+  // one tensor, or views of one block of one array
+  bool same_storage(int x, int t) const {
+    if (x == t) return true;
+    const Tensor &a = tensors[x], &b = tensors[t];
+    if (a.kind != TKind::View || b.kind != TKind::View || a.base != b.base || a.rank != b.rank) return false;
+    for (int i = 0; i < a.rank; ++i)
+      if (a.spec0[i] != b.spec0[i]) return false;
+    return true;
+  }
+
+  // CCQ_HIP_VIEWPERM=0 keeps every tensor in its declared index order
+  void choose_orders() {
+    for (auto& t : tensors) {
+      for (int i = 0; i < t.rank; ++i) {
+        t.perm[i] = i;
+        t.spec0[i] = t.spec[i];
+        if (t.kind == TKind::View) t.dims[i] = view_extent(t.spec[i]);
+      }
+    }
+    if (!view_perm) return;
+    std::vector<std::vector<OrderedOp>> uses(tensors.size());
+    std::vector<std::vector<int>> shared(tensors.size());
+    std::vector<int> lead(tensors.size());
+    for (int t = 0; t < (int)tensors.size(); ++t) {
+      lead[t] = t;
+      if (tensors[t].kind == TKind::View)
+        for (int u = 0; u < t && lead[t] == t; ++u)
+          if (same_storage(u, t)) lead[t] = u;
+      shared[lead[t]].push_back(t);
+    }
+    for (int si = 0; si < (int)sections.size(); ++si)
+      for (int i = 0; i < (int)sections[si].ops.size(); ++i) {
+        const Op& op = sections[si].ops[i];
+        const OrderedOp o = ordered_op(si, i);
+        int ts[3] = {lead[op.a], lead[op.out], op.gemm ? lead[op.b] : -1};
+        for (int k = 0; k < 3; ++k)
+          if (ts[k] >= 0 && (k < 1 || ts[k] != ts[0]) && (k < 2 || ts[k] != ts[1])) uses[ts[k]].push_back(o);
+      }
+    for (int round = 0; round < 3; ++round) {
+      bool changed = false;
+      for (int t = 0; t < (int)tensors.size(); ++t) {
+        const Tensor& T = tensors[t];
+        double time = 0;
+        for (const OrderedOp& o : uses[t]) time += o.time;
+        // the CC(t;3) kernels index the tail's tensors by their declared order
+        if (lead[t] != t || time < kOrderTime || T.rank < 2 || T.rank > 4 || T.id.rfind("cct3:", 0) == 0 ||
+            (T.kind != TKind::Inter && T.kind != TKind::View))
+          continue;
+        std::vector<int> p(T.rank), best;
+        for (int i = 0; i < T.rank; ++i) p[i] = i;
+        double least = -1.0, keep = 0.0;
+        do {
+          double c = 0;
+          for (const OrderedOp& o : uses[t]) {
+            const Op& op = sections[o.sec].ops[o.op];
+            c += op_cost(o, op.gemm, lead[op.a] == t ? permuted(op.la, p) : op.la,
+                         op.gemm && lead[op.b] == t ? permuted(op.lb, p) : op.lb,
+                         lead[op.out] == t ? permuted(op.lc, p) : op.lc);
+          }
+          if (least < 0) keep = least = c;   // the identity comes first
+          else if (c < least) {
+            least = c;
+            best = p;
+          }
+        } while (std::next_permutation(p.begin(), p.end()));
+        if (least < 0.999 * keep) {
+          set_order(t, lead, shared[t], uses[t], best);
+          changed = true;
+        }
+      }
+      if (!changed) break;
+    }
+  }
+  // tensors whose products take less chip time than this (s) keep their order:
+  // their levels last as long as their latencies do
+  static constexpr double kOrderTime = 0.5e-6;
+  int64_t view_extent(const std::string& spec) const {
+    const int64_t occ = spec[1] == 'b' ? ob : oa;
+    return spec[0] == 'o' ? occ : nc - occ;
+  }
+  // new index i of tensor t (and of the views sharing its storage) is old index p[i]
+  void set_order(int t, const std::vector<int>& lead, const std::vector<int>& shared, const std::vector<OrderedOp>& uses,
+                 const std::vector<int>& p) {
+    for (const OrderedOp& o : uses) {
+      Op& op = sections[o.sec].ops[o.op];
+      if (lead[op.a] == t) op.la = permuted(op.la, p);
+      if (op.gemm && lead[op.b] == t) op.lb = permuted(op.lb, p);
+      if (lead[op.out] == t) op.lc = permuted(op.lc, p);
+    }
+    for (int x : shared) {
+      Tensor& T = tensors[x];
+      const Tensor o = T;
+      std::vector<int> inv(T.rank);
+      for (int i = 0; i < T.rank; ++i) {
+        T.dims[i] = o.dims[p[i]];
+        T.spec[i] = o.spec[p[i]];
+        T.perm[i] = o.perm[p[i]];
+        inv[p[i]] = i;
+      }
+      for (auto& pq : T.anti) {
+        const int a = inv[pq.first], b = inv[pq.second];
+        pq = {std::min(a, b), std::max(a, b)};
+      }
+    }
+  }
+
   void resolve_tensors() {
     for (auto& t : tensors) {
       if (t.kind == TKind::Inter) {
@@ -717,27 +918,23 @@ struct ccq_hip_ctx {
         else if (t.base == "Fb") basep = Fb.p, nb = 2;
         else throw Fail("unknown base " + t.base);
         if (nb != t.rank) throw Fail("view rank mismatch for " + t.id);
-        int64_t s = 1;
+        int64_t bs[8];   // strides of the base array
+        for (int64_t i = t.rank - 1, s = 1; i >= 0; --i, s *= nc) bs[i] = s;
         int64_t off = 0;
-        for (int i = t.rank - 1; i >= 0; --i) {
-          t.src_strides[i] = s;
-          const char sp = t.spec[i][0];
-          const bool beta = t.spec[i][1] == 'b';
-          const int64_t occ = beta ? ob : oa;
-          t.dims[i] = sp == 'o' ? occ : nc - occ;
-          if (sp == 'v') off += occ * s;
-          s *= nc;
+        for (int i = 0; i < t.rank; ++i) {
+          t.src_strides[i] = bs[t.perm[i]];
+          t.dims[i] = view_extent(t.spec[i]);
+          if (t.spec[i][0] == 'v') off += (t.spec[i][1] == 'b' ? ob : oa) * t.src_strides[i];
         }
         t.src = basep + off;
         // dense copy shared by identical views
         std::string key = std::to_string((uintptr_t)basep);
-        for (int i = 0; i < t.rank; ++i) key += t.spec[i];
+        for (int i = 0; i < t.rank; ++i) key += t.spec0[i];
         auto hit = view_key.find(key);
-        const std::vector<int> order = view_order(t);
         int64_t d = 1;
         for (int i = t.rank - 1; i >= 0; --i) {
-          t.strides[order[i]] = d;
-          d *= t.dims[order[i]];
+          t.strides[i] = d;
+          d *= t.dims[i];
         }
         if (hit != view_key.end()) {
           t.ptr = hit->second;
@@ -756,53 +953,7 @@ struct ccq_hip_ctx {
   std::map<std::string, double*> view_key;
   std::vector<int> view_owner;
 
-  // Storage order of a view's dense copy (outermost index first).  A view
-  // whose every GEMM consumer contracts it with a small operand (at most
-  // 1024 elements: the T1-dressing products) keeps the indices summed by its
-  // first such consumer outermost, so that the rows those products read are
-  // contiguous; any other view keeps its index order.  A function of the
-  // view's base and spec, so identical views sharing a copy agree.
-  // CCQ_HIP_VIEWPERM=0 keeps every view in index order.
   bool view_perm = true;
-
-  std::vector<int> view_order(const Tensor& t) const {
-    std::vector<int> ident(t.rank);
-    for (int i = 0; i < t.rank; ++i) ident[i] = i;
-    if (!view_perm) return ident;
-    auto same_view = [&](int x) {
-      const Tensor& u = tensors[x];
-      if (u.kind != TKind::View || u.base != t.base || u.rank != t.rank) return false;
-      for (int i = 0; i < t.rank; ++i)
-        if (u.spec[i] != t.spec[i]) return false;
-      return true;
-    };
-    std::string labels, lc;
-    bool any = false;
-    for (const auto& sec : sections)
-      for (const auto& op : sec.ops) {
-        if (!op.gemm) continue;
-        const bool va = same_view(op.a), vb = same_view(op.b);
-        if (!va && !vb) continue;
-        if (va && vb) return ident;
-        const Tensor& other = tensors[va ? op.b : op.a];
-        if (other.kind == TKind::View) return ident;
-        int64_t n = 1;
-        for (int i = 0; i < other.rank; ++i) n *= other.dims[i];
-        if (n > 1024) return ident;
-        if (!any) {
-          labels = va ? op.la : op.lb;
-          lc = op.lc;
-          any = true;
-        }
-      }
-    if (!any) return ident;
-    std::vector<int> order;
-    for (int i = 0; i < t.rank; ++i)
-      if (lc.find(labels[i]) == std::string::npos) order.push_back(i);
-    for (int i = 0; i < t.rank; ++i)
-      if (lc.find(labels[i]) != std::string::npos) order.push_back(i);
-    return order;
-  }
 
   // tables that copy each distinct view out of its base array
   void plan_gathers() {
@@ -1167,6 +1318,12 @@ struct ccq_hip_ctx {
     auto top = [](const std::vector<int64_t>& t) { return t.empty() ? 0 : *std::max_element(t.begin(), t.end()); };
     return top(rows) + top(ks) + 32 * std::max<int64_t>(aff, 1);
   }
+  // k and k + 1 are neighbours for every even k
+  static bool paired(const std::vector<int64_t>& k) {
+    for (size_t i = 0; i + 1 < k.size(); i += 2)
+      if (k[i + 1] != k[i] + 1) return false;
+    return !k.empty();
+  }
   // operands whose last element lies at 4 GiB or beyond need 64-bit addresses
   // in the tile kernel (CCQ_HIP_WIDE=1: all of them do)
   static constexpr int64_t kWideElems = ((int64_t)1 << 32) / (int64_t)sizeof(double);
@@ -1451,8 +1608,8 @@ struct ccq_hip_ctx {
             bool inB = op.lb.find(c) != std::string::npos;
             if (inC && inB) throw Fail("batch label unsupported in " + sec.name);
             if (!inC && !inB) throw Fail("partial trace unsupported in " + sec.name);
-            if (!inC) ks += c;
           }
+          ks = summed(op.la, op.lb, op.lc);
           for (char c : op.lb) {
             bool inC = op.lc.find(c) != std::string::npos;
             bool inA = op.la.find(c) != std::string::npos;
@@ -1546,6 +1703,8 @@ struct ccq_hip_ctx {
                       : (!ns.empty() && stride_of(B, op.lb, ns.back()) == 1 ? 0 : 1));
           g.kA_aff = affine_stride(kAp);
           g.kB_aff = affine_stride(kBp);
+          g.a_pair = g.a_kfast && paired(kAp);
+          g.b_pair = g.b_kfast && paired(kBp);
           g.wide = wide_all || reach(rA, kAp, g.kA_aff) >= kWideElems || reach(cB, kBp, g.kB_aff) >= kWideElems;
           // C contiguous along m (n): its fastest m (n) label has stride 1,
           // so consecutive rows (columns) are adjacent in runs of that extent
@@ -1680,6 +1839,7 @@ struct ccq_hip_ctx {
       for (const auto& sec : sections) progs.insert(sec.prog);
       for (const auto& prog : progs) build_levels(prog);
       lv_ws.alloc(std::max<int64_t>(lv_ws_need, 1));
+      slots.alloc(slot_need);
     }
   }
 
@@ -2460,11 +2620,6 @@ struct ccq_hip_ctx {
     int64_t item0 = 0;
     int nitems = 0;
   };
-  struct SlotBuf {
-    int tensor = -1, slot = 0;
-    DevBuf buf;
-    float* p32 = nullptr;
-  };
   // what a task is built from, for either storage
   struct TaskSrc {
     int kind = 0;
@@ -2484,7 +2639,12 @@ struct ccq_hip_ctx {
     std::vector<ccqk::LevelTask> host[2];             // the same, for the operations with a launch of their own
   };
   std::map<std::string, LevelProg> level_progs;
-  std::map<std::pair<int, int>, std::unique_ptr<SlotBuf>> slot_bufs;   // (canonical tensor, slot)
+  // place of each partial accumulator (canonical tensor, slot) in one buffer
+  // (an allocation of its own for each took 25 ms of a small system's set-up)
+  std::map<std::pair<int, int>, int64_t> slot_off;
+  int64_t slot_need = 0;
+  DevBuf slots;
+  float* slots32 = nullptr;
   DevBuf lv_ws;
   int64_t lv_ws_need = 0;
   bool use_levels() const { return group; }
@@ -2496,53 +2656,56 @@ struct ccq_hip_ctx {
   }
   ccqlv::Key key_of(int t) const { return reinterpret_cast<ccqlv::Key>(tensors[t].ptr); }
 
-  // cycles of one workgroup on a tile of the product, its MFMAs alone, and
-  // the tiles: a slab costs about 150 cycles beside its MFMAs, the first
-  // operands and the epilogue about 4000
+  // Cycles of one workgroup on a tile of the product and its share of the
+  // chip's time.  A slab of a full chip costs its MFMAs over the tile's measured
+  // efficiency (4096 x 4096 x 2048: 65 TF/s in 64x64, about 59 in 64x32, 52 in
+  // 32x32 tiles), alone on its CU at least about 1200 cycles (gemm_plan_ranked);
+  // the first operands and the epilogue take about 4000 more.
   struct TileCost {
-    double item, mfma;
+    double item, share;
     int64_t tiles;
   };
   static TileCost tile_cost(int64_t M, int64_t N, int64_t K, int bm, int bn) {
     const int bk = ccqk::tile_bk(bm, bn);
     const double slabs = (double)((K + bk - 1) / bk);
-    const double slab = (bm / 32.0) * (bn / 32.0) * (bk / 4.0) * 64.0;
-    // a workgroup alone on its CU waits about 700 cycles a slab (gemm_plan_ranked)
-    return {slabs * std::max(slab + 150.0, 1200.0) + 4000.0 + bm * bn / 2.0, slabs * slab,
-            ((M + bm - 1) / bm) * ((N + bn - 1) / bn)};
+    const double eff = bm * bn == 64 * 64 ? 0.85 : bm * bn == 32 * 32 ? 0.68 : 0.77;
+    const double slab = (bm / 32.0) * (bn / 32.0) * (bk / 4.0) * 64.0 / eff;
+    const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    const double ends = 4000.0 + bm * bn / 2.0;
+    return {slabs * std::max(slab, 1200.0) + ends, tiles * (slabs * slab + ends / 3.0) / 256.0, tiles};
+  }
+  static TileCost tile_cost(const Op& op, const ccqk::GemmArgs& g) {
+    return tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, g.bm, g.bn);
   }
 
-  // tile of a product in a level launch: the shape with the least time if it
-  // had the chip to itself plus its share of the chip's time
-  ccqk::GemmArgs level_plan(const Op& op) const {
+  // Tile of a product in a level launch: the shape with the least share of the
+  // chip, counting a single workgroup's time beyond that of the rest of the
+  // level (load).
+  ccqk::GemmArgs level_plan(const Op& op, double load) const {
     ccqk::GemmArgs g = op.plan;
     g.kind = 0;
     g.ksplit = 1;
     g.nsplit = 1;
     g.trans = (g.c_mfast && !g.c_nfast) ? 1 : 0;
-    const int64_t M = g.trans ? op.N : op.M, N = g.trans ? op.M : op.N;
     double best = 1e300;
+    int bm = 32, bn = 32;
     const bool f64 = op.plan.kind == 1;   // register-direct products are FP64 in every precision mode
-    for (int bm : {64, 32})
-      for (int bn : {64, 32}) {
-        if (f64 && (bm != 32 || bn != 32)) continue;
-        const TileCost c = tile_cost(M, N, op.K, bm, bn);
-        const double share = c.tiles * std::max(c.mfma, c.item / 3.0) / 256.0;
-        const double t = std::max(share, c.item) + share;
+    for (int tm : {64, 32})
+      for (int tn : {64, 32}) {
+        if (f64 && (tm != 32 || tn != 32)) continue;
+        const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, tm, tn);
+        const double t = c.share + std::max(0.0, c.item - load);
         if (t < best) {
           best = t;
-          g.bm = bm;
-          g.bn = bn;
+          bm = tm;
+          bn = tn;
         }
       }
-    g.bk = ccqk::tile_bk(g.bm, g.bn);
+    g.bm = bm;
+    g.bn = bn;
+    g.bk = ccqk::tile_bk(bm, bn);
     g.kchunk = (op.K + g.bk - 1) / g.bk * g.bk;
     return g;
-  }
-  // the chip's time the product takes (cycles)
-  static double level_share(const Op& op, const ccqk::GemmArgs& g) {
-    const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, g.bm, g.bn);
-    return c.tiles * std::max(c.mfma, c.item / 3.0) / 256.0;
   }
 
   // operations that keep their own launch
@@ -2615,31 +2778,39 @@ struct ccq_hip_ctx {
       sch.run(v);
       return sch;
     };
-    // first pass: levels without K splits, and the chip time of each
-    std::vector<std::vector<ccqk::GemmArgs>> plans(units.size());
-    for (size_t u = 0; u < units.size(); ++u)
-      for (int i : us[u].ops) {
-        const Op& op = sections[us[u].sec].ops[i];
-        plans[u].push_back(op.gemm ? level_plan(op) : ccqk::GemmArgs{});
-      }
+    // first pass: levels without K splits and the chip time of each; then the
+    // tiles again, knowing the rest of the level
     std::vector<ccqlv::Unit> first = units;
     ccqlv::Scheduler s1 = schedule(first);
     std::vector<double> load(s1.levels + 1, 0.0);
-    for (size_t u = 0; u < units.size(); ++u)
-      for (size_t k = 0; k < us[u].ops.size(); ++k) {
-        const Op& op = sections[us[u].sec].ops[us[u].ops[k]];
-        if (op.gemm && !own_launch(op)) load[first[u].level] += level_share(op, plans[u][k]);
+    std::vector<std::vector<ccqk::GemmArgs>> plans(units.size());
+    for (int pass = 0; pass < 2; ++pass) {
+      std::vector<double> sum(s1.levels + 1, 0.0);
+      for (size_t u = 0; u < units.size(); ++u) {
+        plans[u].clear();
+        for (int i : us[u].ops) {
+          const Op& op = sections[us[u].sec].ops[i];
+          const int l = first[u].level;
+          plans[u].push_back(op.gemm ? level_plan(op, pass ? load[l] : 0.0) : ccqk::GemmArgs{});
+          if (op.gemm && !own_launch(op)) sum[l] += tile_cost(op, plans[u].back()).share;
+        }
       }
-    // a product whose single workgroups would outlast their level by more than
-    // the extra level of a split is split along K
+      load = sum;
+    }
+    // A product whose single workgroups outlast the rest of their level by more
+    // than the extra level of a split is split along K; one with tiles for half
+    // the chip (its partials then cost more than idle CUs) only beyond a third
+    // of a long level.
     std::vector<int64_t> partials(s1.levels + 1, 0);
     for (size_t u = 0; u < units.size(); ++u)
       for (size_t k = 0; k < us[u].ops.size(); ++k) {
         const Op& op = sections[us[u].sec].ops[us[u].ops[k]];
         if (!op.gemm || own_launch(op) || op.K == 0) continue;
         ccqk::GemmArgs& g = plans[u][k];
-        const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, g.bm, g.bn);
-        const double span = std::max(load[first[u].level], kSplitSpan);
+        const TileCost c = tile_cost(op, g);
+        const double span = op.M * op.N <= kSplitDot ? kSplitSpan
+                            : c.tiles < 128          ? std::max(load[first[u].level] / 4.0, kSplitSpan)
+                                                     : std::max(load[first[u].level] / 3.0, kSplitWide);
         if (c.item < span + kSplitGain) continue;
         const int64_t slabs = (op.K + g.bk - 1) / g.bk;
         int64_t split = (int64_t)std::ceil((c.item - 4000.0) / std::max(span - 4000.0, 4000.0));
@@ -2671,12 +2842,7 @@ struct ccq_hip_ctx {
     auto tensor_of = [&](ccqlv::Key k) { return canon.at(k); };
     auto slot_of_tensor = [&](int t, int s) {
       if (!s) return;
-      auto& b = slot_bufs[{t, s}];
-      if (b) return;
-      b.reset(new SlotBuf);
-      b->tensor = t;
-      b->slot = s;
-      b->buf.alloc(tensor_size(t));
+      if (slot_off.emplace(std::make_pair(t, s), slot_need).second) slot_need += (tensor_size(t) + 31) / 32 * 32;
     };
     auto items_of = [&](int64_t total, int chunk) { return (total + chunk - 1) / chunk; };
     for (size_t u = 0; u < units.size(); ++u) {
@@ -2715,7 +2881,7 @@ struct ccq_hip_ctx {
             continue;
           }
           const ccqk::GemmArgs& g = ts.plan;
-          const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, g.bm, g.bn);
+          const TileCost c = tile_cost(op, g);
           ts.kind = op.plan.kind == 1 ? ccqk::kLvTileF64
                                       : g.bm == 64 ? (g.bn == 64 ? ccqk::kLvTile6464 : ccqk::kLvTile6432)
                                                    : (g.bn == 64 ? ccqk::kLvTile3264 : ccqk::kLvTile3232);
@@ -2808,13 +2974,26 @@ struct ccq_hip_ctx {
       HIPCHK(hipMemcpy(lp.items, items.data(), sizeof(ccqk::LevelItem) * items.size(), hipMemcpyHostToDevice));
     if (dump_schedule)
       for (size_t l = 0; l < at.size(); ++l) {
-        std::fprintf(stderr, "[levels] %s level %zu: %d items, %zu own launches\n", prog.c_str(), l, lp.steps[l].nitems,
-                     lp.steps[l].own.size());
+        double fl = 0, by = 0;
         for (const Pending& p : at[l]) {
           const TaskSrc& ts = lp.src[p.task];
-          std::fprintf(stderr, "[levels]   kind %d %s -> %s slot %d items %lld cost %.0f split %d\n", ts.kind,
-                       ts.op >= 0 ? sections[ts.sec].ops[ts.op].cls.c_str() : "", tensors[ts.tensor].id.c_str(), ts.slot,
-                       (long long)p.n, p.cost, ts.plan.nsplit);
+          if (ts.op < 0 || ts.kind == ccqk::kLvReduce) continue;
+          fl += sections[ts.sec].ops[ts.op].flops;
+          by += sections[ts.sec].ops[ts.op].bytes;
+        }
+        std::fprintf(stderr, "[levels] %s level %zu: %d items, %zu own launches, %.2f GF, %.1f MB\n", prog.c_str(), l,
+                     lp.steps[l].nitems, lp.steps[l].own.size(), fl * 1e-9, by * 1e-6);
+        for (const Pending& p : at[l]) {
+          const TaskSrc& ts = lp.src[p.task];
+          std::string form;   // how the operands' summed indices lie: v contiguous, a strided, p pairs, t table
+          if (ts.op >= 0 && sections[ts.sec].ops[ts.op].gemm) {
+            const ccqk::GemmArgs& g = ts.plan;
+            form = std::string(" ") + (g.kA_aff < 0 ? (g.a_pair ? 'p' : 't') : g.a_kfast && g.kA_aff == 1 ? 'v' : 'a') + (g.a_kfast ? "k" : "m") +
+                   (g.kB_aff < 0 ? (g.b_pair ? 'p' : 't') : g.b_kfast && g.kB_aff == 1 ? 'v' : 'a') + (g.b_kfast ? "k" : "n");
+          }
+          std::fprintf(stderr, "[levels]   kind %d %s%s -> %s slot %d items %lld cost %.0f split %d\n", ts.kind,
+                       ts.op >= 0 ? sections[ts.sec].ops[ts.op].cls.c_str() : "", form.c_str(), tensors[ts.tensor].id.c_str(),
+                       ts.slot, (long long)p.n, p.cost, ts.plan.nsplit);
         }
         for (auto& o : lp.steps[l].own)
           std::fprintf(stderr, "[levels]   own %s %s\n", sections[o.first].name.c_str(),
@@ -2827,8 +3006,8 @@ struct ccq_hip_ctx {
     if (lp.tasks[st]) return;
     auto dst = [&](int t, int s) -> double* {
       if (!s) return sp(t);
-      SlotBuf& b = *slot_bufs.at({t, s});
-      return st ? reinterpret_cast<double*>(b.p32) : b.buf.p;
+      const int64_t o = slot_off.at({t, s});
+      return st ? reinterpret_cast<double*>(slots32 + o) : slots.p + o;
     };
     std::vector<ccqk::LevelTask>& v = lp.host[st];
     v.assign(lp.src.size(), ccqk::LevelTask{});
@@ -2884,13 +3063,10 @@ struct ccq_hip_ctx {
     if (!level_progs.count(prog)) throw Fail("no level schedule of program " + prog);
     LevelProg& lp = level_progs.at(prog);
     if (lp.tasks[st]) return;
-    if (st)
-      for (auto& kv : slot_bufs) {
-        SlotBuf& b = *kv.second;
-        if (b.p32) continue;
-        HIPCHK(hipMalloc(&b.p32, sizeof(float) * tensor_size(b.tensor)));
-        f32_bufs.push_back(b.p32);
-      }
+    if (st && !slots32 && slot_need) {
+      HIPCHK(hipMalloc(&slots32, sizeof(float) * slot_need));
+      f32_bufs.push_back(slots32);
+    }
     const int keep = run_prec;
     run_prec = st ? 2 : 0;
     try {
@@ -2935,7 +3111,8 @@ struct ccq_hip_ctx {
   }
   // a single workgroup's cycles below which splitting never pays, and what the
   // extra level costs
-  static constexpr double kSplitSpan = 12000.0, kSplitGain = 10000.0;
+  static constexpr int64_t kSplitDot = 1 << 14;   // outputs whose partials cost nothing
+  static constexpr double kSplitSpan = 12000.0, kSplitWide = 80000.0, kSplitGain = 10000.0;
   // partials of one product and of one level (doubles)
   static constexpr int64_t kSplitMax = 4 << 20, kLevelPartials = 32 << 20;
 
@@ -3644,6 +3821,7 @@ int ccq_hip_set_ints(ccq_hip_ctx* ctx, const double* f_a, const double* f_b, con
     HIPCHK(hipMemcpy(ctx->fdiag_a.p, da.data(), sizeof(double) * nc, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(ctx->fdiag_b.p, db.data(), sizeof(double) * nc, hipMemcpyHostToDevice));
     if (!ctx->ints_ready) {
+      ctx->choose_orders();
       ctx->resolve_tensors();
       ctx->plan();
     }
@@ -4012,7 +4190,29 @@ int ccq_hip_debug_read(ccq_hip_ctx* ctx, const char* tensor_id, double* out, int
     for (int d = 0; d < t.rank; ++d) total *= t.dims[d];
     if (n != total) throw Fail("debug_read size mismatch");
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(out, t.ptr, sizeof(double) * total, hipMemcpyDeviceToHost));
+    bool moved = false;
+    for (int d = 0; d < t.rank; ++d) moved = moved || t.perm[d] != d;
+    if (!moved) {
+      HIPCHK(hipMemcpy(out, t.ptr, sizeof(double) * total, hipMemcpyDeviceToHost));
+      return;
+    }
+    // storage order -> declared order
+    std::vector<double> buf((size_t)total);
+    HIPCHK(hipMemcpy(buf.data(), t.ptr, sizeof(double) * total, hipMemcpyDeviceToHost));
+    int64_t dec[8], str[8];   // declared extents; stride of each stored index in the output
+    for (int d = 0; d < t.rank; ++d) dec[t.perm[d]] = t.dims[d];
+    for (int d = 0; d < t.rank; ++d) {
+      str[d] = 1;
+      for (int e = t.perm[d] + 1; e < t.rank; ++e) str[d] *= dec[e];
+    }
+    for (int64_t e = 0; e < total; ++e) {
+      int64_t r = e, o = 0;
+      for (int d = t.rank - 1; d >= 0; --d) {
+        o += (r % t.dims[d]) * str[d];
+        r /= t.dims[d];
+      }
+      out[o] = buf[(size_t)e];
+    }
   }, true);
 }
 

@@ -32,6 +32,9 @@ struct GemmArgs {
   int c_mfast = 0, c_nfast = 0;
   // kA[k] == k * kA_aff for every k when kA_aff >= 0 (same for B)
   int64_t kA_aff = -1, kB_aff = -1;
+  // a k-contiguous operand's table: kA[k + 1] == kA[k] + 1 for every even k
+  // (same for B)
+  int a_pair = 0, b_pair = 0;
   // A or B reaches 4 GiB: the tile kernel addresses both with 64 bits
   int wide = 0;
   // launch plan (gemm_plan)

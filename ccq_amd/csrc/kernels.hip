@@ -893,6 +893,8 @@ static GemmArgs transposed(const GemmArgs& g) {
   t.colC2 = g.rowC2;
   t.a_kfast = g.b_kfast;
   t.b_kfast = g.a_kfast;
+  t.a_pair = g.b_pair;
+  t.b_pair = g.a_pair;
   t.trans = 0;
   return t;
 }

@@ -426,3 +426,25 @@ def test_wide_addresses_equal_narrow(method, n, o, ob, prec, monkeypatch):
         eng.close()
     assert out[0][0] == out[1][0]
     np.testing.assert_array_equal(out[1][1], out[0][1])
+
+
+@pytest.mark.parametrize("n,o,ob", [(64, 8, 8), (71, 9, 8)])
+def test_storage_orders_read_back_declared(n, o, ob, monkeypatch):
+    """Intermediates stored in an order chosen for their products read back in
+    their declared order: after two sweeps they and the amplitudes are within
+    1e-11 of those of the declared orders (CCQ_HIP_VIEWPERM=0)."""
+    _say(f"case storage orders n={n} o={o} ob={ob}")
+    c = Case(n, o, 2 * n, 43, occ_b=ob)
+    vec = _state(c, "CCSD", 19)
+    va, vb = n - o, n - ob
+    inters = {"Wr.ovvo.aaaa": (o, va, va, o), "Wr.ovvo.baba": (ob, va, vb, o), "Wr.ovvo.abba": (o, vb, vb, o)}
+    out = []
+    for perm in ("0", "1"):
+        eng = _engine_env(c, "CCSD", monkeypatch, {"CCQ_HIP_VIEWPERM": perm}, shift=0.02)
+        eng.set_t(vec)
+        for _ in range(2):
+            eng.update()
+        out.append([eng.debug_read(tid, shape) for tid, shape in inters.items()] + [eng.get_t()])
+        eng.close()
+    for x, y in zip(*out):
+        assert np.abs(y - x).max() <= 1e-11 * np.abs(x).max()
