@@ -61,9 +61,9 @@ constexpr int64_t kWsCap = 16 << 20;   // split-K workspace bound (doubles)
 // ---------------------------------------------------------------------------
 // device buffers
 
-// Pinned host array for the small device-to-host copies of the partial sums
-// (energy, residuum, DIIS Gram matrix): a copy into pageable memory goes
-// through a staging buffer and costs several times as long.
+// Pinned host array for partial sums (energy, residuum, DIIS Gram matrix), which
+// the kernels write there: a copy after them costs 5 - 10 us, into pageable memory
+// several times that.
 struct PinnedVec {
   double* p = nullptr;
   size_t cap = 0;
@@ -3294,11 +3294,11 @@ struct ccq_hip_ctx {
   // partial sums (rpart); a residuum of the same iteration that is the very
   // next call of the C ABI uses them (api_calls counts the calls)
   int64_t api_calls = 0, rec_call = -10, rec_iter = -1;
-  DevBuf rpart;
+  PinnedVec rpart;
 
-  double reduce_partials(int count, const double* src = nullptr) {
+  double reduce_partials(int count) {
     host_partial.resize(count);
-    HIPCHK(hipMemcpyAsync(host_partial.data(), src ? src : partial.p, sizeof(double) * count,
+    HIPCHK(hipMemcpyAsync(host_partial.data(), partial.p, sizeof(double) * count,
                           hipMemcpyDeviceToHost, stream));
     HIPCHK(hipStreamSynchronize(stream));
     double s = 0.0;
@@ -3306,59 +3306,33 @@ struct ccq_hip_ctx {
     return s;
   }
 
+  // partial sums that a kernel has written to pinned memory
+  double sum_partials(int count, PinnedVec& v) {
+    HIPCHK(hipStreamSynchronize(stream));
+    double s = 0.0;
+    for (int i = 0; i < count; ++i) s += v[i];
+    return s;
+  }
+
   double energy() {
     // src/energy.f90:138-270, same eight pieces
     double* t1a = tvec.p + blk_off["t1a"];
     double* t1b = tvec.p + blk_off["t1b"];
-    // each piece's block partials in its own slice, one copy to the host,
-    // then the pieces summed in order
-    HIPCHK(ccqk::launch_dot_strided(stream, oa, va, Fa.p + oa, nc, t1a, partial.p, kPartialBlocks));
-    HIPCHK(ccqk::launch_dot_strided(stream, ob, vb, Fb.p + ob, nc, t1b, partial.p + kPartialBlocks,
-                                    kPartialBlocks));
-    struct Case {
-      const double* V;
-      int64_t o1, o2;
-      const char* t2;
-      double* x;
-      double* y;
-      double w2, w11;
-    };
-    Case cases[3] = {{Vaa.p, oa, oa, "t2aa", t1a, t1a, 0.25, 0.5},
-                     {Vab.p, oa, ob, "t2ab", t1a, t1b, 1.0, 1.0},
-                     {vbb_ptr, ob, ob, "t2bb", t1b, t1b, 0.25, 0.5}};
-    int piece = 2;
-    for (auto& c : cases) {
-      ccqk::EnergyParams P{};
-      P.V = c.V;
-      P.vs0 = nc * nc * nc;
-      P.vs1 = nc * nc;
-      P.vs2 = nc;
-      P.vs3 = 1;
-      P.vo1 = c.o1;
-      P.vo2 = c.o2;
-      P.t2 = tvec.p + blk_off[c.t2];
-      P.t1x = c.x;
-      P.t1y = c.y;
-      P.o1 = c.o1;
-      P.o2 = c.o2;
-      P.v1 = nc - c.o1;
-      P.v2 = nc - c.o2;
-      P.w2 = c.w2;
-      P.w11 = c.w11;
-      HIPCHK(ccqk::launch_energy_pairs(stream, P, partial.p + (int64_t)piece++ * kPartialBlocks,
-                                       kPartialBlocks));
-    }
-    host_partial.resize((size_t)piece * kPartialBlocks);
-    HIPCHK(hipMemcpyAsync(host_partial.data(), partial.p, sizeof(double) * piece * kPartialBlocks,
-                          hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    double total = 0.0;
-    for (int q = 0; q < piece; ++q) {
-      double sp = 0.0;
-      for (int b = 0; b < kPartialBlocks; ++b) sp += host_partial[(size_t)q * kPartialBlocks + b];
-      total += sp;
-    }
-    return total;
+    ccqk::EnergyParams P{};
+    P.c[0] = {Vaa.p, tvec.p + blk_off["t2aa"], t1a, t1a, oa, oa, 0.25, 0.5};
+    P.c[1] = {Vab.p, tvec.p + blk_off["t2ab"], t1a, t1b, oa, ob, 1.0, 1.0};
+    P.c[2] = {vbb_ptr, tvec.p + blk_off["t2bb"], t1b, t1b, ob, ob, 0.25, 0.5};
+    P.f[0] = Fa.p;
+    P.f[1] = Fb.p;
+    P.t1[0] = t1a;
+    P.t1[1] = t1b;
+    P.occ[0] = oa;
+    P.occ[1] = ob;
+    P.nc = nc;
+    host_partial.resize(kPartialBlocks);
+    int used = 0;
+    HIPCHK(ccqk::launch_energy(stream, P, host_partial.data(), kPartialBlocks, &used));
+    return sum_partials(used, host_partial);
   }
 
   // -------------------------------------------------------------------------
@@ -3833,7 +3807,7 @@ int ccq_hip_create(const ccq_hip_dims* dims, const ccq_hip_opts* opts, ccq_hip_c
       ctx->cpart.alloc(4 * kPartialBlocks * 4);
       if (ctx->l_size > ctx->vec_size) throw Fail("DIIS ring too small for l_vec");
     }
-    ctx->partial.alloc(kPartialBlocks * 128);
+    ctx->partial.alloc(kPartialBlocks);
     if (ctx->level == 2) ctx->load_ir(ctx->rhf ? kIR_CCSD_RHF : kIR_CCSD_UHF);
     else if (ctx->active) {
       ctx->load_ir(kIR_CCSDT_ACT_UHF);
@@ -4076,9 +4050,9 @@ int ccq_hip_diis_record(ccq_hip_ctx* ctx, int64_t iter) {
       return;
     }
     const double* prev = iter == 1 ? nullptr : ctx->ring.p + ctx->slot_of(iter - 1) * ctx->vec_size;
-    if (!ctx->rpart.p) ctx->rpart.alloc(kPartialBlocks);
+    ctx->rpart.resize(kPartialBlocks);
     HIPCHK(ccqk::launch_copy_diff_sq(ctx->stream, ctx->ring.p + s * ctx->vec_size, ctx->tvec.p, prev,
-                                     ctx->vec_size, ctx->rpart.p, kPartialBlocks));
+                                     ctx->vec_size, ctx->rpart.data(), ccqk::sum_blocks(ctx->vec_size)));
     ctx->rec_call = ctx->api_calls;
     ctx->rec_iter = iter;
   }, true);
@@ -4087,14 +4061,16 @@ int ccq_hip_diis_record(ccq_hip_ctx* ctx, int64_t iter) {
 int ccq_hip_residuum(ccq_hip_ctx* ctx, int64_t iter, double* res) {
   return guarded(ctx, [&] {
     if (!ctx->left_mode && !ctx->active && ctx->rec_iter == iter && ctx->rec_call == ctx->api_calls - 1) {
-      *res = std::sqrt(std::sqrt(ctx->reduce_partials(kPartialBlocks, ctx->rpart.p)));
+      *res = std::sqrt(std::sqrt(ctx->sum_partials(ccqk::sum_blocks(ctx->vec_size), ctx->rpart)));
       return;
     }
     const int64_t len = ctx->diis_len();
     const double* cur = ctx->ring.p + ctx->slot_of(iter) * len;
     const double* prev = iter == 1 ? nullptr : ctx->ring.p + ctx->slot_of(iter - 1) * len;
-    HIPCHK(ccqk::launch_diff_sq(ctx->stream, prev, cur, len, ctx->partial.p, kPartialBlocks));
-    *res = std::sqrt(std::sqrt(ctx->reduce_partials(kPartialBlocks)));
+    const int nb = ccqk::sum_blocks(len);
+    ctx->host_partial.resize(nb);
+    HIPCHK(ccqk::launch_diff_sq(ctx->stream, prev, cur, len, ctx->host_partial.data(), nb));
+    *res = std::sqrt(std::sqrt(ctx->sum_partials(nb, ctx->host_partial)));
   }, true);
 }
 
@@ -4103,14 +4079,12 @@ int ccq_hip_diis_extrapolate(ccq_hip_ctx* ctx) {
     const int n = ctx->diis;
     const int np = n * (n + 1) / 2;
     const int64_t len = ctx->diis_len();
-    HIPCHK(ccqk::launch_diis_gram(ctx->stream, ctx->ring.p, len, n, ctx->partial.p,
-                                  kPartialBlocks));
-    ctx->host_partial.resize((size_t)kPartialBlocks * np);
-    HIPCHK(hipMemcpyAsync(ctx->host_partial.data(), ctx->partial.p,
-                          sizeof(double) * kPartialBlocks * np, hipMemcpyDeviceToHost, ctx->stream));
+    const int nb = ccqk::sum_blocks(len);
+    ctx->host_partial.resize((size_t)nb * np);
+    HIPCHK(ccqk::launch_diis_gram(ctx->stream, ctx->ring.p, len, n, ctx->host_partial.data(), nb));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     std::vector<double> g(np, 0.0);
-    for (int b = 0; b < kPartialBlocks; ++b)
+    for (int b = 0; b < nb; ++b)
       for (int q = 0; q < np; ++q) g[q] += ctx->host_partial[(size_t)b * np + q];
     const int m = n + 1;
     std::vector<double> B((size_t)m * m, 0.0), c(m, 0.0);

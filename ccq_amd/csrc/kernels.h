@@ -121,15 +121,20 @@ struct Cct3Params {
   const double* d3[8];
 };
 
-struct EnergyParams {
-  const double* V;       // full-range base array
-  int64_t vs0, vs1, vs2, vs3;   // strides of V
-  int64_t vo1, vo2;      // virtual offsets of the two virtual indices
-  const double* t2;      // [m][n][e][f]
-  const double* t1x;     // [m][e]
+struct EnergyCase {
+  const double* V;       // full-range base array, nc^4
+  const double* t2;      // [m][n][a][f]
+  const double* t1x;     // [m][a]
   const double* t1y;     // [n][f]
-  int64_t o1, o2, v1, v2;
+  int64_t o1, o2;
   double w2, w11;
+};
+struct EnergyParams {
+  EnergyCase c[3];
+  const double* f[2];    // Fock matrices, nc^2, and singles of the two spins
+  const double* t1[2];
+  int64_t occ[2], nc;
+  int tile0[3] = {}, tiles = 0;   // (launch_energy)
 };
 
 struct Coeffs {
@@ -308,9 +313,11 @@ hipError_t launch_guess_apply(hipStream_t s, const GuessBlock& B, const float* p
 // training data of the block at its current (converged) t: features X[n][5],
 // M = m / sm, Y = (t - m) / sm, for every tuple in C order
 hipError_t launch_guess_data(hipStream_t s, const GuessBlock& B, float* X, float* M, float* Y);
-hipError_t launch_energy_pairs(hipStream_t s, const EnergyParams& P, double* partial, int blocks);
-hipError_t launch_dot_strided(hipStream_t s, int64_t rows, int64_t cols, const double* a,
-                              int64_t lda, const double* b, double* partial, int blocks);
+// partial sums of the energy's pieces; used: how many (at most blocks)
+hipError_t launch_energy(hipStream_t s, EnergyParams P, double* partial, int blocks, int* used);
+// blocks of a sum over len elements (at most 1024): four elements a thread
+// before a block sums more than that
+int sum_blocks(int64_t len);
 hipError_t launch_diis_gram(hipStream_t s, const double* ring, int64_t len, int n, double* partial,
                             int blocks);
 // dst = src with diff_sq(prev, dst)'s partials in the same pass
