@@ -2928,6 +2928,9 @@ struct ccq_hip_ctx {
       if (!s) return;
       if (slot_off.emplace(std::make_pair(t, s), slot_need).second) slot_need += (tensor_size(t) + 31) / 32 * 32;
     };
+    // elements of an add's or sum's item: the latency of one load a thread while
+    // that leaves at most a workgroup a CU, else as many as an item can have in flight
+    auto add_chunk = [](int64_t total) { return total <= 512 * 256 ? 512 : total <= 1024 * 256 ? 1024 : 2048; };
     auto items_of = [&](int64_t total, int chunk) { return (total + chunk - 1) / chunk; };
     for (size_t u = 0; u < units.size(); ++u) {
       const ccqlv::Unit& un = units[u];
@@ -2976,8 +2979,9 @@ struct ccq_hip_ctx {
             ws_used[un.level] += g.nsplit * op.M * op.N;
             TaskSrc r = ts;
             r.kind = ccqk::kLvReduce;
-            while ((1 << r.pshift) < g.nsplit && r.pshift < 5 && op.M * op.N * (2 << r.pshift) <= 262144) ++r.pshift;
-            r.chunk = 256 >> r.pshift;
+            // a thread sums at least four partials; about 512 items
+            while ((4 << r.pshift) < g.nsplit && r.pshift < 5 && op.M * op.N * (2 << r.pshift) <= 262144) ++r.pshift;
+            r.chunk = (256 >> r.pshift) * (int)std::clamp<int64_t>((op.M * op.N << r.pshift) / (256 * 512), 1, 8);
             at[un.level + 1].push_back({(int)lp.src.size(), items_of(op.M * op.N, r.chunk), 3000.0});
             lp.src.push_back(r);
           }
@@ -2989,7 +2993,7 @@ struct ccq_hip_ctx {
             continue;
           }
           ts.kind = op.flat ? ccqk::kLvFlat : ccqk::kLvPerm;
-          ts.chunk = 1024;
+          ts.chunk = add_chunk(op.M * op.N);
           n = items_of(op.M * op.N, ts.chunk);
           cost = 3000.0;
         }
@@ -3002,7 +3006,7 @@ struct ccq_hip_ctx {
       ts.kind = ccqk::kLvSum;
       ts.tensor = tensor_of(sm.out);
       ts.nslots = sm.nslots;
-      ts.chunk = 1024;
+      ts.chunk = add_chunk(tensor_size(ts.tensor));
       at[sm.level].push_back({(int)lp.src.size(), items_of(tensor_size(ts.tensor), ts.chunk), 3000.0});
       lp.src.push_back(ts);
     }

@@ -8,9 +8,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
 #include "kernels.h"
 
 typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 namespace ccqk {
@@ -730,70 +732,136 @@ __global__ __launch_bounds__(256, kTileWaves<1>) void gemm_tab_group(GemmGroup g
 // sweep as 176 launches, 185 us in 27 levels.
 // The descriptors are read through the constant address space: nothing
 // writes them while the kernel runs, so they stay scalar loads.
+// Adds and sums move up to 2048 elements an item, all loads of a thread in
+// flight before its first store: an item lasts as long as its latencies do, and beside
+// large products it has one of a CU's three places (1024 elements an item, loads
+// of 8 bytes: CCSD, 100 orbitals, 1900 us a sweep, this 1867).
 template <typename IO>
-__device__ __forceinline__ void level_add(const LevelTask& t, int idx) {
+struct Pair2 {
+  typedef IO type __attribute__((ext_vector_type(2), aligned(sizeof(IO))));
+};
+template <typename IO>
+__device__ __forceinline__ d2 ldg2(const double* p, int64_t i) {
+  const auto v = *reinterpret_cast<const typename Pair2<IO>::type*>(reinterpret_cast<const IO*>(p) + i);
+  return d2{(double)v.x, (double)v.y};
+}
+template <typename IO>
+__device__ __forceinline__ void stg2(double* p, int64_t i, d2 v) {
+  typename Pair2<IO>::type w;
+  w.x = (IO)v.x;
+  w.y = (IO)v.y;
+  *reinterpret_cast<typename Pair2<IO>::type*>(reinterpret_cast<IO*>(p) + i) = w;
+}
+
+template <typename IO>
+__device__ __forceinline__ void level_perm(const LevelTask& t, int idx) {
   const GemmArgs& g = t.g;
   const uint32_t N = (uint32_t)g.N, total = (uint32_t)(g.M * g.N);
   const uint32_t e0 = (uint32_t)idx * (uint32_t)t.chunk;
   const uint32_t e1 = total - e0 < (uint32_t)t.chunk ? total : e0 + (uint32_t)t.chunk;
-  const bool flat = t.kind == kLvFlat;
-  for (uint32_t b = e0 + threadIdx.x; b < e1; b += 1024) {
-    int64_t ia[4], ic[4];
-    double v[4], c[4];
+  auto run = [&](uint32_t b, auto count) {   // count elements a thread, 256 apart
+    constexpr int J = decltype(count)::value;
+    int64_t ia[J], ic[J];
+    double v[J], c[J];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < J; ++j) {
       const uint32_t e = b + 256u * j < e1 ? b + 256u * j : b;
-      if (flat) {
-        ia[j] = ic[j] = e;
-      } else {
-        const uint32_t r = e / N, n = e - r * N;
-        ia[j] = (int64_t)g.rowA[r] + g.kA[n];
-        ic[j] = (int64_t)g.rowC[r] + g.colC[n];
-      }
+      const uint32_t r = e / N, n = e - r * N;
+      ia[j] = (int64_t)g.rowA[r] + g.kA[n];
+      ic[j] = (int64_t)g.rowC[r] + g.colC[n];
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < J; ++j) {
       v[j] = ldg<IO>(g.A, ia[j]);
       c[j] = g.accumulate ? ldg<IO>(g.C, ic[j]) : 0.0;
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < J; ++j)
       if (b + 256u * j < e1) stg<IO>(g.C, ic[j], g.accumulate ? c[j] + g.alpha * v[j] : g.alpha * v[j]);
-  }
+  };
+  uint32_t b = e0 + threadIdx.x;
+  if (t.chunk > 512)
+    for (; b < e1; b += 2048) run(b, std::integral_constant<int, 8>{});
+  else
+    for (; b < e1; b += 512) run(b, std::integral_constant<int, 2>{});
 }
 
+// C (+)= alpha A (n = 0), or C += the sum of n arrays; whole pairs, then the last one
 template <typename IO>
-__device__ __forceinline__ void level_sum(const LevelTask& t, int idx) {
-  const int64_t total = t.g.M, e0 = (int64_t)idx * t.chunk;
+__device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
+  const GemmArgs& g = t.g;
+  const int64_t total = t.kind == kLvSum ? g.M : g.M * g.N, e0 = (int64_t)idx * t.chunk;
   const int64_t e1 = e0 + t.chunk < total ? e0 + t.chunk : total;
-  for (int64_t e = e0 + threadIdx.x; e < e1; e += 256) {
-    double v[kMaxLevelSrc];
+  const bool add = t.kind != kLvSum;
+  auto one = [&](int64_t e) {
+    double s = add ? g.alpha * ldg<IO>(g.A, e) : 0.0;
+    if (!add) {
+      s = ldg<IO>(g.C, e);
+      for (int k = 0; k < t.nsrc; ++k) s += ldg<IO>(t.src[k], e);
+    } else if (g.accumulate) {
+      s = ldg<IO>(g.C, e) + s;
+    }
+    stg<IO>(g.C, e, s);
+  };
+  auto pairs = [&](int64_t e, auto count) {   // count pairs a thread, 512 elements apart
+    constexpr int J = decltype(count)::value;
+    d2 s[J];
+    if (add) {
+      d2 v[J];
 #pragma unroll
-    for (int k = 0; k < kMaxLevelSrc; ++k) v[k] = k < t.nsrc ? ldg<IO>(t.src[k], e) : 0.0;
-    double s = ldg<IO>(t.g.C, e);
+      for (int j = 0; j < J; ++j) {
+        v[j] = ldg2<IO>(g.A, e + 512 * j);
+        s[j] = g.accumulate ? ldg2<IO>(g.C, e + 512 * j) : d2{0.0, 0.0};
+      }
 #pragma unroll
-    for (int k = 0; k < kMaxLevelSrc; ++k)
-      if (k < t.nsrc) s += v[k];
-    stg<IO>(t.g.C, e, s);
-  }
+      for (int j = 0; j < J; ++j)
+        s[j] = g.accumulate ? s[j] + g.alpha * v[j] : g.alpha * v[j];
+    } else {
+      d2 v[kMaxLevelSrc - 1][J];
+#pragma unroll
+      for (int j = 0; j < J; ++j) s[j] = ldg2<IO>(g.C, e + 512 * j);
+#pragma unroll
+      for (int k = 0; k < kMaxLevelSrc - 1; ++k)
+        if (k < t.nsrc)
+#pragma unroll
+          for (int j = 0; j < J; ++j) v[k][j] = ldg2<IO>(t.src[k], e + 512 * j);
+#pragma unroll
+      for (int k = 0; k < kMaxLevelSrc - 1; ++k)
+        if (k < t.nsrc)
+#pragma unroll
+          for (int j = 0; j < J; ++j) s[j] += v[k][j];
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) stg2<IO>(g.C, e + 512 * j, s[j]);
+  };
+  int64_t e = e0 + 2 * threadIdx.x;
+  for (; e - 2 * threadIdx.x + 1024 <= e1; e += 1024) pairs(e, std::integral_constant<int, 2>{});
+  for (; e + 2 <= e1; e += 512) pairs(e, std::integral_constant<int, 1>{});
+  if (e < e1) one(e);
 }
 
-// P = 2^pshift threads share an element (splits p, p + P, ...), combined in p order
+// P = 2^pshift threads share an element (splits p, p + P, ...), combined in p
+// order; 256 / P elements a pass
 template <typename IO>
 __device__ __forceinline__ void level_reduce(const LevelTask& t, int idx, double* red) {
   const GemmArgs& g = t.g;
   const int P = 1 << t.pshift, p = threadIdx.x & (P - 1);
   const uint32_t total = (uint32_t)(g.M * g.N), N = (uint32_t)g.N;
-  const uint32_t e = (uint32_t)idx * (uint32_t)t.chunk + (threadIdx.x >> t.pshift);
-  double s = 0.0;
-  if (e < total) s = sum_strided(g.ws + (int64_t)p * total + e, (int64_t)P * total, (g.nsplit - p + P - 1) >> t.pshift);
-  if (P > 1) {
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if (p == 0)
-      for (int x = 1; x < P; ++x) s += red[threadIdx.x + x];
+  const uint32_t e0 = (uint32_t)idx * (uint32_t)t.chunk;
+  const uint32_t e1 = total - e0 < (uint32_t)t.chunk ? total : e0 + (uint32_t)t.chunk;
+  for (uint32_t b = e0; b < e1; b += 256u >> t.pshift) {
+    const uint32_t e = b + (threadIdx.x >> t.pshift);
+    double s = 0.0;
+    if (e < e1) s = sum_strided(g.ws + (int64_t)p * total + e, (int64_t)P * total, (g.nsplit - p + P - 1) >> t.pshift);
+    if (P > 1) {
+      if (b > e0) __syncthreads();
+      red[threadIdx.x] = s;
+      __syncthreads();
+      if (p == 0)
+        for (int x = 1; x < P; ++x) s += red[threadIdx.x + x];
+    }
+    if (e < e1 && p == 0) store_c<IO>(g, e / N, e % N, s);
   }
-  if (e < total && p == 0) store_c<IO>(g, e / N, e % N, s);
 }
 
 template <typename T, typename IO>
@@ -809,10 +877,10 @@ __global__ __launch_bounds__(256, kTileWaves<1>) void level_kernel(const LevelTa
   const int idx = it.idx;
   if (t.kind >= kLvPerm) {
     switch (t.kind) {
-      case kLvPerm:
-      case kLvFlat: level_add<IO>(t, idx); break;
+      case kLvPerm: level_perm<IO>(t, idx); break;
+      case kLvFlat:
+      case kLvSum: level_flat<IO>(t, idx); break;
       case kLvReduce: level_reduce<IO>(t, idx, reinterpret_cast<double*>(smem)); break;
-      case kLvSum: level_sum<IO>(t, idx); break;
       default: {
         const int64_t e0 = (int64_t)idx * t.chunk;
         const int64_t e1 = e0 + t.chunk < t.g.M ? e0 + t.chunk : t.g.M;
