@@ -213,8 +213,30 @@ __global__ void fill(double* __restrict__ x, int64_t n, double v) {
     x[e] = v;
 }
 
-// One thread per element of the full block; only canonical tuples (strictly
-// increasing inside every antisymmetric group) do work.
+// Sums over a block of 256 threads, valid in thread 0: lane exchanges inside a
+// wave, then the four waves in order (eight barriers of a tree in LDS otherwise).
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+__device__ __forceinline__ double block_sum(double v) {
+  __shared__ double red[4];
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return red[0] + red[1] + (red[2] + red[3]);
+}
+
+// Amplitude step of a block: for every canonical tuple (strictly increasing
+// inside each antisymmetric group) the mean R of the residual's signed images,
+// t -= R / (D + shift), and the new value to every image.  2^lshift lanes share a
+// tuple: lane l gathers and scatters images l, l + L, ..., the partial sums meet in
+// a butterfly.  Bound by latency while the tuples do not fill the chip, then
+// by the lines the images touch; so the images' strides are looked up once
+// a block, in LDS, and four images' loads are in flight (with the strides read
+// per image and one load at a time, a T3 block of 6160 tuples and 36 images
+// took 33 us, this 9; 65450 tuples 40, this 31).
 template <bool SUMSQ, typename IO, int RANK>
 __global__ __launch_bounds__(256) void jacobi_update(UpdateParams P, double* __restrict__ t,
                                                      const double* __restrict__ U,
@@ -222,24 +244,40 @@ __global__ __launch_bounds__(256) void jacobi_update(UpdateParams P, double* __r
                                                      const double* __restrict__ signs,
                                                      const double* __restrict__ fdiag_a,
                                                      const double* __restrict__ fdiag_b,
-                                                     double* __restrict__ sumsq) {
+                                                     double* __restrict__ sumsq, int lshift) {
   // the block's rank (P.rank) as a constant: every index loop unrolls
   constexpr int rank = RANK;
   constexpr int half = RANK / 2;
+  // stride of index d in image g (a block has fewer than 2^31 elements), sign of image g
+  extern __shared__ __align__(8) unsigned char lds[];
+  double* sg = reinterpret_cast<double*>(lds);
+  int* st = reinterpret_cast<int*>(sg + P.nimg);
+  for (int i = threadIdx.x; i < P.nimg * rank; i += 256) {
+    const int g = i / rank, d = i - g * rank, q = perms[g * 8 + d];
+    int64_t v = P.strides[0];
+#pragma unroll
+    for (int x = 1; x < rank; ++x)
+      if (q == x) v = P.strides[x];
+    st[i] = (int)v;
+    if (d == 0) sg[g] = signs[g];
+  }
+  __syncthreads();
+  const int L = 1 << lshift, lane = threadIdx.x & (L - 1);
+  const int64_t ngroups = ((int64_t)gridDim.x * blockDim.x) >> lshift;
   double sq = 0.0;
-  // one thread per canonical tuple (occupied half oc, virtual half vc; the
-  // virtual half runs fastest, so the identity image is read and written
-  // along its last index)
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < P.total;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    int64_t idx[8];
+  for (int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> lshift; e < P.total; e += ngroups) {
+    // occupied half oc, virtual half vc; the virtual half runs fastest, so the
+    // identity image is read and written along its last index
+    int idx[8];
     const int64_t oc = e / P.n_vc, vc = e - oc * P.n_vc;
+#pragma unroll
     for (int d = 0; d < half; ++d) {
       idx[d] = P.coc[oc * half + d];
       idx[half + d] = P.cvc[vc * half + d];
     }
     if (P.mask) {
       bool occ_act = false, vir_a = false, vir_b = false;
+#pragma unroll
       for (int d = 0; d < rank; ++d) {
         if (!P.isvir[d]) {
           occ_act |= idx[d] >= P.occ_start;
@@ -251,114 +289,45 @@ __global__ __launch_bounds__(256) void jacobi_update(UpdateParams P, double* __r
       const bool forbid = ((P.vforbid & 1) && vir_a) || ((P.vforbid & 2) && vir_b);
       if (!occ_act || !need || forbid) continue;
     }
-    double R = 0.0;
-    for (int g = 0; g < P.nimg; ++g) {
-      int64_t off = 0;
-      for (int d = 0; d < rank; ++d) off += idx[d] * P.strides[perms[g * 8 + d]];
-      R += signs[g] * ldg<IO>(U, off);
-    }
-    R /= (double)P.nimg;
-    if (SUMSQ) sq += (double)P.nimg * R * R;
+    auto offset = [&](int g) {
+      int off = 0;
+#pragma unroll
+      for (int d = 0; d < rank; ++d) off += idx[d] * st[g * rank + d];
+      return off;
+    };
     double D = 0.0;
+#pragma unroll
     for (int d = 0; d < rank; ++d)
       if (P.isvir[d]) D += (P.spin[d] ? fdiag_b : fdiag_a)[P.occ[d] + idx[d]];
+#pragma unroll
     for (int d = 0; d < rank; ++d)
       if (!P.isvir[d]) D -= (P.spin[d] ? fdiag_b : fdiag_a)[idx[d]];
     D += P.shift;
     int64_t off0 = 0;
-    for (int d = 0; d < rank; ++d) off0 += idx[d] * P.strides[d];
-    const double tn = t[off0] - R / D;
-    for (int g = 0; g < P.nimg; ++g) {
-      int64_t off = 0;
-      for (int d = 0; d < rank; ++d) off += idx[d] * P.strides[perms[g * 8 + d]];
-      t[off] = signs[g] * tn;
-    }
-  }
-  if (SUMSQ) {
-    __shared__ double red[256];
-    red[threadIdx.x] = sq;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) sumsq[blockIdx.x] = red[0];
-  }
-}
-
-// The same step with one wave per canonical tuple, for blocks with many
-// images (a T4 block of one spin has 576): lane l gathers and scatters images
-// l, l + 64, ...; the image sum is a fixed butterfly over the wave.
-template <bool SUMSQ, typename IO, int RANK>
-__global__ __launch_bounds__(256) void jacobi_update_wave(UpdateParams P, double* __restrict__ t,
-                                                          const double* __restrict__ U,
-                                                          const int* __restrict__ perms,
-                                                          const double* __restrict__ signs,
-                                                          const double* __restrict__ fdiag_a,
-                                                          const double* __restrict__ fdiag_b,
-                                                          double* __restrict__ sumsq) {
-  // the block's rank (P.rank) as a constant: every index loop unrolls
-  constexpr int rank = RANK;
-  constexpr int half = RANK / 2;
-  const int lane = threadIdx.x & 63;
-  const int64_t nwaves = ((int64_t)gridDim.x * blockDim.x) >> 6;
-  double sq = 0.0;
-  for (int64_t e = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; e < P.total; e += nwaves) {
-    int64_t idx[8];
-    const int64_t oc = e / P.n_vc, vc = e - oc * P.n_vc;
-    for (int d = 0; d < half; ++d) {
-      idx[d] = P.coc[oc * half + d];
-      idx[half + d] = P.cvc[vc * half + d];
-    }
-    if (P.mask) {
-      bool occ_act = false, vir_a = false, vir_b = false;
-      for (int d = 0; d < rank; ++d) {
-        if (!P.isvir[d]) {
-          occ_act |= idx[d] >= P.occ_start;
-        } else if (idx[d] < P.vir_end[P.spin[d]]) {
-          if (P.spin[d]) vir_b = true; else vir_a = true;
-        }
-      }
-      const bool need = ((P.vneed & 1) && vir_a) || ((P.vneed & 2) && vir_b);
-      const bool forbid = ((P.vforbid & 1) && vir_a) || ((P.vforbid & 2) && vir_b);
-      if (!occ_act || !need || forbid) continue;
-    }
-    double R = 0.0;
-    for (int g = lane; g < P.nimg; g += 64) {
-      int64_t off = 0;
-      for (int d = 0; d < rank; ++d) off += idx[d] * P.strides[perms[g * 8 + d]];
-      R += signs[g] * ldg<IO>(U, off);
-    }
 #pragma unroll
-    for (int m = 32; m > 0; m >>= 1) R += __shfl_xor(R, m);
+    for (int d = 0; d < rank; ++d) off0 += idx[d] * P.strides[d];
+    const double t0 = t[off0];
+    double R = 0.0;
+    for (int g = lane; g < P.nimg; g += 4 * L) {
+      double u[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[j] = ldg<IO>(U, offset(g + j * L < P.nimg ? g + j * L : g));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (g + j * L < P.nimg) R += sg[g + j * L] * u[j];
+    }
+    for (int m = L >> 1; m > 0; m >>= 1) R += __shfl_xor(R, m);
     R /= (double)P.nimg;
     if (SUMSQ && lane == 0) sq += (double)P.nimg * R * R;
-    double D = 0.0;
-    for (int d = 0; d < rank; ++d)
-      if (P.isvir[d]) D += (P.spin[d] ? fdiag_b : fdiag_a)[P.occ[d] + idx[d]];
-    for (int d = 0; d < rank; ++d)
-      if (!P.isvir[d]) D -= (P.spin[d] ? fdiag_b : fdiag_a)[idx[d]];
-    D += P.shift;
-    int64_t off0 = 0;
-    for (int d = 0; d < rank; ++d) off0 += idx[d] * P.strides[d];
-    // every lane has read t[off0] before any lane stores an image (the store
-    // depends on tn)
-    const double tn = t[off0] - R / D;
-    for (int g = lane; g < P.nimg; g += 64) {
-      int64_t off = 0;
-      for (int d = 0; d < rank; ++d) off += idx[d] * P.strides[perms[g * 8 + d]];
-      t[off] = signs[g] * tn;
-    }
+    // every lane has read t0 before any lane stores an image (the stores
+    // depend on all lanes' sums)
+    const double tn = t0 - R / D;
+#pragma unroll 4
+    for (int g = lane; g < P.nimg; g += L) t[offset(g)] = sg[g] * tn;
   }
   if (SUMSQ) {
-    __shared__ double red[256];
-    red[threadIdx.x] = sq;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if ((int)threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) sumsq[blockIdx.x] = red[0];
+    sq = block_sum(sq);
+    if (threadIdx.x == 0) sumsq[blockIdx.x] = sq;
   }
 }
 
@@ -532,21 +501,6 @@ __global__ __launch_bounds__(256) void cct3_correction(Cct3Params P, const doubl
   }
   if (threadIdx.x == 0)
     for (int x = 0; x < 4; ++x) partial[blockIdx.x * 4 + x] = red[x][0];
-}
-
-// Sums over a block of 256 threads, valid in thread 0: lane exchanges inside a
-// wave, then the four waves in order (eight barriers of a tree in LDS otherwise).
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-__device__ __forceinline__ double block_sum(double v) {
-  __shared__ double red[4];
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return red[0] + red[1] + (red[2] + red[3]);
 }
 
 // The correlation energy in one launch: a block's sum over its share of the tiles.
@@ -1141,10 +1095,19 @@ hipError_t launch_fill(hipStream_t s, double* x, int64_t n, double v) {
   return hipGetLastError();
 }
 
-// blocks with at least kWaveImages images run one wave per canonical tuple
-constexpr int kWaveImages = 128;
+// lanes of a tuple, as a shift: a wave where there are images for it (a T4 block
+// of one spin has 576); else 4 or 16 while the tuples leave the SIMDs without a
+// second wave each.  us with 1 / 4 / 16 lanes: 6160 tuples of 36 images 16.9 / 10.2 /
+// 9.1, 27225 tuples of rank 8 11.8 / 9.4 / 15.3, 65450 of 36 images 31 / 34 / 43.
+static int update_lanes(const UpdateParams& P) {
+  if (P.nimg >= 128) return 6;
+  int l = 0;
+  while (l < 4 && (4 << l) <= P.nimg && (P.total << l) < 256 * 128) l += 2;
+  return l;
+}
 int update_blocks(const UpdateParams& P) {
-  return P.nimg >= kWaveImages ? grid_for(P.total * 64, 256, 16384) : grid_for(P.total, 256);
+  const int l = update_lanes(P);
+  return grid_for(P.total << l, 256, l == 6 ? 16384 : 4096);
 }
 
 template <typename IO, int R>
@@ -1152,17 +1115,13 @@ static void launch_update_r(hipStream_t s, const UpdateParams& P, double* t, con
                             const int* perms, const double* signs, const double* fa,
                             const double* fb, double* sumsq) {
   const dim3 grid(update_blocks(P)), blk(256);
-  if (P.nimg >= kWaveImages) {
-    if (sumsq)
-      hipLaunchKernelGGL((jacobi_update_wave<true, IO, R>), grid, blk, 0, s, P, t, U, perms, signs, fa, fb, sumsq);
-    else
-      hipLaunchKernelGGL((jacobi_update_wave<false, IO, R>), grid, blk, 0, s, P, t, U, perms, signs, fa, fb, sumsq);
-    return;
-  }
+  const size_t lds = (size_t)P.nimg * (sizeof(double) + R * sizeof(int));
   if (sumsq)
-    hipLaunchKernelGGL((jacobi_update<true, IO, R>), grid, blk, 0, s, P, t, U, perms, signs, fa, fb, sumsq);
+    hipLaunchKernelGGL((jacobi_update<true, IO, R>), grid, blk, lds, s, P, t, U, perms, signs, fa, fb, sumsq,
+                       update_lanes(P));
   else
-    hipLaunchKernelGGL((jacobi_update<false, IO, R>), grid, blk, 0, s, P, t, U, perms, signs, fa, fb, sumsq);
+    hipLaunchKernelGGL((jacobi_update<false, IO, R>), grid, blk, lds, s, P, t, U, perms, signs, fa, fb, sumsq,
+                       update_lanes(P));
 }
 
 template <typename IO>
@@ -1183,6 +1142,7 @@ hipError_t launch_update(hipStream_t s, const UpdateParams& P, double* t, const 
   if (!P.coc || !P.cvc || P.n_vc <= 0) return hipErrorInvalidValue;
   if (P.rank != 2 && P.rank != 4 && P.rank != 6 && P.rank != 8) return hipErrorInvalidValue;
   if (P.total <= 0) return hipSuccess;
+  if (P.nimg < 1 || P.nimg > 1152) return hipErrorInvalidValue;   // 45 KB of LDS at rank 8
   if (P.u32) launch_update_io<float>(s, P, t, U, perms, signs, fa, fb, sumsq);
   else launch_update_io<double>(s, P, t, U, perms, signs, fa, fb, sumsq);
   return hipGetLastError();
