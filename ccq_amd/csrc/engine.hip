@@ -870,7 +870,8 @@ struct ccq_hip_ctx {
       }
     }
     if (!view_perm) return;
-    std::vector<std::vector<OrderedOp>> uses(tensors.size());
+    std::vector<OrderedOp> all;
+    std::vector<std::vector<int>> uses(tensors.size());   // (all)
     std::vector<std::vector<int>> shared(tensors.size());
     std::vector<int> lead(tensors.size());
     for (int t = 0; t < (int)tensors.size(); ++t) {
@@ -883,17 +884,20 @@ struct ccq_hip_ctx {
     for (int si = 0; si < (int)sections.size(); ++si)
       for (int i = 0; i < (int)sections[si].ops.size(); ++i) {
         const Op& op = sections[si].ops[i];
-        const OrderedOp o = ordered_op(si, i);
+        all.push_back(ordered_op(si, i));
         int ts[3] = {lead[op.a], lead[op.out], op.gemm ? lead[op.b] : -1};
         for (int k = 0; k < 3; ++k)
-          if (ts[k] >= 0 && (k < 1 || ts[k] != ts[0]) && (k < 2 || ts[k] != ts[1])) uses[ts[k]].push_back(o);
+          if (ts[k] >= 0 && (k < 1 || ts[k] != ts[0]) && (k < 2 || ts[k] != ts[1])) uses[ts[k]].push_back((int)all.size() - 1);
       }
+    std::vector<char> open(tensors.size(), 1);   // an operation's other tensors may have changed since
     for (int round = 0; round < 3; ++round) {
       bool changed = false;
       for (int t = 0; t < (int)tensors.size(); ++t) {
         const Tensor& T = tensors[t];
+        if (!open[t]) continue;
+        open[t] = 0;
         double time = 0;
-        for (const OrderedOp& o : uses[t]) time += o.time;
+        for (int u : uses[t]) time += all[u].time;
         // the CC(t;3) kernels index the tail's tensors by their declared order
         if (lead[t] != t || time < kOrderTime || T.rank < 2 || T.rank > 4 || T.id.rfind("cct3:", 0) == 0 ||
             (T.kind != TKind::Inter && T.kind != TKind::View))
@@ -903,7 +907,8 @@ struct ccq_hip_ctx {
         double least = -1.0, keep = 0.0;
         do {
           double c = 0;
-          for (const OrderedOp& o : uses[t]) {
+          for (int u : uses[t]) {
+            const OrderedOp& o = all[u];
             const Op& op = sections[o.sec].ops[o.op];
             c += op_cost(o, op.gemm, lead[op.a] == t ? permuted(op.la, p) : op.la,
                          op.gemm && lead[op.b] == t ? permuted(op.lb, p) : op.lb,
@@ -916,7 +921,13 @@ struct ccq_hip_ctx {
           }
         } while (std::next_permutation(p.begin(), p.end()));
         if (least < 0.999 * keep) {
-          set_order(t, lead, shared[t], uses[t], best);
+          for (int u : uses[t]) {
+            Op& op = sections[all[u].sec].ops[all[u].op];
+            order_op(t, lead, op, best);
+            for (int x : {lead[op.a], lead[op.out], op.gemm ? lead[op.b] : t})
+              if (x != t) open[x] = 1;
+          }
+          set_order(shared[t], best);
           changed = true;
         }
       }
@@ -931,14 +942,12 @@ struct ccq_hip_ctx {
     return spec[0] == 'o' ? occ : nc - occ;
   }
   // new index i of tensor t (and of the views sharing its storage) is old index p[i]
-  void set_order(int t, const std::vector<int>& lead, const std::vector<int>& shared, const std::vector<OrderedOp>& uses,
-                 const std::vector<int>& p) {
-    for (const OrderedOp& o : uses) {
-      Op& op = sections[o.sec].ops[o.op];
-      if (lead[op.a] == t) op.la = permuted(op.la, p);
-      if (op.gemm && lead[op.b] == t) op.lb = permuted(op.lb, p);
-      if (lead[op.out] == t) op.lc = permuted(op.lc, p);
-    }
+  static void order_op(int t, const std::vector<int>& lead, Op& op, const std::vector<int>& p) {
+    if (lead[op.a] == t) op.la = permuted(op.la, p);
+    if (op.gemm && lead[op.b] == t) op.lb = permuted(op.lb, p);
+    if (lead[op.out] == t) op.lc = permuted(op.lc, p);
+  }
+  void set_order(const std::vector<int>& shared, const std::vector<int>& p) {
     for (int x : shared) {
       Tensor& T = tensors[x];
       const Tensor o = T;
