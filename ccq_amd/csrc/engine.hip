@@ -2893,7 +2893,8 @@ struct ccq_hip_ctx {
     // A product whose single workgroups outlast the rest of their level by more
     // than the extra level of a split is split along K; one with tiles for half
     // the chip (its partials then cost more than idle CUs) only beyond a third
-    // of a long level.
+    // of a long level, one of a small output beyond a sixteenth (to the shortest item
+    // whatever the level: CCSD, 100 orbitals, 1874 us a sweep, this 1846; a sixth: 1867).
     std::vector<int64_t> partials(s1.levels + 1, 0);
     for (size_t u = 0; u < units.size(); ++u)
       for (size_t k = 0; k < us[u].ops.size(); ++k) {
@@ -2901,7 +2902,7 @@ struct ccq_hip_ctx {
         if (!op.gemm || own_launch(op) || op.K == 0) continue;
         ccqk::GemmArgs& g = plans[u][k];
         const TileCost c = tile_cost(op, g);
-        const double span = op.M * op.N <= kSplitDot ? kSplitSpan
+        const double span = op.M * op.N <= kSplitDot ? std::max(load[first[u].level] / 16.0, kSplitSpan)
                             : c.tiles < 128          ? std::max(load[first[u].level] / 4.0, kSplitSpan)
                                                      : std::max(load[first[u].level] / 3.0, kSplitWide);
         if (c.item < span + kSplitGain) continue;
