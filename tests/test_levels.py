@@ -121,7 +121,7 @@ int main(int argc, char** argv) {
 
 
 @pytest.fixture(scope="module")
-def checker(tmp_path_factory):
+def program(tmp_path_factory):
     d = tmp_path_factory.mktemp("levels")
     (d / "t.cpp").write_text(SRC)
     exe = str(d / "t")
@@ -131,7 +131,7 @@ def checker(tmp_path_factory):
 
 
 @pytest.mark.parametrize("seed", [1, 2, 3, 4])
-def test_levels_equal_program_order(checker, seed):
-    r = subprocess.run([checker, str(seed)], capture_output=True, text=True, timeout=120)
+def test_levels_equal_program_order(program, seed):
+    r = subprocess.run([program, str(seed)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
     assert r.stdout.strip() == "ok"
