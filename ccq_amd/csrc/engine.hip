@@ -2694,6 +2694,7 @@ struct ccq_hip_ctx {
 
   void sweep(int64_t nsec = -1) {
     if (prec == 2) prep_sweep32();
+    if (use_levels() && !profile && nsec < 0) prep_levels("sweep");
     run_program("sweep", nsec);
   }
 
@@ -3150,9 +3151,12 @@ struct ccq_hip_ctx {
       g.C = dst(ts.tensor, ts.slot);
       g.accumulate = ts.overwrite ? 0 : 1;
     }
-    HIPCHK(hipMalloc(&lp.tasks[st], sizeof(ccqk::LevelTask) * std::max<size_t>(v.size(), 1)));
-    if (!v.empty())
-      HIPCHK(hipMemcpy(lp.tasks[st], v.data(), sizeof(ccqk::LevelTask) * v.size(), hipMemcpyHostToDevice));
+    ccqk::LevelTask* d = nullptr;
+    HIPCHK(hipMalloc(&d, sizeof(ccqk::LevelTask) * std::max<size_t>(v.size(), 1)));
+    const hipError_t e = hipMemcpy(d, v.data(), sizeof(ccqk::LevelTask) * v.size(), hipMemcpyHostToDevice);
+    if (e != hipSuccess) (void)hipFree(d);
+    HIPCHK(e);
+    lp.tasks[st] = d;   // only a whole table is ever launched
   }
 
   // outside any capture: the schedule of a program and its tables
@@ -3179,6 +3183,7 @@ struct ccq_hip_ctx {
   void run_levels(const std::string& prog) {
     LevelProg& lp = level_progs.at(prog);
     const int st = run_prec == 2;
+    if (!lp.tasks[st]) throw Fail("level tables of program " + prog + " not prepared");
     for (const LevelStep& step : lp.steps) {
       for (size_t k = 0; k < step.own.size(); ++k) {
         const Section& sec = sections[step.own[k].first];

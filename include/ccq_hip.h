@@ -245,7 +245,9 @@ int ccq_hip_profile_report(ccq_hip_ctx* ctx, char* buf, int64_t buflen);
  * mode 2 sweep, intermediates and residuals hold the last FP64 / mode-1
  * sweep's values (amplitude blocks are always current). */
 int ccq_hip_debug_read(ccq_hip_ctx* ctx, const char* tensor_id, double* out, int64_t n);
-/* Run only the first nsections sections of one sweep (inspection only). */
+/* Run only the first nsections sections of one sweep, operation by operation
+ * (inspection only); nsections < 0: a whole sweep as ccq_hip_update runs it,
+ * without the graph. */
 int ccq_hip_debug_sweep(ccq_hip_ctx* ctx, int64_t nsections);
 
 /* Block until the context's stream is idle. */
