@@ -21,13 +21,12 @@
 #include <sstream>
 #include <stdexcept>
 #include <string>
-#include <system_error>
-#include <thread>
 #include <vector>
 
 #include "../../include/ccq_hip.h"
 #include "kernels.h"
 #include "levels.h"
+#include "pool.h"
 #include "restart_io.h"
 
 #include "ir_ccsd_rhf.inc"
@@ -124,14 +123,7 @@ class Download {
         std::memcpy(static_cast<char*>(dst) + o, buf, len);
       }
     };
-    std::vector<std::thread> pool;
-    pool.reserve(n);
-    try {
-      for (int w = 1; w < n; ++w) pool.emplace_back(work, w);
-    } catch (const std::system_error&) {   // fewer threads than hoped for
-    }
-    work(0);
-    for (std::thread& t : pool) t.join();
+    ccqpool::run(n, work);
     if (err != (int)hipSuccess) {
       (void)hipStreamSynchronize(stream);   // no copy into the pinned buffers is left
       throw Fail(std::string("download: ") + hipGetErrorString((hipError_t)err.load()));
