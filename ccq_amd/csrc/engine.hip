@@ -93,6 +93,7 @@ struct PinnedVec {
 class Download {
  public:
   void run(int device, hipStream_t stream, void* dst, const void* src, size_t bytes) {
+    if (!dst && bytes) throw Fail("download: null destination");
     if (bytes < kMin || known(dst)) {
       HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
       HIPCHK(hipStreamSynchronize(stream));
