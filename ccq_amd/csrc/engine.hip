@@ -1097,7 +1097,9 @@ struct ccq_hip_ctx {
         const size_t bytes = sizeof(float) * (size_t)std::max<int64_t>(n, 1);
         HIPCHK(hipMalloc(&p, bytes));
         f32_bufs.push_back(p);
-        HIPCHK(hipMemset(p, 0, bytes));
+        // on the context's stream, which does not wait for the null stream: the
+        // casts below write the same memory
+        HIPCHK(hipMemsetAsync(p, 0, bytes, stream));
         return p;
       };
       tvec32 = alloc32(dev_t);
