@@ -2539,11 +2539,12 @@ struct ccq_hip_ctx {
     }
   }
 
-  void run_add(const Op& op, const double* A, double* C, int acc) {
-    const int io32 = run_prec == 2;
+  // c64: C is FP64 in an FP32-storage sweep too (GemmArgs::c64)
+  void run_add(const Op& op, const double* A, double* C, int acc, int c64 = 0) {
+    const int io32 = run_prec == 2 ? 1 + c64 : 0;
     // the float form has no alignment condition
     const bool aligned = io32 || ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(C)) & 15) == 0;
-    if (op.flat && aligned)
+    if (op.flat && aligned && !c64)
       HIPCHK(ccqk::launch_axpy_flat(stream, op.M * op.N, A, C, op.coef, acc, io32));
     else
       HIPCHK(ccqk::launch_perm_add(stream, op.M, op.N, A, tables32 + op.t_rowA, tables32 + op.t_kA, C,
@@ -2732,8 +2733,9 @@ struct ccq_hip_ctx {
   // (an allocation of its own for each took 25 ms of a small system's set-up)
   std::map<std::pair<int, int>, int64_t> slot_off;
   int64_t slot_need = 0;
+  // FP64 in every precision mode: an FP32-storage sweep rounds a sum of
+  // partial accumulators once, when it is added to the accumulator itself
   DevBuf slots;
-  float* slots32 = nullptr;
   DevBuf lv_ws;
   int64_t lv_ws_need = 0;
   bool use_levels() const { return group; }
@@ -3098,11 +3100,7 @@ struct ccq_hip_ctx {
   // device task table of a program for the storage of run_prec
   void bind_levels(LevelProg& lp, int st) {
     if (lp.tasks[st]) return;
-    auto dst = [&](int t, int s) -> double* {
-      if (!s) return sp(t);
-      const int64_t o = slot_off.at({t, s});
-      return st ? reinterpret_cast<double*>(slots32 + o) : slots.p + o;
-    };
+    auto dst = [&](int t, int s) { return s ? slots.p + slot_off.at({t, s}) : sp(t); };
     std::vector<ccqk::LevelTask>& v = lp.host[st];
     v.assign(lp.src.size(), ccqk::LevelTask{});
     for (size_t i = 0; i < lp.src.size(); ++i) {
@@ -3116,6 +3114,7 @@ struct ccq_hip_ctx {
         g.M = tensor_size(ts.tensor);
         g.N = 1;
         g.C = dst(ts.tensor, ts.kind == ccqk::kLvSum ? 0 : ts.slot);
+        g.c64 = st && ts.kind == ccqk::kLvZero;
         t.nsrc = ts.kind == ccqk::kLvSum ? ts.nslots - 1 : 0;
         for (int k = 0; k < t.nsrc; ++k) t.src[k] = dst(ts.tensor, k + 1);
         continue;
@@ -3144,6 +3143,7 @@ struct ccq_hip_ctx {
         if (op.M * op.N > 0x7fffffffLL) throw Fail("level add too large");
       }
       g.C = dst(ts.tensor, ts.slot);
+      g.c64 = st && ts.slot > 0;
       g.accumulate = ts.overwrite ? 0 : 1;
     }
     ccqk::LevelTask* d = nullptr;
@@ -3160,10 +3160,6 @@ struct ccq_hip_ctx {
     if (!level_progs.count(prog)) throw Fail("no level schedule of program " + prog);
     LevelProg& lp = level_progs.at(prog);
     if (lp.tasks[st]) return;
-    if (st && !slots32 && slot_need) {
-      HIPCHK(hipMalloc(&slots32, sizeof(float) * slot_need));
-      f32_bufs.push_back(slots32);
-    }
     const int keep = run_prec;
     run_prec = st ? 2 : 0;
     try {
@@ -3201,7 +3197,7 @@ struct ccq_hip_ctx {
           g.ws = cur_ws;
           HIPCHK(ccqk::launch_gemm(stream, g));
         } else {
-          run_add(op, g.A, g.C, g.accumulate);
+          run_add(op, g.A, g.C, g.accumulate, g.c64);
         }
       }
       HIPCHK(ccqk::launch_level(stream, run_prec, lp.tasks[st], lp.items + step.item0, step.nitems));

@@ -44,23 +44,19 @@ __device__ __forceinline__ void put_c(double* base, int64_t off, double v, int a
   if (accumulate) stg<IO>(base, off, ldg<IO>(base, off) + v); else stg<IO>(base, off, v);
 }
 
-template <typename IO>
+// IOC: the stored type of C (GemmArgs::c64: double beside float operands)
+template <typename IO, typename IOC = IO>
 __device__ __forceinline__ void store_c(const GemmArgs& g, int64_t m, int64_t n, double s, double alpha) {
   const int64_t r = g.rowC[m], c = g.colC[n];
   double v = alpha * s;
   if (g.D) v += g.dcoef * ldg<IO>(g.D, (int64_t)g.rowD[m] + g.colD[n]);
-  put_c<IO>(g.C, r + c, v, g.accumulate);
+  put_c<IOC>(g.C, r + c, v, g.accumulate);
   if (g.rowC2) {
     const int64_t r2 = g.rowC2[m];
-    put_c<IO>(g.C, r2 + c, -v, g.accumulate);
-    if (g.colC2) put_c<IO>(g.C, r2 + g.colC2[n], v, g.accumulate);
+    put_c<IOC>(g.C, r2 + c, -v, g.accumulate);
+    if (g.colC2) put_c<IOC>(g.C, r2 + g.colC2[n], v, g.accumulate);
   }
-  if (g.colC2) put_c<IO>(g.C, r + g.colC2[n], -v, g.accumulate);
-}
-
-template <typename IO>
-__device__ __forceinline__ void store_c(const GemmArgs& g, int64_t m, int64_t n, double s) {
-  store_c<IO>(g, m, n, s, g.alpha);
+  if (g.colC2) put_c<IOC>(g.C, r + g.colC2[n], -v, g.accumulate);
 }
 
 // sum_{i < cnt} q[i * stride] with four interleaved partial sums (fixed order)
@@ -327,7 +323,7 @@ struct Mma<float> {
 // epilogue serialises a table load, a C load and the store for every
 // element.  Outputs with mirrored images (packed pairs) take the
 // element-by-element path.
-template <typename IO, int TM, int TN, typename MM, typename V>
+template <typename IO, typename IOC, int TM, int TN, typename MM, typename V>
 __device__ __forceinline__ void store_tile(const GemmArgs& g, int64_t m0, int64_t n0, int wm, int wn, int lane,
                                            double alpha, const V (&val)[TM][TN]) {
   if (g.rowC2 || g.colC2) {
@@ -340,7 +336,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, int64_t m0, int64_
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
           const int64_t gm = m0 + wm + 16 * i + MM::row(lane, v);
-          if (gm < g.M) store_c<IO>(g, gm, gn, (double)val[i][j][v], alpha);
+          if (gm < g.M) store_c<IO, IOC>(g, gm, gn, (double)val[i][j][v], alpha);
         }
     }
     return;
@@ -382,7 +378,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, int64_t m0, int64_
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) old[i][v] = rc[i][v] >= 0 ? ldg<IO>(g.C, (int64_t)rc[i][v] + cc) : 0.0;
+        for (int v = 0; v < 4; ++v) old[i][v] = rc[i][v] >= 0 ? ldg<IOC>(g.C, (int64_t)rc[i][v] + cc) : 0.0;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -392,7 +388,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, int64_t m0, int64_
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        if (rc[i][v] >= 0) stg<IO>(g.C, (int64_t)rc[i][v] + cc, out[i][v]);
+        if (rc[i][v] >= 0) stg<IOC>(g.C, (int64_t)rc[i][v] + cc, out[i][v]);
   }
 }
 
@@ -605,7 +601,10 @@ __device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty,
   }
 
   if (g.nsplit == 1) {
-    store_tile<IO, TM, TN, MM>(g, m0, n0, wm, wn, lane, g.alpha, acc);
+    if (sizeof(IO) == 4 && g.c64)
+      store_tile<IO, double, TM, TN, MM>(g, m0, n0, wm, wn, lane, g.alpha, acc);
+    else
+      store_tile<IO, IO, TM, TN, MM>(g, m0, n0, wm, wn, lane, g.alpha, acc);
     return;
   }
 #pragma unroll
@@ -681,7 +680,7 @@ __device__ __forceinline__ void tile_entries(const GemmArgs* es, int e0, int e1,
   }
 
   if (kend < 0 || o.nsplit == 1) {
-    store_tile<IO, TM, TN, MM>(o, m0, n0, wm, wn, lane, 1.0, sum);
+    store_tile<IO, IO, TM, TN, MM>(o, m0, n0, wm, wn, lane, 1.0, sum);
     return;
   }
 #pragma unroll
@@ -753,7 +752,8 @@ __device__ __forceinline__ void stg2(double* p, int64_t i, d2 v) {
   *reinterpret_cast<typename Pair2<IO>::type*>(reinterpret_cast<IO*>(p) + i) = w;
 }
 
-template <typename IO>
+// (IOC: the stored type of C, as in store_c)
+template <typename IO, typename IOC>
 __device__ __forceinline__ void level_perm(const LevelTask& t, int idx) {
   const GemmArgs& g = t.g;
   const uint32_t N = (uint32_t)g.N, total = (uint32_t)(g.M * g.N);
@@ -773,11 +773,11 @@ __device__ __forceinline__ void level_perm(const LevelTask& t, int idx) {
 #pragma unroll
     for (int j = 0; j < J; ++j) {
       v[j] = ldg<IO>(g.A, ia[j]);
-      c[j] = g.accumulate ? ldg<IO>(g.C, ic[j]) : 0.0;
+      c[j] = g.accumulate ? ldg<IOC>(g.C, ic[j]) : 0.0;
     }
 #pragma unroll
     for (int j = 0; j < J; ++j)
-      if (b + 256u * j < e1) stg<IO>(g.C, ic[j], g.accumulate ? c[j] + g.alpha * v[j] : g.alpha * v[j]);
+      if (b + 256u * j < e1) stg<IOC>(g.C, ic[j], g.accumulate ? c[j] + g.alpha * v[j] : g.alpha * v[j]);
   };
   uint32_t b = e0 + threadIdx.x;
   if (t.chunk > 512)
@@ -787,7 +787,7 @@ __device__ __forceinline__ void level_perm(const LevelTask& t, int idx) {
 }
 
 // C (+)= alpha A (n = 0), or C += the sum of n arrays; whole pairs, then the last one
-template <typename IO>
+template <typename IO, typename IOC>
 __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
   const GemmArgs& g = t.g;
   const int64_t total = t.kind == kLvSum ? g.M : g.M * g.N, e0 = (int64_t)idx * t.chunk;
@@ -796,12 +796,12 @@ __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
   auto one = [&](int64_t e) {
     double s = add ? g.alpha * ldg<IO>(g.A, e) : 0.0;
     if (!add) {
-      s = ldg<IO>(g.C, e);
-      for (int k = 0; k < t.nsrc; ++k) s += ldg<IO>(t.src[k], e);
+      s = ldg<IOC>(g.C, e);
+      for (int k = 0; k < t.nsrc; ++k) s += ldg<double>(t.src[k], e);
     } else if (g.accumulate) {
-      s = ldg<IO>(g.C, e) + s;
+      s = ldg<IOC>(g.C, e) + s;
     }
-    stg<IO>(g.C, e, s);
+    stg<IOC>(g.C, e, s);
   };
   auto pairs = [&](int64_t e, auto count) {   // count pairs a thread, 512 elements apart
     constexpr int J = decltype(count)::value;
@@ -811,7 +811,7 @@ __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
 #pragma unroll
       for (int j = 0; j < J; ++j) {
         v[j] = ldg2<IO>(g.A, e + 512 * j);
-        s[j] = g.accumulate ? ldg2<IO>(g.C, e + 512 * j) : d2{0.0, 0.0};
+        s[j] = g.accumulate ? ldg2<IOC>(g.C, e + 512 * j) : d2{0.0, 0.0};
       }
 #pragma unroll
       for (int j = 0; j < J; ++j)
@@ -819,12 +819,12 @@ __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
     } else {
       d2 v[kMaxLevelSrc - 1][J];
 #pragma unroll
-      for (int j = 0; j < J; ++j) s[j] = ldg2<IO>(g.C, e + 512 * j);
+      for (int j = 0; j < J; ++j) s[j] = ldg2<IOC>(g.C, e + 512 * j);
 #pragma unroll
       for (int k = 0; k < kMaxLevelSrc - 1; ++k)
         if (k < t.nsrc)
 #pragma unroll
-          for (int j = 0; j < J; ++j) v[k][j] = ldg2<IO>(t.src[k], e + 512 * j);
+          for (int j = 0; j < J; ++j) v[k][j] = ldg2<double>(t.src[k], e + 512 * j);
 #pragma unroll
       for (int k = 0; k < kMaxLevelSrc - 1; ++k)
         if (k < t.nsrc)
@@ -832,7 +832,7 @@ __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
           for (int j = 0; j < J; ++j) s[j] += v[k][j];
     }
 #pragma unroll
-    for (int j = 0; j < J; ++j) stg2<IO>(g.C, e + 512 * j, s[j]);
+    for (int j = 0; j < J; ++j) stg2<IOC>(g.C, e + 512 * j, s[j]);
   };
   int64_t e = e0 + 2 * threadIdx.x;
   for (; e - 2 * threadIdx.x + 1024 <= e1; e += 1024) pairs(e, std::integral_constant<int, 2>{});
@@ -842,7 +842,7 @@ __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
 
 // P = 2^pshift threads share an element (splits p, p + P, ...), combined in p
 // order; 256 / P elements a pass
-template <typename IO>
+template <typename IO, typename IOC>
 __device__ __forceinline__ void level_reduce(const LevelTask& t, int idx, double* red) {
   const GemmArgs& g = t.g;
   const int P = 1 << t.pshift, p = threadIdx.x & (P - 1);
@@ -860,7 +860,7 @@ __device__ __forceinline__ void level_reduce(const LevelTask& t, int idx, double
       if (p == 0)
         for (int x = 1; x < P; ++x) s += red[threadIdx.x + x];
     }
-    if (e < e1 && p == 0) store_c<IO>(g, e / N, e % N, s);
+    if (e < e1 && p == 0) store_c<IO, IOC>(g, e / N, e % N, s, g.alpha);
   }
 }
 
@@ -876,17 +876,27 @@ __global__ __launch_bounds__(256, kTileWaves<1>) void level_kernel(const LevelTa
   const LevelTask& t = *(const LevelTask*)((ConstTask)tasks + it.task);
   const int idx = it.idx;
   if (t.kind >= kLvPerm) {
-    switch (t.kind) {
-      case kLvPerm: level_perm<IO>(t, idx); break;
-      case kLvFlat:
-      case kLvSum: level_flat<IO>(t, idx); break;
-      case kLvReduce: level_reduce<IO>(t, idx, reinterpret_cast<double*>(smem)); break;
-      default: {
-        const int64_t e0 = (int64_t)idx * t.chunk;
-        const int64_t e1 = e0 + t.chunk < t.g.M ? e0 + t.chunk : t.g.M;
-        for (int64_t e = e0 + threadIdx.x; e < e1; e += 256) stg<IO>(t.g.C, e, 0.0);
+    auto run = [&](auto c) {
+      using IOC = decltype(c);
+      switch (t.kind) {
+        case kLvPerm: level_perm<IO, IOC>(t, idx); break;
+        case kLvFlat:
+        case kLvSum: level_flat<IO, IOC>(t, idx); break;
+        case kLvReduce: level_reduce<IO, IOC>(t, idx, reinterpret_cast<double*>(smem)); break;
+        default: {
+          const int64_t e0 = (int64_t)idx * t.chunk;
+          const int64_t e1 = e0 + t.chunk < t.g.M ? e0 + t.chunk : t.g.M;
+          for (int64_t e = e0 + threadIdx.x; e < e1; e += 256) stg<IOC>(t.g.C, e, 0.0);
+        }
+      }
+    };
+    if constexpr (sizeof(IO) == 4) {
+      if (t.g.c64) {
+        run(double());
+        return;
       }
     }
+    run(IO());
     return;
   }
   const GemmArgs& g = t.g;
@@ -1033,7 +1043,10 @@ __global__ __launch_bounds__(256) void gemm_f64_reg(GemmArgs g) {
   // lane l, register v of 16x16 block (i, j) holds row 16i + l/16 + 4v and
   // column 16j + l%16: the FP64 MFMA output layout of the tile epilogue
   if (g.nsplit == 1) {
-    store_tile<IO, RM, RN, Mma<double>>(g, wm0, n0, 0, 0, lane, g.alpha, acc);
+    if (sizeof(IO) == 4 && g.c64)
+      store_tile<IO, double, RM, RN, Mma<double>>(g, wm0, n0, 0, 0, lane, g.alpha, acc);
+    else
+      store_tile<IO, IO, RM, RN, Mma<double>>(g, wm0, n0, 0, 0, lane, g.alpha, acc);
     return;
   }
 #pragma unroll

@@ -51,6 +51,9 @@ struct GemmArgs {
   // LDS-tiled kernel: 2 = two 4-wave groups share a 32x32 tile and split its K
   // slabs, 1 = one group
   int ksplit = 1;
+  // C holds FP64 whatever the storage (level launches: the partial
+  // accumulators of an FP32-storage sweep)
+  int c64 = 0;
   // split-K workspace of at least gemm_ws_need doubles
   double* ws = nullptr;
   // optional addend folded into the epilogue: C (+)= alpha A B + dcoef D,
@@ -211,7 +214,7 @@ struct LevelTask {
   int pshift;    // kLvReduce: 2^pshift threads share an element
   int nsrc;
   GemmArgs g;
-  const double* src[kMaxLevelSrc];
+  const double* src[kMaxLevelSrc];   // FP64 in either storage
 };
 struct LevelItem {
   int task, idx;   // task < 0: nothing
@@ -232,7 +235,7 @@ struct AddGroup {
   int64_t start[kMaxAddGroup + 1];   // first element of each member
   int n;
 };
-// io32: the arrays hold floats (FP32-storage sweeps)
+// io32: the arrays hold floats (FP32-storage sweeps); 2: C holds doubles
 hipError_t launch_axpy_group(hipStream_t s, const AddGroup& ag, int io32 = 0);
 // up to kMaxPermGroup permuted adds C_i(perm) (+)= alpha_i A_i(perm) with
 // their own offset tables in one launch (the irrep blocks of one add)

@@ -53,14 +53,17 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce(GemmArgs g, int pshift
         for (int x = 1; x < P; ++x) s += red[threadIdx.x + x];
       __syncthreads();
     }
-    if (in && p == 0) store_c<IO>(g, m, n, s);
+    if (in && p == 0) {
+      if (sizeof(IO) == 4 && g.c64) store_c<IO, double>(g, m, n, s, g.alpha);
+      else store_c<IO>(g, m, n, s, g.alpha);
+    }
   }
 }
 
 // C(perm) (+)= alpha A through int32 offset tables: element (m, n) reads
 // A[rowA[m] + colA[n]] and updates C[rowC[m] + colC[n]].  A block covers
 // 256 >> tn_shift rows x (1 << tn_shift) columns per pass.
-template <typename IO>
+template <typename IO, typename IOC>
 __global__ __launch_bounds__(256) void perm_add(int64_t M, int N, int tn_shift,
                                                 const double* __restrict__ A,
                                                 const int* __restrict__ rowA,
@@ -77,7 +80,7 @@ __global__ __launch_bounds__(256) void perm_add(int64_t M, int N, int tn_shift,
     const int64_t ra = rowA[m], rc = rowC[m];
     for (int n = n0; n < N; n += tn) {
       const double v = alpha * ldg<IO>(A, ra + colA[n]);
-      put_c<IO>(C, rc + colC[n], v, accumulate);
+      put_c<IOC>(C, rc + colC[n], v, accumulate);
     }
   }
 }
@@ -977,11 +980,14 @@ hipError_t launch_perm_add(hipStream_t s, int64_t M, int64_t N, const double* A,
   while ((1 << shift) < N && shift < 8) ++shift;
   const int64_t rows_per_block = 256 >> shift;
   const dim3 grid(grid_for(M, (int)rows_per_block, 8192));
-  if (io32)
-    hipLaunchKernelGGL(perm_add<float>, grid, dim3(256), 0, s, M, (int)N, shift, A, rowA, colA, C, rowC,
+  if (io32 == 2)
+    hipLaunchKernelGGL((perm_add<float, double>), grid, dim3(256), 0, s, M, (int)N, shift, A, rowA, colA, C, rowC,
+                       colC, alpha, accumulate);
+  else if (io32)
+    hipLaunchKernelGGL((perm_add<float, float>), grid, dim3(256), 0, s, M, (int)N, shift, A, rowA, colA, C, rowC,
                        colC, alpha, accumulate);
   else
-    hipLaunchKernelGGL(perm_add<double>, grid, dim3(256), 0, s, M, (int)N, shift, A, rowA, colA, C, rowC,
+    hipLaunchKernelGGL((perm_add<double, double>), grid, dim3(256), 0, s, M, (int)N, shift, A, rowA, colA, C, rowC,
                        colC, alpha, accumulate);
   return hipGetLastError();
 }

@@ -1,0 +1,40 @@
+"""Rounding error of one sweep in precision modes 1 and 2 against the FP64 sweep
+from the same amplitudes.  Each bound is the root mean square difference that
+the sweep had when every product was a launch of its own (grouped and chained
+launches, FP64 exactly in the register-direct products): level launches may not
+compute with less."""
+
+import numpy as np
+import pytest
+
+from ccq_amd import engine as E
+from ccq_amd import synth
+from ccq_amd.inputs import build_integrals
+
+pytestmark = pytest.mark.gpu
+
+
+def _error(method, n, o, mode, block):
+    s = synth.make_system(n, o, 2 * n, 1, sigma=min(0.05, synth.regime_sigma(n, o, 2 * n)))
+    ints = build_integrals(s.h, s.e2int(), 0.0, 0, o, o)
+    eng = E.Engine(0, o, o, n, method, rhf=True)
+    eng.set_ints(ints.f_a, ints.f_b, ints.v_aa, ints.v_ab, ints.v_bb)
+    out = []
+    for m in (0, mode):
+        eng.set_precision(0)
+        eng.guess("mp2")
+        for _ in range(3):
+            eng.update()
+        eng.set_precision(m)
+        eng.update()
+        out.append(eng.debug_read(*block) if block else eng.get_t())
+    eng.close()
+    return float(np.sqrt(np.mean((out[1] - out[0]) ** 2)))
+
+
+@pytest.mark.parametrize("n,o,bound", [(20, 5, 4.550e-11)])
+def test_partial_accumulators_of_fp32_storage(n, o, bound):
+    """Terms that go to a partial accumulator are rounded to FP32 once, with their sum."""
+    print(f"case FP32-storage partial accumulators CCSDT n={n} o={o}", flush=True)
+    err = _error("CCSDT", n, o, 2, None)
+    assert 0.0 < err <= bound
