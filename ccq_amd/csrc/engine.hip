@@ -2532,7 +2532,9 @@ struct ccq_hip_ctx {
     if (op.fused) return;
     const int acc = op.assign ? 0 : 1;
     if (op.gemm) {
-      HIPCHK(ccqk::launch_gemm(stream, gemm_args(op)));
+      ccqk::GemmArgs g = gemm_args(op);
+      if (run_prec && g.kind == 0 && op.K > 0 && ccqk::fp64_in_mixed(op.M, op.N, op.K)) ccqk::gemm_plan_reg(g, ws.n);
+      HIPCHK(ccqk::launch_gemm(stream, g));
     } else {
       if (amp_in_fp64(1, [&](size_t) { return op.out; }, [&] { run_op(op); })) return;
       run_add(op, sp(op.a), sp(op.out), acc);
@@ -2780,10 +2782,10 @@ struct ccq_hip_ctx {
     g.trans = (g.c_mfast && !g.c_nfast) ? 1 : 0;
     double best = 1e300;
     int bm = 32, bn = 32;
-    const bool f64 = op.plan.kind == 1;   // register-direct products are FP64 in every precision mode
+    const bool small = op.plan.kind == 1;
     for (int tm : {64, 32})
       for (int tn : {64, 32}) {
-        if (f64 && (tm != 32 || tn != 32)) continue;
+        if (small && (tm != 32 || tn != 32)) continue;
         const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, tm, tn);
         const double t = c.share + std::max(0.0, c.item - load);
         if (t < best) {
@@ -2977,9 +2979,8 @@ struct ccq_hip_ctx {
           }
           const ccqk::GemmArgs& g = ts.plan;
           const TileCost c = tile_cost(op, g);
-          ts.kind = op.plan.kind == 1 ? ccqk::kLvTileF64
-                                      : g.bm == 64 ? (g.bn == 64 ? ccqk::kLvTile6464 : ccqk::kLvTile6432)
-                                                   : (g.bn == 64 ? ccqk::kLvTile3264 : ccqk::kLvTile3232);
+          ts.kind = (ccqk::fp64_in_mixed(op.M, op.N, op.K) ? ccqk::kLvTileF64 : ccqk::kLvTile6464) +
+                    (g.bm == 64 ? 0 : 2) + (g.bn == 64 ? 0 : 1);
           n = c.tiles * g.nsplit;
           cost = c.item / g.nsplit;
           if (g.nsplit > 1) {

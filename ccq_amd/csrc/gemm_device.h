@@ -867,7 +867,8 @@ __device__ __forceinline__ void level_reduce(const LevelTask& t, int idx, double
 template <typename T, typename IO>
 __global__ __launch_bounds__(256, kTileWaves<1>) void level_kernel(const LevelTask* __restrict__ tasks,
                                                                    const LevelItem* __restrict__ items) {
-  constexpr int b1 = TabLds<T, 64, 64, tile_bk(64, 64), 1>::bytes, b2 = TabLds<double, 32, 32, tile_bk(32, 32), 1>::bytes;
+  // the FP64 tiles are in every arithmetic's kernel; theirs is the largest LDS
+  constexpr int b1 = TabLds<double, 64, 64, tile_bk(64, 64), 1>::bytes, b2 = TabLds<double, 32, 32, tile_bk(32, 32), 1>::bytes;
   __shared__ __align__(16) unsigned char smem[b1 > b2 ? b1 : b2];
   typedef const __attribute__((address_space(4))) LevelTask* ConstTask;
   typedef const __attribute__((address_space(4))) LevelItem* ConstItem;
@@ -905,18 +906,20 @@ __global__ __launch_bounds__(256, kTileWaves<1>) void level_kernel(const LevelTa
   const int tz = idx / per_z;
   int tx, ty;
   tile_in_group(idx - tz * per_z, tm, tn, g.group, tx, ty);
-#define CCQ_LV(A, BM, BN) gemm_tab_tile<A, IO, BM, BN, tile_bk(BM, BN), 1>(g, tx, ty, tz, smem)
-  switch (t.kind) {
-    case kLvTile6464: CCQ_LV(T, 64, 64); break;
-    case kLvTile6432: CCQ_LV(T, 64, 32); break;
-    case kLvTile3264: CCQ_LV(T, 32, 64); break;
-    case kLvTileF64:
-      if constexpr (sizeof(T) == 4) {
-        CCQ_LV(double, 32, 32);
-        break;
-      }
-    default: CCQ_LV(T, 32, 32); break;
+#define CCQ_LV(A)                                                                        \
+  switch ((t.kind - kLvTile6464) & 3) {                                                  \
+    case 0: gemm_tab_tile<A, IO, 64, 64, tile_bk(64, 64), 1>(g, tx, ty, tz, smem); break; \
+    case 1: gemm_tab_tile<A, IO, 64, 32, tile_bk(64, 32), 1>(g, tx, ty, tz, smem); break; \
+    case 2: gemm_tab_tile<A, IO, 32, 64, tile_bk(32, 64), 1>(g, tx, ty, tz, smem); break; \
+    default: gemm_tab_tile<A, IO, 32, 32, tile_bk(32, 32), 1>(g, tx, ty, tz, smem);       \
   }
+  if constexpr (sizeof(T) == 4) {
+    if (t.kind >= kLvTileF64) {
+      CCQ_LV(double)
+      return;
+    }
+  }
+  CCQ_LV(T)
 #undef CCQ_LV
 }
 

@@ -6,6 +6,8 @@
 #include <utility>
 #include <vector>
 
+#include "precision.h"
+
 namespace ccqk {
 
 constexpr int kMaxRank = 8;
@@ -152,6 +154,8 @@ constexpr int tile_bk(int bm, int bn) { return bm * bn > 32 * 32 ? 16 : 32; }
 // Choose kernel, tile shape and split-K for a GEMM; ws_cap bounds the
 // split-K workspace (doubles).
 void gemm_plan(GemmArgs& g, int64_t ws_cap);
+// the same among the register-direct kernel's shapes (a side of at most 64)
+void gemm_plan_reg(GemmArgs& g, int64_t ws_cap);
 // the same, also returning every candidate plan with its modelled cycles,
 // best first (the input for the measuring autotuner)
 void gemm_plan_ranked(GemmArgs& g, int64_t ws_cap, std::vector<std::pair<double, GemmArgs>>* ranked);
@@ -200,8 +204,8 @@ enum LevelKind {
   kLvTile6432,
   kLvTile3264,
   kLvTile3232,
-  kLvTileF64,        // 32 x 32 in FP64 arithmetic whatever the precision mode
-  kLvPerm,           // C(perm) (+)= alpha A(perm): rowA / kA, rowC / colC
+  kLvTileF64,        // kLvTileF64 + tile kind - 1: in FP64 arithmetic whatever the precision mode
+  kLvPerm = kLvTileF64 + 4,           // C(perm) (+)= alpha A(perm): rowA / kA, rowC / colC
   kLvFlat,           // C (+)= alpha A, identical layouts
   kLvReduce,         // split-K completion of a GEMM of the previous level
   kLvSum,            // C += sum of src

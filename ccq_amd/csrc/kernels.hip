@@ -672,6 +672,17 @@ static double splitk_cycles(int64_t M, int64_t N, int64_t split) {
 
 void gemm_plan(GemmArgs& g, int64_t ws_cap) { gemm_plan_ranked(g, ws_cap, nullptr); }
 
+void gemm_plan_reg(GemmArgs& g, int64_t ws_cap) {
+  std::vector<std::pair<double, GemmArgs>> ranked;
+  GemmArgs all = g;
+  gemm_plan_ranked(all, ws_cap, &ranked);
+  for (const auto& c : ranked)
+    if (c.second.kind == 1) {
+      g = c.second;
+      return;
+    }
+}
+
 // The planner's cycle model over every kernel / tile / split-K choice; the
 // best one goes into g, and every candidate with its modelled cycles into
 // ranked when given (the autotuner measures the best few).

@@ -38,3 +38,14 @@ def test_partial_accumulators_of_fp32_storage(n, o, bound):
     print(f"case FP32-storage partial accumulators CCSDT n={n} o={o}", flush=True)
     err = _error("CCSDT", n, o, 2, None)
     assert 0.0 < err <= bound
+
+
+T2AB = ("T2.oovv.abab", (5, 5, 19, 19))
+
+
+@pytest.mark.parametrize("method,n,o,block,bound", [("CCSD", 24, 5, T2AB, 2.080e-10), ("CCSDT", 12, 3, None, 2.048e-11)])
+def test_arithmetic_of_small_products(method, n, o, block, bound):
+    """Small and narrow products are computed in FP64 in the FP32 modes, whatever
+    the planner's cost model or a timing says of them."""
+    print(f"case FP64 products of FP32 sweeps {method} n={n} o={o}", flush=True)
+    assert 0.0 < _error(method, n, o, 1, block) <= bound
