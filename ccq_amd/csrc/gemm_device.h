@@ -305,7 +305,8 @@ struct Mma<float> {
 // FP32-storage sweeps) through int32 row offset tables (rowA, colB) and their
 // summed indices' stride or table (kA, kB), and staged into LDS as T.  T =
 // double runs on v_mfma_f64_16x16x4f64; T = float rounds the operands to FP32
-// and accumulates in FP32 on v_mfma_f32_16x16x4f32 (the mixed-precision form).
+// and multiplies on v_mfma_f32_16x16x4f32 (the mixed-precision form): kF32Run
+// summed indices at a time accumulate in FP32, the runs in FP64.
 // FP64, against one slab of look-ahead with two barriers a slab, predicated
 // loads and single-k fragment reads: 1225 x 4375 x 1225 303 -> 244 us (54 TF/s),
 // 900^3 58.6 -> 42 us, 8100 x 100 x 8100 448 -> 328 us, 4096 x 4096 x 2048
@@ -403,10 +404,20 @@ template <typename T, int BM, int BN, int BK, int KS>
 struct TabLds {
   static constexpr int slab = LdsTile<T, BM, BK>::size + LdsTile<T, BN, BK>::size;
   static constexpr int tile = 2 * KS * slab * (int)sizeof(T);
-  static constexpr int red = (KS - 1) * 256 * (BM / 32) * (BN / 32) * 4 * (int)sizeof(T);
+  static constexpr int red = (KS - 1) * 256 * (BM / 32) * (BN / 32) * 4 * (int)sizeof(double);
   static constexpr int kts = (tile > red ? tile : red);   // offset of the K offsets
   static constexpr int bytes = kts + 2 * kKCache * (int)sizeof(int);
 };
+
+// Summed indices that FP32 products accumulate before they are added to the FP64
+// sums.  The rounding of an FP32 accumulator grows with its length, so a bound of
+// the kernel's own keeps it independent of tiles and K splits, which levels
+// choose longer than a launch per product would.  The FP64 sums take 32 registers
+// in a 64 x 64 tile (some spill in the table modes: FP32-storage sweeps of CCSD 61
+// orbitals 362 -> 375 us, CCSDT 31 1131 -> 1160); two workgroups a CU without
+// spills are slower (428, 1282), sums of runs in FP32 too (394, 1198), and runs
+// of 128 no faster.
+constexpr int kF32Run = 64;
 
 // The K-slab loop of the tile kernel: acc += A(m0.., kbeg..kend) B(kbeg..kend, n0..)
 // (the caller zeroes acc; group grp of KS takes slabs grp, grp + KS, ...).
@@ -417,7 +428,7 @@ struct TabLds {
 // k + 6: the same products, summed in another order).
 template <typename T, typename IO, int BM, int BN, int BK, int KS, KMode MA, KMode MB>
 __device__ __forceinline__ void tile_run(const GemmArgs& g, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
-                                         unsigned char* smem, typename Mma<T>::acc_t (&acc)[BM / 32][BN / 32]) {
+                                         unsigned char* smem, d4 (&acc)[BM / 32][BN / 32]) {
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int TM = WM / 16, TN = WN / 16;
   using FA = Feed<T, IO, BM, BK, MA>;
@@ -435,6 +446,25 @@ __device__ __forceinline__ void tile_run(const GemmArgs& g, int64_t m0, int64_t 
   const T* fa = lds + ((wave & 1) * WM + (lane & 15)) * FA::pitch + 2 * (lane >> 4);
   const T* fb = lds + LdsTile<T, BM, BK>::size + ((wave >> 1) * WN + (lane & 15)) * FB::pitch + 2 * (lane >> 4);
 
+  constexpr bool f32 = sizeof(T) == 4;
+  f4 low[f32 ? TM : 1][f32 ? TN : 1];   // FP32 sums of the current run
+  auto flush = [&] {
+#pragma unroll
+    for (int i = 0; f32 && i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        acc[i][j] += __builtin_convertvector(low[i][j], d4);
+        low[i][j] = f4{0, 0, 0, 0};
+      }
+  };
+  auto fma = [&](T a, T b, int i, int j) {
+    if constexpr (f32) low[i][j] = MM::step(a, b, low[i][j]);
+    else acc[i][j] = MM::step(a, b, acc[i][j]);
+  };
+#pragma unroll
+  for (int i = 0; f32 && i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) low[i][j] = f4{0, 0, 0, 0};
   auto mma = [&](int b) {
 #pragma unroll
     for (int ks = 0; ks < BK; ks += 8) {
@@ -446,11 +476,11 @@ __device__ __forceinline__ void tile_run(const GemmArgs& g, int64_t m0, int64_t 
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = MM::step(af[i].x, bf[j].x, acc[i][j]);
+        for (int j = 0; j < TN; ++j) fma(af[i].x, bf[j].x, i, j);
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = MM::step(af[i].y, bf[j].y, acc[i][j]);
+        for (int j = 0; j < TN; ++j) fma(af[i].y, bf[j].y, i, j);
     }
   };
   const int64_t run = tab ? (int64_t)kKCache : kend - kbeg;
@@ -517,22 +547,29 @@ __device__ __forceinline__ void tile_run(const GemmArgs& g, int64_t m0, int64_t 
     if (nsteps > 1) fetch_any(1, 1);
     stash_any(0, 0);
     if (nsteps > 2) fetch_any(0, 2);
+    // a run's slabs are counted per group; after slab s, s odd
+    auto end_run = [&](int s) {
+      if (f32 && (s + 1) % (kF32Run / BK) == 0) flush();
+    };
     int s = 0;
     for (; s + 4 < nfull / KS; s += 2) {
       step(0, s);
       step(1, s + 1);
+      end_run(s + 1);
     }
     for (; s + 2 <= nsteps; s += 2) {
       step_any(0, s);
       step_any(1, s + 1);
+      end_run(s + 1);
     }
     if (s < nsteps) step_any(0, s);
+    if (f32) flush();
   }
 }
 
 template <typename T, typename IO, int BM, int BN, int BK, int KS>
 __device__ __forceinline__ void tile_mma(const GemmArgs& g, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
-                                         unsigned char* smem, typename Mma<T>::acc_t (&acc)[BM / 32][BN / 32]) {
+                                         unsigned char* smem, d4 (&acc)[BM / 32][BN / 32]) {
   // 0 contiguous, 1 strided, 2 pairs, 3 k-contiguous table, 4 table
   const int ma = g.kA_aff >= 0 ? (g.a_kfast && g.kA_aff == 1 ? 0 : 1) : g.a_kfast ? (g.a_pair ? 2 : 3) : 4;
   const int mb = g.kB_aff >= 0 ? (g.b_kfast && g.kB_aff == 1 ? 0 : 1) : g.b_kfast ? (g.b_pair ? 2 : 3) : 4;
@@ -570,17 +607,17 @@ __device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty,
   const int wm = (wave & 1) * WM;
   const int wn = (wave >> 1) * WN;
 
-  typename MM::acc_t acc[TM][TN];
+  d4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
+    for (int j = 0; j < TN; ++j) acc[i][j] = d4{0, 0, 0, 0};
   tile_mma<T, IO, BM, BN, BK, KS>(g, m0, n0, kbeg, kend, smem, acc);
 
   if (KS > 1) {
     // group 1 hands its accumulators to group 0 (slab order: group 0's sum
     // plus group 1's sum, the same for every launch)
-    T* red = reinterpret_cast<T*>(smem);
+    double* red = reinterpret_cast<double*>(smem);
     __syncthreads();
     if (grp == 1) {
 #pragma unroll
@@ -617,7 +654,7 @@ __device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty,
       for (int v = 0; v < 4; ++v) {
         const int64_t gm = m0 + wm + 16 * i + MM::row(lane, v);
         if (gm >= g.M) continue;
-        store_partial(g, tz, gm, gn, (double)acc[i][j][v]);
+        store_partial(g, tz, gm, gn, acc[i][j][v]);
       }
   }
 }
@@ -663,11 +700,11 @@ __device__ __forceinline__ void tile_entries(const GemmArgs* es, int e0, int e1,
     const int64_t a = lo - off, b = hi - off;
     off += g.K;
     if (a >= b) continue;
-    typename MM::acc_t acc[TM][TN];
+    d4 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = typename MM::acc_t{0, 0, 0, 0};
+      for (int j = 0; j < TN; ++j) acc[i][j] = d4{0, 0, 0, 0};
     // the previous entry's waves are past their last LDS reads
     if (e > e0) __syncthreads();
     tile_mma<T, IO, BM, BN, BK, 1>(g, m0, n0, a, b, smem, acc);
@@ -676,7 +713,7 @@ __device__ __forceinline__ void tile_entries(const GemmArgs* es, int e0, int e1,
 #pragma unroll
       for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sum[i][j][v] += g.alpha * (double)acc[i][j][v];
+        for (int v = 0; v < 4; ++v) sum[i][j][v] += g.alpha * acc[i][j][v];
   }
 
   if (kend < 0 || o.nsplit == 1) {
@@ -906,20 +943,31 @@ __global__ __launch_bounds__(256, kTileWaves<1>) void level_kernel(const LevelTa
   const int tz = idx / per_z;
   int tx, ty;
   tile_in_group(idx - tz * per_z, tm, tn, g.group, tx, ty);
-#define CCQ_LV(A)                                                                        \
-  switch ((t.kind - kLvTile6464) & 3) {                                                  \
-    case 0: gemm_tab_tile<A, IO, 64, 64, tile_bk(64, 64), 1>(g, tx, ty, tz, smem); break; \
-    case 1: gemm_tab_tile<A, IO, 64, 32, tile_bk(64, 32), 1>(g, tx, ty, tz, smem); break; \
-    case 2: gemm_tab_tile<A, IO, 32, 64, tile_bk(32, 64), 1>(g, tx, ty, tz, smem); break; \
-    default: gemm_tab_tile<A, IO, 32, 32, tile_bk(32, 32), 1>(g, tx, ty, tz, smem);       \
-  }
+  const int tile = (t.kind - kLvTile6464) & 3;
+#define CCQ_LV(A, BM, BN, TY) gemm_tab_tile<A, IO, BM, BN, tile_bk(BM, BN), 1>(g, tx, TY, tz, smem)
   if constexpr (sizeof(T) == 4) {
     if (t.kind >= kLvTileF64) {
-      CCQ_LV(double)
+      // a 64 x 64 tile as two of 64 x 32, whose registers fit beside the FP32 forms'
+      if (tile == 0) {
+        CCQ_LV(double, 64, 32, 2 * ty);
+        __syncthreads();
+        CCQ_LV(double, 64, 32, 2 * ty + 1);
+      } else if (tile == 1) {
+        CCQ_LV(double, 64, 32, ty);
+      } else if (tile == 2) {
+        CCQ_LV(double, 32, 64, ty);
+      } else {
+        CCQ_LV(double, 32, 32, ty);
+      }
       return;
     }
   }
-  CCQ_LV(T)
+  switch (tile) {
+    case 0: CCQ_LV(T, 64, 64, ty); break;
+    case 1: CCQ_LV(T, 64, 32, ty); break;
+    case 2: CCQ_LV(T, 32, 64, ty); break;
+    default: CCQ_LV(T, 32, 32, ty); break;
+  }
 #undef CCQ_LV
 }
 

@@ -49,3 +49,10 @@ def test_arithmetic_of_small_products(method, n, o, block, bound):
     the planner's cost model or a timing says of them."""
     print(f"case FP64 products of FP32 sweeps {method} n={n} o={o}", flush=True)
     assert 0.0 < _error(method, n, o, 1, block) <= bound
+
+
+@pytest.mark.parametrize("n,o,bound", [(80, 8, 4.037e-11)])
+def test_length_of_fp32_sums(n, o, bound):
+    """FP32 sums end after a bounded number of summed indices, however few K splits a level takes."""
+    print(f"case FP32 sums CCSD n={n} o={o}", flush=True)
+    assert 0.0 < _error("CCSD", n, o, 1, ("T2.oovv.abab", (o, o, n - o, n - o))) <= bound
