@@ -407,7 +407,10 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step(const float* __restrict
       }
     }
     __syncthreads();
-    for (int s = 0; s < kStepTile; ++s) {
+    // (rows past the batch are left out, not weighted by zero: with infinite
+    // weights they hold NaN)
+    const int ns = batch - s0 < kStepTile ? (int)(batch - s0) : kStepTile;
+    for (int s = 0; s < ns; ++s) {
       const float* r = rows + s * kRow;
       const float4 h = *reinterpret_cast<const float4*>(r + C_H1 + p0);
       const float4 g = *reinterpret_cast<const float4*>(r + C_G2 + q0);
