@@ -2910,7 +2910,9 @@ struct ccq_hip_ctx {
         int64_t split = (int64_t)std::ceil((c.item - 4000.0) / std::max(span - 4000.0, 4000.0));
         split = std::min({split, slabs / 4, (int64_t)256, std::max<int64_t>(1, kSplitMax / (op.M * op.N))});
         if (split < 2) continue;
-        if ((partials[first[u].level] += split * op.M * op.N) > kLevelPartials) continue;
+        int64_t& level_sum = partials[first[u].level];
+        if (level_sum + split * op.M * op.N > kLevelPartials) continue;
+        level_sum += split * op.M * op.N;
         const int64_t per = (slabs + split - 1) / split;
         g.nsplit = (int)((slabs + per - 1) / per);
         g.kchunk = per * g.bk;
@@ -3208,7 +3210,8 @@ struct ccq_hip_ctx {
   // extra level costs
   static constexpr int64_t kSplitDot = 1 << 14;   // outputs whose partials cost nothing
   static constexpr double kSplitSpan = 12000.0, kSplitWide = 80000.0, kSplitGain = 10000.0;
-  // partials of one product and of one level (doubles)
+  // partials of one product and, by the levels of the schedule without splits
+  // (a split moves what follows it), of one level (doubles)
   static constexpr int64_t kSplitMax = 4 << 20, kLevelPartials = 32 << 20;
 
   std::string cur_sec;   // section being run (profile attribution)
