@@ -158,12 +158,16 @@ struct DevBuf {
   double* p = nullptr;
   int64_t n = 0;
   void alloc(int64_t count) {
-    n = count;
+    release();
     if (count > 0) HIPCHK(hipMalloc(&p, sizeof(double) * count));
+    n = count;
   }
-  ~DevBuf() {
+  void release() {
     if (p) (void)hipFree(p);
+    p = nullptr;
+    n = 0;
   }
+  ~DevBuf() { release(); }
 };
 
 // ---------------------------------------------------------------------------
@@ -369,11 +373,7 @@ struct ccq_hip_ctx {
 
   ~ccq_hip_ctx() {
     for (auto& kv : graphs) drop_graph(kv.second);
-    for (auto& kv : level_progs) {
-      if (kv.second.items) (void)hipFree(kv.second.items);
-      for (auto* t : kv.second.tasks)
-        if (t) (void)hipFree(t);
-    }
+    drop_levels();
     for (float* p : f32_bufs) (void)hipFree(p);
     if (guess_params) (void)hipFree(guess_params);
     if (d3tab) (void)hipFree(d3tab);
@@ -1597,6 +1597,51 @@ struct ccq_hip_ctx {
     sections = std::move(out);
   }
 
+  // Storage orders, buffers, plans and schedules of the programs.  After a failure
+  // (out of device memory) the programs are as they were loaded, but for the
+  // storage orders, which the tensors' perm already tells; so a later call starts over.
+  bool ordered = false;
+  void set_up() {
+    if (!ordered) choose_orders();
+    ordered = true;
+    const std::vector<Section> loaded = sections;
+    try {
+      resolve_tensors();
+      plan();
+    } catch (...) {
+      sections = loaded;
+      undo_set_up();
+      throw;
+    }
+  }
+  void undo_set_up() {
+    drop_levels();
+    for (float* p : f32_bufs) (void)hipFree(p);
+    f32_bufs.clear();
+    f32_ready = false;
+    tvec32 = nullptr;
+    for (Tensor& t : tensors) t.p32 = nullptr;
+    for (DevBuf* b : {&ws, &lsq}) b->release();
+    cur_ws = nullptr;
+    auto drop = [](auto*& p) {
+      if (p) (void)hipFree(p);
+      p = nullptr;
+    };
+    drop(tables32);
+    drop(itab);
+    drop(dtab);
+    drop(gather_tab);
+    gathers.clear();
+    view_owner.clear();
+    view_key.clear();
+    view_buf.clear();
+    inter_buf.clear();
+    resid_buf.clear();
+    ws_need = 0;
+    part_count = 0;
+    (void)hipGetLastError();
+  }
+
   void plan() {
     if (merge_sections) merge_compute_sections();
     std::vector<int> host32;
@@ -2741,6 +2786,18 @@ struct ccq_hip_ctx {
   DevBuf lv_ws;
   int64_t lv_ws_need = 0;
   bool use_levels() const { return group; }
+  void drop_levels() {
+    for (auto& kv : level_progs) {
+      if (kv.second.items) (void)hipFree(kv.second.items);
+      for (auto* t : kv.second.tasks)
+        if (t) (void)hipFree(t);
+    }
+    level_progs.clear();
+    slot_off.clear();
+    slot_need = lv_ws_need = 0;
+    slots.release();
+    lv_ws.release();
+  }
 
   int64_t tensor_size(int t) const {
     int64_t n = 1;
@@ -3892,11 +3949,7 @@ int ccq_hip_set_ints(ccq_hip_ctx* ctx, const double* f_a, const double* f_b, con
     HIPCHK(hipMemcpy(ctx->Fb.p, fb.data(), sizeof(double) * nc * nc, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(ctx->fdiag_a.p, da.data(), sizeof(double) * nc, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(ctx->fdiag_b.p, db.data(), sizeof(double) * nc, hipMemcpyHostToDevice));
-    if (!ctx->ints_ready) {
-      ctx->choose_orders();
-      ctx->resolve_tensors();
-      ctx->plan();
-    }
+    if (!ctx->ints_ready) ctx->set_up();
     ctx->gather_views();
     ctx->ints_ready = true;
   });
