@@ -1970,11 +1970,35 @@ struct ccq_hip_ctx {
     if (use_levels()) {
       std::set<std::string> progs;
       for (const auto& sec : sections) progs.insert(sec.prog);
-      for (const auto& prog : progs) build_levels(prog);
+      for (lean = false;; lean = true) {
+        for (const auto& prog : progs) build_levels(prog);
+        if (scratch_fits() || lean) break;
+        drop_levels();
+      }
       lv_ws.alloc(std::max<int64_t>(lv_ws_need, 1));
       slots.alloc(slot_need);
     }
   }
+
+  // Whether the partial accumulators and split-K partials of the level launches
+  // may be allocated: they save time, not memory (CCSDTQ, 14 orbitals: 220 of
+  // 320 MB), so they must not take what the context still needs, the float
+  // shadows of the FP32-storage sweeps, or more than CCQ_HIP_SCRATCH_MB.  Without
+  // them (lean) every term adds to its accumulator in turn and products run
+  // their whole summed range.
+  bool lean = false;
+  int64_t scratch_mb = -1;
+  bool scratch_fits() const {
+    const size_t want = sizeof(double) * (size_t)(lv_ws_need + slot_need);
+    if (scratch_mb >= 0 && want > (size_t)scratch_mb << 20) return false;
+    size_t shadows = sizeof(float) * (size_t)dev_t, free = 0, total = 0;
+    for (const auto* bufs : {&inter_buf, &view_buf})
+      for (const auto& b : *bufs) shadows += sizeof(float) * (size_t)b->n;
+    for (const auto& kv : resid_buf) shadows += sizeof(float) * (size_t)kv.second->n;
+    HIPCHK(hipMemGetInfo(&free, &total));
+    return want + shadows + kKeepFree <= free;
+  }
+  static constexpr size_t kKeepFree = (size_t)256 << 20;   // task tables, kernels' scratch, pinned staging
 
   // Fold an add op (C (+)= c A) into the GEMM that next updates C, when that
   // GEMM accumulates into C, does not read C, and A is not written in
@@ -2925,6 +2949,7 @@ struct ccq_hip_ctx {
     // full is false there, so its slot starts from zeros
     auto schedule = [&](std::vector<ccqlv::Unit>& v) {
       ccqlv::Scheduler sch;
+      if (lean) sch.slot_cap = 1;
       sch.run(v);
       return sch;
     };
@@ -2956,7 +2981,7 @@ struct ccq_hip_ctx {
     for (size_t u = 0; u < units.size(); ++u)
       for (size_t k = 0; k < us[u].ops.size(); ++k) {
         const Op& op = sections[us[u].sec].ops[us[u].ops[k]];
-        if (!op.gemm || own_launch(op) || op.K == 0) continue;
+        if (lean || !op.gemm || own_launch(op) || op.K == 0) continue;
         ccqk::GemmArgs& g = plans[u][k];
         const TileCost c = tile_cost(op, g);
         const double span = op.M * op.N <= kSplitDot ? std::max(load[first[u].level] / 16.0, kSplitSpan)
@@ -3128,6 +3153,9 @@ struct ccq_hip_ctx {
     HIPCHK(hipMalloc(&lp.items, sizeof(ccqk::LevelItem) * std::max<size_t>(items.size(), 1)));
     if (!items.empty())
       HIPCHK(hipMemcpy(lp.items, items.data(), sizeof(ccqk::LevelItem) * items.size(), hipMemcpyHostToDevice));
+    if (dump_schedule)
+      std::fprintf(stderr, "[levels] %s: %zu levels; so far partial accumulators %.1f MB, split partials %.1f MB%s\n", prog.c_str(),
+                   at.size(), slot_need * 8e-6, lv_ws_need * 8e-6, lean ? " (lean)" : "");
     if (dump_schedule)
       for (size_t l = 0; l < at.size(); ++l) {
         double fl = 0, by = 0;
@@ -3856,6 +3884,7 @@ int ccq_hip_create(const ccq_hip_dims* dims, const ccq_hip_opts* opts, ccq_hip_c
     if (const char* g = std::getenv("CCQ_HIP_GROUP_MINK")) ctx->group_min_k = std::max(1, std::atoi(g));
     if (const char* g = std::getenv("CCQ_HIP_GROUP_REG")) ctx->group_reg = std::string(g) != "0";
     if (const char* g = std::getenv("CCQ_HIP_WIDE")) ctx->wide_all = std::string(g) == "1";
+    if (const char* g = std::getenv("CCQ_HIP_SCRATCH_MB")) ctx->scratch_mb = std::max(0, std::atoi(g));
     if (const char* g = std::getenv("CCQ_HIP_MERGE")) ctx->merge_sections = std::string(g) != "0";
     HIPCHK(hipSetDevice(ctx->device));
     HIPCHK(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));

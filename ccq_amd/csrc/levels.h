@@ -58,6 +58,7 @@ class Scheduler {
   std::vector<Sum> sums;
   std::vector<Zero> zeros;
   int levels = 0;
+  int slot_cap = kMaxSlots;   // 1: no partial accumulators
 
   void run(std::vector<Unit>& units) {
     for (Unit& u : units) place(u);
@@ -147,7 +148,7 @@ class Scheduler {
           if (std::max(l, e.free[s]) < at) at = std::max(l, e.free[s]), best = s;
         const int fresh = (int)e.free.size();
         u.overwrite = false;
-        if (fresh < std::min(max_slots(u.size), kMaxSlots)) {
+        if (fresh < std::min(max_slots(u.size), slot_cap)) {
           const Track& st = slot_track_[{out, fresh}];
           const int from = std::max({floor_, st.wr + 1, st.rd + 1});
           const int fl = std::max(l, from + (u.full ? 0 : 1));

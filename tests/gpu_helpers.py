@@ -97,6 +97,16 @@ class Case:
         return osolver.energy(fa, fb, self.vaa, self.vab, self.vbb, self.ca, self.cb, t)
 
 
+def leave_free(nbytes):
+    """Tensors that take the device's memory but for about nbytes (what the driver
+    reports as free is not all there after one large allocation)."""
+    import torch
+    blocks = []
+    while len(blocks) < 8 and torch.cuda.mem_get_info()[0] > nbytes + (32 << 20):
+        blocks.append(torch.empty(torch.cuda.mem_get_info()[0] - nbytes, dtype=torch.uint8, device="cuda"))
+    return blocks
+
+
 def ccsdtq_sweep_case():
     """Inputs of the stored CCSDTQ sweep fixture (golden/make_ccsdtq_sweep.py):
     8 orbitals, 4 alpha / 3 beta occupied, random antisymmetric T1-T4."""

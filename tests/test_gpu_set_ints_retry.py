@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from ccq_amd import engine as E
-from gpu_helpers import Case
+from gpu_helpers import Case, leave_free
 
 pytestmark = pytest.mark.gpu
 
@@ -20,8 +20,7 @@ def test_set_ints_after_out_of_memory():
 
     eng = engine()
     # set_ints needs about 1 GB here; a quarter of it is left
-    free = torch.cuda.mem_get_info()[0]
-    block = torch.empty(free - (256 << 20), dtype=torch.uint8, device="cuda")
+    block = leave_free(256 << 20)
     with pytest.raises(E.EngineError, match="memory"):
         eng.set_ints(c.fa, c.fb, c.vaa, c.vab, c.vbb)
     del block
