@@ -29,9 +29,10 @@ Protocol (per workload)
      only FP64 sweeps count as converged;
   6. value = the mixed+learned leg's wall time until the first FP64
      iteration with |E - E_conv| < 1e-7.
-  Roofline: the contraction class with the largest share of one profiled
-  FP64 sweep (HIP events on the engine's stream): 2*M*N*K flops per launch
-  over its average launch time.  traffic: HBM bytes per launch of that class
+  Roofline: the launch with the largest share of one FP64 sweep's contraction
+  time, of the launches the timed sweeps make (a level launch, or a product
+  with a launch of its own; HIP events on the engine's stream): the 2*M*N*K
+  flops of its products over its time.  traffic: HBM bytes of that launch
   from the rocprofv3 FETCH_SIZE / WRITE_SIZE summaries under profiles/
   (copy-calibrated), when one is recorded for it.
   cpu_baseline: the CPU oracle (numpy / OpenBLAS on the host cores) on the
@@ -301,15 +302,13 @@ def measure(name, steps, warmup, rhf, with_cpu, profile=True):
                guess=guess_kind)
     if profile:
         eng.set_t(t_conv)
-        # the profiled sweep's own launches are not the timed sweep's: the first
-        # one loads their code
-        eng.profile(True)
+        eng.profile(2)
         eng.update()
-        eng.profile(True)
+        eng.profile(2)
         eng.update()
         rep = eng.profile_report()
-        eng.profile(False)
-        gemms = {k: v for k, v in rep.items() if k.startswith("gemm:")}
+        eng.profile(0)
+        gemms = {k: v for k, v in rep.items() if k.startswith(("gemm:", "level:"))}
         dom_name, d = max(gemms.items(), key=lambda kv: kv[1]["ms"])
         avg_s = d["ms"] / d["calls"] * 1e-3
         fl_per = d["flops"] / d["calls"]
@@ -317,7 +316,7 @@ def measure(name, steps, warmup, rhf, with_cpu, profile=True):
         gemm_ms = sum(v["ms"] for v in gemms.values())
         gemm_fl = sum(v["flops"] for v in gemms.values())
         log(f"{name}: dominant {dom_name}: {d['calls']} launches, avg {avg_s * 1e6:.1f} us, "
-            f"{fl_per / avg_s / 1e12:.2f} TF/s; all GEMMs {gemm_fl / 1e9:.1f} GF in "
+            f"{fl_per / avg_s / 1e12:.2f} TF/s; all products and adds {gemm_fl / 1e9:.1f} GF in "
             f"{gemm_ms:.2f} ms ({gemm_fl / (gemm_ms * 1e-3) / 1e12:.2f} TF/s); profiled sweep "
             f"{sweep_ms:.2f} ms")
         for k, v in sorted(rep.items(), key=lambda kv: -kv[1]["ms"])[:24]:

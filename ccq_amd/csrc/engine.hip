@@ -366,7 +366,8 @@ struct ccq_hip_ctx {
   struct Had { int out; const double* X; const double* Y; int64_t M, K, xr, xk, yr, yk; double scale; };
   std::vector<Had> hads;
   // profiling
-  bool profile = false;
+  int profile = 0;   // ccq_hip_profile: 1 per operation, 2 the sweep's own launches
+  hipEvent_t prof_ev[2] = {};
   std::map<std::string, ProfEntry> prof;
   PinnedVec host_partial;
   Download down;
@@ -374,6 +375,8 @@ struct ccq_hip_ctx {
   ~ccq_hip_ctx() {
     for (auto& kv : graphs) drop_graph(kv.second);
     drop_levels();
+    for (hipEvent_t e : prof_ev)
+      if (e) (void)hipEventDestroy(e);
     for (float* p : f32_bufs) (void)hipFree(p);
     if (guess_params) (void)hipFree(guess_params);
     if (d3tab) (void)hipFree(d3tab);
@@ -2732,7 +2735,7 @@ struct ccq_hip_ctx {
 
   void run_graphed(const std::string& prog, double key = 0.0) {
     if (prog == "sweep" && prec == 2) prep_sweep32();
-    if (use_levels() && !profile) prep_levels(prog);
+    if (runs_levels()) prep_levels(prog);
     if (!use_graph || profile) {
       run_program(prog);
       return;
@@ -2761,7 +2764,7 @@ struct ccq_hip_ctx {
 
   void sweep(int64_t nsec = -1) {
     if (prec == 2) prep_sweep32();
-    if (use_levels() && !profile && nsec < 0) prep_levels("sweep");
+    if (runs_levels(nsec)) prep_levels("sweep");
     run_program("sweep", nsec);
   }
 
@@ -2774,12 +2777,16 @@ struct ccq_hip_ctx {
   // One stream, so the captured graph is a chain: a graph with parallel
   // branches costs about 4 us of host time a node when it is launched (CCSD 24
   // orbitals: 870 us for 176 nodes, as long as the sweep itself), a chain 0.4.
-  // Profiling and CCQ_HIP_GROUP=0 run the sections' own launches.
+  // Profile 1 and CCQ_HIP_GROUP=0 run the sections' own launches.
   struct LevelStep {
     std::vector<std::pair<int, int>> own;   // (section, op or -1: the whole section)
     std::vector<int> own_task;              // for an op: its task (arguments), else -1
     int64_t item0 = 0;
     int nitems = 0;
+    // the level launch in a profile: "level:<program>:<level>:<operations>ops:" and
+    // the M x N x K of its largest product
+    std::string cls;
+    double flops = 0, bytes = 0;
   };
   // what a task is built from, for either storage
   struct TaskSrc {
@@ -2810,6 +2817,7 @@ struct ccq_hip_ctx {
   DevBuf lv_ws;
   int64_t lv_ws_need = 0;
   bool use_levels() const { return group; }
+  bool runs_levels(int64_t nsec = -1) const { return use_levels() && profile != 1 && nsec < 0; }
   void drop_levels() {
     for (auto& kv : level_progs) {
       if (kv.second.items) (void)hipFree(kv.second.items);
@@ -3156,17 +3164,26 @@ struct ccq_hip_ctx {
     if (dump_schedule)
       std::fprintf(stderr, "[levels] %s: %zu levels; so far partial accumulators %.1f MB, split partials %.1f MB%s\n", prog.c_str(),
                    at.size(), slot_need * 8e-6, lv_ws_need * 8e-6, lean ? " (lean)" : "");
+    for (size_t l = 0; l < at.size(); ++l) {
+      LevelStep& step = lp.steps[l];
+      const Op* top = nullptr;
+      int nops = 0;
+      for (const Pending& p : at[l]) {
+        const TaskSrc& ts = lp.src[p.task];
+        if (ts.op < 0 || ts.kind == ccqk::kLvReduce) continue;
+        const Op& op = sections[ts.sec].ops[ts.op];
+        ++nops;
+        step.flops += op.flops;
+        step.bytes += op.bytes;
+        if (op.gemm && (!top || op.flops > top->flops)) top = &op;
+      }
+      step.cls = "level:" + prog + ":" + std::to_string(l) + ":" + std::to_string(nops) + "ops";
+      if (top) step.cls += ":" + std::to_string(top->M) + "x" + std::to_string(top->N) + "x" + std::to_string(top->K);
+    }
     if (dump_schedule)
       for (size_t l = 0; l < at.size(); ++l) {
-        double fl = 0, by = 0;
-        for (const Pending& p : at[l]) {
-          const TaskSrc& ts = lp.src[p.task];
-          if (ts.op < 0 || ts.kind == ccqk::kLvReduce) continue;
-          fl += sections[ts.sec].ops[ts.op].flops;
-          by += sections[ts.sec].ops[ts.op].bytes;
-        }
         std::fprintf(stderr, "[levels] %s level %zu: %d items, %zu own launches, %.2f GF, %.1f MB\n", prog.c_str(), l,
-                     lp.steps[l].nitems, lp.steps[l].own.size(), fl * 1e-9, by * 1e-6);
+                     lp.steps[l].nitems, lp.steps[l].own.size(), lp.steps[l].flops * 1e-9, lp.steps[l].bytes * 1e-6);
         for (const Pending& p : at[l]) {
           const TaskSrc& ts = lp.src[p.task];
           std::string form;   // how the operands' summed indices lie: v contiguous, a strided, p pairs, t table
@@ -3269,26 +3286,34 @@ struct ccq_hip_ctx {
         const int oi = step.own[k].second;
         cur_sec = sec.name;
         if (oi < 0) {
-          if (sec.kind == Section::Update) run_update(sec.upd);
-          else if (sec.kind == Section::Copy) run_copy(sec.dst, sec.src);
-          else run_cct3(sec.upd);
+          if (sec.kind == Section::Update)
+            timed("update:" + sec.upd.block, 0, 8.0 * 3 * (double)tensor_size(sec.upd.resid), [&] { run_update(sec.upd); });
+          else if (sec.kind == Section::Copy)
+            timed("copy:" + sec.dst, 0, 8.0 * 2 * (double)blk_size.at(sec.dst), [&] { run_copy(sec.dst, sec.src); });
+          else
+            timed("cct3:" + sec.upd.block, 0, 0, [&] { run_cct3(sec.upd); });
           continue;
         }
         const Op& op = sec.ops[oi];
-        if (step.own_task[k] < 0) {
-          run_op(op);
-          continue;
-        }
-        ccqk::GemmArgs g = lp.host[st][step.own_task[k]].g;
-        if (op.gemm) {
-          g.prec = run_prec;
-          g.ws = cur_ws;
-          HIPCHK(ccqk::launch_gemm(stream, g));
-        } else {
-          run_add(op, g.A, g.C, g.accumulate, g.c64);
-        }
+        timed(op.cls, op.flops, op.bytes, [&] {
+          if (step.own_task[k] < 0) {
+            run_op(op);
+            return;
+          }
+          ccqk::GemmArgs g = lp.host[st][step.own_task[k]].g;
+          if (op.gemm) {
+            g.prec = run_prec;
+            g.ws = cur_ws;
+            HIPCHK(ccqk::launch_gemm(stream, g));
+          } else {
+            run_add(op, g.A, g.C, g.accumulate, g.c64);
+          }
+        });
       }
-      HIPCHK(ccqk::launch_level(stream, run_prec, lp.tasks[st], lp.items + step.item0, step.nitems));
+      if (!step.nitems) continue;
+      cur_sec = "levels:" + prog;
+      timed(step.cls, step.flops, step.bytes,
+            [&] { HIPCHK(ccqk::launch_level(stream, run_prec, lp.tasks[st], lp.items + step.item0, step.nitems)); });
     }
   }
   // a single workgroup's cycles below which splitting never pays, and what the
@@ -3301,42 +3326,39 @@ struct ccq_hip_ctx {
 
   std::string cur_sec;   // section being run (profile attribution)
 
-  void run_program(const std::string& prog, int64_t nsec = -1) {
-    if (!ints_ready) throw Fail("integrals not uploaded");
-    run_prec = prog == "sweep" ? prec : std::min(prec, 1);
-    if (run_prec == 2 && (!f32_ready || views32_stale)) throw Fail("FP32 shadows not prepared");
-    if (use_levels() && !profile && nsec < 0) {
-      run_levels(prog);
+  // fn's launches, timed as class cls and summed per section
+  // ("section:<name>") while profiling
+  template <typename F>
+  void timed(const std::string& cls, double fl, double by, F&& fn) {
+    if (!profile) {
+      fn();
       return;
     }
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (profile) {
-      HIPCHK(hipEventCreate(&e0));
-      HIPCHK(hipEventCreate(&e1));
-    }
-    auto timed = [&](const std::string& cls, double fl, double by, auto&& fn) {
-      if (!profile) {
-        fn();
-        return;
-      }
-      HIPCHK(hipEventRecord(e0, stream));
-      fn();
-      HIPCHK(hipEventRecord(e1, stream));
-      HIPCHK(hipEventSynchronize(e1));
-      float ms = 0;
-      HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-      auto& p = prof[cls];
+    for (hipEvent_t& e : prof_ev)
+      if (!e) HIPCHK(hipEventCreate(&e));
+    HIPCHK(hipEventRecord(prof_ev[0], stream));
+    fn();
+    HIPCHK(hipEventRecord(prof_ev[1], stream));
+    HIPCHK(hipEventSynchronize(prof_ev[1]));
+    float ms = 0;
+    HIPCHK(hipEventElapsedTime(&ms, prof_ev[0], prof_ev[1]));
+    for (const std::string& name : {cls, "section:" + cur_sec}) {
+      auto& p = prof[name];
       p.calls++;
       p.ms += ms;
       p.flops += fl;
       p.bytes += by;
-      // the same launch, summed per section (reported as "section:<name>")
-      auto& q = prof["section:" + cur_sec];
-      q.calls++;
-      q.ms += ms;
-      q.flops += fl;
-      q.bytes += by;
-    };
+    }
+  }
+
+  void run_program(const std::string& prog, int64_t nsec = -1) {
+    if (!ints_ready) throw Fail("integrals not uploaded");
+    run_prec = prog == "sweep" ? prec : std::min(prec, 1);
+    if (run_prec == 2 && (!f32_ready || views32_stale)) throw Fail("FP32 shadows not prepared");
+    if (runs_levels(nsec)) {
+      run_levels(prog);
+      return;
+    }
     int64_t isec = 0;
     for (auto& sec : sections) {
       if (sec.prog != prog) continue;
@@ -3382,10 +3404,6 @@ struct ccq_hip_ctx {
       } else {
         run_copy(sec.dst, sec.src);
       }
-    }
-    if (profile) {
-      (void)hipEventDestroy(e0);
-      (void)hipEventDestroy(e1);
     }
   }
 
@@ -3467,7 +3485,7 @@ struct ccq_hip_ctx {
   // hbar2 + add_twobody_hbar (src/hbar.f90:10-720) from the current T1, T2
   void hbar() {
     if (!tail) throw Fail("H-bar needs the CC(t;3) program (level 6)");
-    if (use_levels() && !profile) prep_levels("hbar");
+    if (runs_levels()) prep_levels("hbar");
     run_program("hbar");
     auto diag = [&](const char* src, int64_t n, double* dst) {
       HIPCHK(ccqk::launch_diag(stream, tens(src).ptr, n, n, dst));
@@ -3663,7 +3681,7 @@ struct ccq_hip_ctx {
       HIPCHK(ccqk::launch_hadamard_sum(stream, h.M, h.K, h.X, d3tab + h.xr, d3tab + h.xk, h.Y,
                                        d3tab + h.yr, d3tab + h.yk, tensors[h.out].ptr, h.scale));
     HIPCHK(hipMemsetAsync(cpart.p, 0, sizeof(double) * cpart.n, stream));
-    if (use_levels() && !profile) prep_levels("cct3");
+    if (runs_levels()) prep_levels("cct3");
     run_program("cct3");
     host_partial.resize((size_t)cpart.n);
     HIPCHK(hipMemcpyAsync(host_partial.data(), cpart.p, sizeof(double) * cpart.n,
@@ -4275,7 +4293,7 @@ int ccq_hip_set_precision(ccq_hip_ctx* ctx, int64_t mode) {
 
 int ccq_hip_profile(ccq_hip_ctx* ctx, int64_t enable) {
   return guarded(ctx, [&] {
-    ctx->profile = enable != 0;
+    ctx->profile = enable == 2 ? 2 : enable != 0;
     ctx->prof.clear();
   }, true);
 }
@@ -4283,6 +4301,7 @@ int ccq_hip_profile(ccq_hip_ctx* ctx, int64_t enable) {
 int ccq_hip_profile_report(ccq_hip_ctx* ctx, char* buf, int64_t buflen) {
   return guarded(ctx, [&] {
     std::ostringstream os;
+    os.precision(15);
     for (auto& kv : ctx->prof)
       os << kv.first << " " << kv.second.calls << " " << kv.second.ms << " " << kv.second.flops
          << " " << kv.second.bytes << "\n";

@@ -268,7 +268,9 @@ class Engine:
         self._check(self.lib.ccq_hip_cct3(self.h, e), "cct3")
         return tuple(e)
 
-    def profile(self, enable: bool):
+    def profile(self, enable):
+        """False / 0 off; True / 1 times sweeps run operation by operation; 2 times
+        the launches that an untimed sweep makes (one class per level launch)."""
         self._check(self.lib.ccq_hip_profile(self.h, int(enable)), "profile")
 
     def set_irreps(self, irreps):

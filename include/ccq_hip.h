@@ -233,8 +233,12 @@ const char* ccq_hip_mlp_last_error(void);
  * before it stops.  No counterpart in ccq (FP64 only). */
 int ccq_hip_set_precision(ccq_hip_ctx* ctx, int64_t mode);
 
-/* Optional per-operation timing with HIP events on the context's stream.
- * ccq has no counterpart (it prints only wall time per iteration). */
+/* Optional timing with HIP events on the context's stream (0 off).  1: later
+ * sweeps run and time the operations section by section, in launches of their
+ * own, grouped or chained; an untimed sweep does not make these launches.  2:
+ * the launches of an untimed sweep, one class per level launch ("level:...")
+ * and per operation with a launch of its own.  ccq has no counterpart (it
+ * prints only wall time per iteration). */
 int ccq_hip_profile(ccq_hip_ctx* ctx, int64_t enable);
 /* Writes one line per op class: "<name> <calls> <total_ms> <flops> <bytes>". */
 int ccq_hip_profile_report(ccq_hip_ctx* ctx, char* buf, int64_t buflen);
