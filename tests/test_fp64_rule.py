@@ -10,8 +10,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 # computed in FP64 when each was a launch of its own, and the largest ones of
 # each kind in a search over sides of 1 to 60000 and K of 1 to 30000
 FP64 = [(20412, 7, 54), (49, 49, 2916), (54, 54, 2646), (7, 54, 2646), (35, 5, 2975), (5, 5, 2975), (2435, 53, 279),
-        (4225, 28, 247), (2530, 45, 287), (2339, 61, 216), (12, 60000, 10000), (64, 60000, 64), (1, 1, 1)]
-FP32 = [(900, 900, 900), (8100, 100, 8100), (64, 4375, 1225), (65, 65, 8)]
+        (4225, 28, 247), (2530, 45, 287), (2339, 61, 216), (12, 60000, 10000), (64, 60000, 20), (32, 3000000, 29), (1, 1, 1)]
+FP32 = [(900, 900, 900), (8100, 100, 8100), (64, 4375, 1225), (65, 65, 8), (35, 153125, 35)]
 
 
 def test_rule(tmp_path):
