@@ -2871,10 +2871,8 @@ struct ccq_hip_ctx {
     g.trans = (g.c_mfast && !g.c_nfast) ? 1 : 0;
     double best = 1e300;
     int bm = 32, bn = 32;
-    const bool small = op.plan.kind == 1;
     for (int tm : {64, 32})
       for (int tn : {64, 32}) {
-        if (small && (tm != 32 || tn != 32)) continue;
         const TileCost c = tile_cost(g.trans ? op.N : op.M, g.trans ? op.M : op.N, op.K, tm, tn);
         const double t = c.share + std::max(0.0, c.item - load);
         if (t < best) {
