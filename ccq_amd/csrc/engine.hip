@@ -322,6 +322,7 @@ struct ccq_hip_ctx {
   std::map<std::string, std::unique_ptr<DevBuf>> resid_buf;
   std::vector<std::unique_ptr<DevBuf>> inter_buf;
   int* tables32 = nullptr;   // offset tables of every op
+  size_t tables32_n = 0;
   int64_t* gather_tab = nullptr;
   std::vector<std::unique_ptr<DevBuf>> view_buf;
   struct Gather { int t; int64_t rows, cols, t_src_row, t_src_col, t_dst_row, t_dst_col; };
@@ -1624,7 +1625,8 @@ struct ccq_hip_ctx {
     f32_ready = false;
     tvec32 = nullptr;
     for (Tensor& t : tensors) t.p32 = nullptr;
-    for (DevBuf* b : {&ws, &lsq}) b->release();
+    for (DevBuf* b : {&ws, &lsq, &ws_sections}) b->release();
+    sections_planned = false;
     cur_ws = nullptr;
     auto drop = [](auto*& p) {
       if (p) (void)hipFree(p);
@@ -1951,17 +1953,17 @@ struct ccq_hip_ctx {
           }
     }
     fuse_adds(push32);
-    // groups first; products left alone are chained where they can be
-    group_gemms(false);
-    chain_gemms(host32);
-    for (auto& sec : sections) {
-      sec.launches.clear();
-      sec.launch_cls.clear();
+    if (use_levels()) {
+      int64_t own = 1;
+      for (const auto& sec : sections)
+        for (const auto& op : sec.ops)
+          if (op.gemm && own_launch(op))
+            own = std::max({own, ccqk::gemm_ws_need(op.plan), op.has_plan32 ? ccqk::gemm_ws_need(op.plan32) : 0});
+      ws.alloc(own);
+      cur_ws = ws.p;
     }
-    group_gemms(dump_schedule);
-    ws.alloc(std::max<int64_t>(ws_need, 1));
-    cur_ws = ws.p;
     if (lsq_n) lsq.alloc(lsq_n);
+    tables32_n = host32.size();
     HIPCHK(hipMalloc(&tables32, sizeof(int) * std::max<size_t>(host32.size(), 1)));
     if (!host32.empty())
       HIPCHK(hipMemcpy(tables32, host32.data(), sizeof(int) * host32.size(), hipMemcpyHostToDevice));
@@ -1981,6 +1983,42 @@ struct ccq_hip_ctx {
       lv_ws.alloc(std::max<int64_t>(lv_ws_need, 1));
       slots.alloc(slot_need);
     }
+    if (!use_levels() || dump_schedule) plan_sections();
+  }
+
+  // The sections' own launches: grouped and chained products and adds, or with
+  // CCQ_HIP_GROUP=0 one launch per operation.  Level launches need none of it, so
+  // with them it is made when a profile 1 or a partial sweep first asks for it
+  // (set_ints of CC(t;3) 36 orbitals with irreps 363 -> 314 ms, CCSDT 13 8.5 -> 7.5).
+  DevBuf ws_sections;          // their split-K workspace
+  bool sections_planned = false;
+  void plan_sections() {
+    if (sections_planned) return;
+    std::vector<int> tables(tables32_n);
+    if (tables32_n) HIPCHK(hipMemcpy(tables.data(), tables32, sizeof(int) * tables32_n, hipMemcpyDeviceToHost));
+    auto clear = [&] {
+      for (auto& sec : sections) {
+        sec.launches.clear();
+        sec.launch_cls.clear();
+      }
+    };
+    for (auto& sec : sections) {
+      sec.chains.clear();
+      sec.chain_flip.clear();
+      sec.chain_plan.clear();
+      for (Op& op : sec.ops) {
+        op.chain = -1;
+        op.chain_head = false;
+      }
+    }
+    clear();
+    // groups first; products left alone are chained where they can be
+    group_gemms(false);
+    chain_gemms(tables);
+    clear();
+    group_gemms(dump_schedule);
+    ws_sections.alloc(std::max<int64_t>(ws_need, 1));
+    sections_planned = true;
   }
 
   // Whether the partial accumulators and split-K partials of the level launches
@@ -2605,7 +2643,7 @@ struct ccq_hip_ctx {
     const int acc = op.assign ? 0 : 1;
     if (op.gemm) {
       ccqk::GemmArgs g = gemm_args(op);
-      if (run_prec && g.kind == 0 && op.K > 0 && ccqk::fp64_in_mixed(op.M, op.N, op.K)) ccqk::gemm_plan_reg(g, ws.n);
+      if (run_prec && g.kind == 0 && op.K > 0 && ccqk::fp64_in_mixed(op.M, op.N, op.K)) ccqk::gemm_plan_reg(g, ws_sections.n);
       HIPCHK(ccqk::launch_gemm(stream, g));
     } else {
       if (amp_in_fp64(1, [&](size_t) { return op.out; }, [&] { run_op(op); })) return;
@@ -3357,6 +3395,14 @@ struct ccq_hip_ctx {
       run_levels(prog);
       return;
     }
+    // (with level launches this is a profile or a partial sweep, never captured)
+    plan_sections();
+    struct Workspace {
+      double*& p;
+      double* keep;
+      ~Workspace() { p = keep; }
+    } restore{cur_ws, cur_ws};
+    cur_ws = ws_sections.p;
     int64_t isec = 0;
     for (auto& sec : sections) {
       if (sec.prog != prog) continue;
