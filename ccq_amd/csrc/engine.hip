@@ -1432,14 +1432,14 @@ struct ccq_hip_ctx {
     return t + "s" + std::to_string(g.nsplit);
   }
 
-  // Measuring autotuner.  For every product launched on its own, the
-  // planner's kTuneCandidates best plans by modelled cycles are each run, in
-  // two rounds, once to warm up and kTuneReps times timed with HIP events on
-  // the context's stream (before the first sweep: products only write
-  // intermediates and residual accumulators, which every sweep recomputes),
-  // and the fastest by its better round is kept.  Results are shared by every product with the
-  // same shape and operand layouts for the life of the process, so every
-  // context of a process makes the same choices.
+  // Measuring autotuner.  For every product that may have a launch of its own (with
+  // CCQ_HIP_GROUP=0: every product), the planner's kTuneCandidates best plans by
+  // modelled cycles are each run, in two rounds, once to warm up and kTuneReps
+  // times timed with HIP events on the context's stream (before the first sweep:
+  // products only write intermediates and residual accumulators, which every
+  // sweep recomputes), and the fastest by its better round is kept.  Results are
+  // shared by every product with the same shape and operand layouts for the life
+  // of the process, so every context of a process makes the same choices.
   static constexpr int kTuneCandidates = 6;
   static constexpr int kTuneReps = 3;
 
@@ -1503,7 +1503,9 @@ struct ccq_hip_ctx {
       for (auto& sec : sections) {
         if (sec.kind != Section::Compute || (prec == 2 && sec.prog != "sweep")) continue;
         for (auto& op : sec.ops) {
-          if (!op.gemm || op.has_gplan || op.K == 0) continue;
+          // level launches plan their tiles by level: there only a product that may
+          // have a launch of its own has a plan to choose
+          if (!op.gemm || op.has_gplan || op.K == 0 || (use_levels() && !streams(op))) continue;
           const std::string key = (prec == 2 ? "p2:" : "") + tune_key(op);
           if (prec == 2) {
             op.plan32 = op.plan;
@@ -1524,6 +1526,8 @@ struct ccq_hip_ctx {
           std::vector<ccqk::GemmArgs> cands;
           for (auto& rc : ranked) {
             const ccqk::GemmArgs& c = rc.second;
+            // a timing does not choose the arithmetic of the FP32 modes
+            if (c.kind == 1 && op.plan.kind == 0 && !ccqk::fp64_in_mixed(op.M, op.N, op.K)) continue;
             bool dup = false;
             for (auto& d : cands)
               dup = dup || (d.kind == c.kind && d.trans == c.trans && d.bm == c.bm && d.bn == c.bn &&
@@ -2929,10 +2933,11 @@ struct ccq_hip_ctx {
   // operations that keep their own launch
   bool own_launch(const Op& op) const {
     if (!op.gemm) return tensors[op.out].kind == TKind::Amp || (op.M * op.N >= kOwnAdd && op.part_of < 0);
-    // a short summed range and one long side: store bound, and the
-    // register-direct kernel streams it (5 x 1071875 x 5: 2.2 TB/s)
-    return op.plan.kind == 1 && op.K <= 64 && op.M * op.N >= kOwnStream;
+    return op.plan.kind == 1 && streams(op);
   }
+  // a product with a short summed range and a large output: store bound, and the
+  // register-direct kernel, where it applies, streams it (5 x 1071875 x 5: 2.2 TB/s)
+  static bool streams(const Op& op) { return op.K <= 64 && op.M * op.N >= kOwnStream; }
   static constexpr int64_t kOwnAdd = 1 << 21, kOwnStream = 1 << 19;
 
   void build_levels(const std::string& prog) {
