@@ -930,6 +930,12 @@ struct ccq_hip_ctx {
       }
       if (!changed) break;
     }
+    if (dump_schedule)
+      for (const Tensor& t : tensors) {
+        std::string p;
+        for (int i = 0; i < t.rank; ++i) p += (char)('0' + t.perm[i]);
+        if (!std::is_sorted(p.begin(), p.end())) std::fprintf(stderr, "[orders] %s %s\n", t.id.c_str(), p.c_str());
+      }
   }
   // tensors whose products take less chip time than this (s) keep their order:
   // their levels last as long as their latencies do
