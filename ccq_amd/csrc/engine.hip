@@ -2774,6 +2774,12 @@ struct ccq_hip_ctx {
     G.g = nullptr;
   }
 
+  // before anything that reads the integrals or is laid out with them (the float
+  // shadows, the level tables)
+  void need_ints() const {
+    if (!ints_ready) throw Fail("integrals not uploaded");
+  }
+
   // float shadows ready, and the float copy of t_vec refreshed unless it
   // was still valid at this call (cast on the stream, outside any graph)
   void prep_sweep32() {
@@ -2782,6 +2788,7 @@ struct ccq_hip_ctx {
   }
 
   void run_graphed(const std::string& prog, double key = 0.0) {
+    need_ints();
     if (prog == "sweep" && prec == 2) prep_sweep32();
     if (runs_levels()) prep_levels(prog);
     if (!use_graph || profile) {
@@ -2811,6 +2818,7 @@ struct ccq_hip_ctx {
   void run_sweep() { run_graphed("sweep"); }
 
   void sweep(int64_t nsec = -1) {
+    need_ints();
     if (prec == 2) prep_sweep32();
     if (runs_levels(nsec)) prep_levels("sweep");
     run_program("sweep", nsec);
@@ -3399,7 +3407,7 @@ struct ccq_hip_ctx {
   }
 
   void run_program(const std::string& prog, int64_t nsec = -1) {
-    if (!ints_ready) throw Fail("integrals not uploaded");
+    need_ints();
     run_prec = prog == "sweep" ? prec : std::min(prec, 1);
     if (run_prec == 2 && (!f32_ready || views32_stale)) throw Fail("FP32 shadows not prepared");
     if (runs_levels(nsec)) {
@@ -3487,6 +3495,7 @@ struct ccq_hip_ctx {
   }
 
   double energy() {
+    need_ints();
     // src/energy.f90:138-270, same eight pieces
     double* t1a = tvec.p + blk_off["t1a"];
     double* t1b = tvec.p + blk_off["t1b"];
@@ -3540,6 +3549,7 @@ struct ccq_hip_ctx {
   // hbar2 + add_twobody_hbar (src/hbar.f90:10-720) from the current T1, T2
   void hbar() {
     if (!tail) throw Fail("H-bar needs the CC(t;3) program (level 6)");
+    need_ints();
     if (runs_levels()) prep_levels("hbar");
     run_program("hbar");
     auto diag = [&](const char* src, int64_t n, double* dst) {
@@ -3784,7 +3794,7 @@ struct ccq_hip_ctx {
 
   // mode 0: T = 0; 1: T2 = MP2 amplitudes; 2: T2 = MP2 (1 + MLP); T1, T3, T4 = 0
   void guess(int64_t mode, const float* params, int64_t nparams) {
-    if (!ints_ready) throw Fail("integrals not uploaded");
+    need_ints();
     if (mode < 0 || mode > 2) throw Fail("guess mode must be 0 (zero), 1 (MP2) or 2 (learned)");
     if (mode == 2 && (!params || nparams != ccqk::kGuessParams))
       throw Fail("learned guess needs " + std::to_string(ccqk::kGuessParams) + " parameters");
@@ -3807,7 +3817,7 @@ struct ccq_hip_ctx {
 
   // features / targets of every T2 tuple at the current amplitudes
   void guess_data(float* X, float* M, float* Y, int64_t n) {
-    if (!ints_ready) throw Fail("integrals not uploaded");
+    need_ints();
     if (n != guess_data_size()) throw Fail("guess data size mismatch");
     float *dX = nullptr, *dM = nullptr, *dY = nullptr;
     auto release = [&] {
