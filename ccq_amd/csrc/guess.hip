@@ -407,10 +407,7 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step(const float* __restrict
       }
     }
     __syncthreads();
-    // (rows past the batch are left out, not weighted by zero: with infinite
-    // weights they hold NaN)
-    const int ns = batch - s0 < kStepTile ? (int)(batch - s0) : kStepTile;
-    for (int s = 0; s < ns; ++s) {
+    auto add = [&](int s) {
       const float* r = rows + s * kRow;
       const float4 h = *reinterpret_cast<const float4*>(r + C_H1 + p0);
       const float4 g = *reinterpret_cast<const float4*>(r + C_G2 + q0);
@@ -422,7 +419,14 @@ __global__ __launch_bounds__(kStepThreads) void mlp_step(const float* __restrict
 #pragma unroll
       for (int x = 0; x < kExtra; ++x)
         if (ea[x] >= 0) ext[x] += (double)r[ea[x]] * (double)r[eb[x]];
-    }
+    };
+    // (rows past the batch are left out, not weighted by zero: with infinite
+    // weights they hold NaN; a full pass keeps its constant length: 25 steps of
+    // 4096 samples 1009 us, with the run-time one 1027)
+    if (batch - s0 >= kStepTile)
+      for (int s = 0; s < kStepTile; ++s) add(s);
+    else
+      for (int s = 0; s < (int)(batch - s0); ++s) add(s);
   }
 
   double* out = partial + (int64_t)blockIdx.x * kGradN;
