@@ -2047,6 +2047,7 @@ struct ccq_hip_ctx {
       for (const auto& b : *bufs) shadows += sizeof(float) * (size_t)b->n;
     for (const auto& kv : resid_buf) shadows += sizeof(float) * (size_t)kv.second->n;
     HIPCHK(hipMemGetInfo(&free, &total));
+    if (shadows + kKeepFree > free) shadows = 0;   // there is no room for them either way
     return want + shadows + kKeepFree <= free;
   }
   static constexpr size_t kKeepFree = (size_t)256 << 20;   // task tables, kernels' scratch, pinned staging
