@@ -2868,8 +2868,14 @@ struct ccq_hip_ctx {
   // (an allocation of its own for each took 25 ms of a small system's set-up)
   std::map<std::pair<int, int>, int64_t> slot_off;
   int64_t slot_need = 0;
-  // FP64 in every precision mode: an FP32-storage sweep rounds a sum of
-  // partial accumulators once, when it is added to the accumulator itself
+  // The partial accumulators of an FP32-storage sweep lie in the same memory.  Up to
+  // kSlot64 elements they stay FP64, so a sum of them is rounded once, when it is
+  // added to the accumulator: such outputs take many slots and their products are
+  // the ones that a chain would have summed in FP64.  Larger ones (two slots at
+  // most) are float as their accumulators are: in FP64 their traffic made a level
+  // of CCSDT 40 orbitals with one product into one (875x6125x5) 25.6 -> 34.5 us.
+  bool slot64(int t) const { return tensor_size(t) <= kSlot64; }
+  static constexpr int64_t kSlot64 = 1 << 21;
   DevBuf slots;
   DevBuf lv_ws;
   int64_t lv_ws_need = 0;
@@ -3275,7 +3281,7 @@ struct ccq_hip_ctx {
         g.M = tensor_size(ts.tensor);
         g.N = 1;
         g.C = dst(ts.tensor, ts.kind == ccqk::kLvSum ? 0 : ts.slot);
-        g.c64 = st && ts.kind == ccqk::kLvZero;
+        g.c64 = st && slot64(ts.tensor);
         t.nsrc = ts.kind == ccqk::kLvSum ? ts.nslots - 1 : 0;
         for (int k = 0; k < t.nsrc; ++k) t.src[k] = dst(ts.tensor, k + 1);
         continue;
@@ -3304,7 +3310,7 @@ struct ccq_hip_ctx {
         if (op.M * op.N > 0x7fffffffLL) throw Fail("level add too large");
       }
       g.C = dst(ts.tensor, ts.slot);
-      g.c64 = st && ts.slot > 0;
+      g.c64 = st && ts.slot > 0 && slot64(ts.tensor);
       g.accumulate = ts.overwrite ? 0 : 1;
     }
     ccqk::LevelTask* d = nullptr;

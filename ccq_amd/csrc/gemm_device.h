@@ -823,7 +823,8 @@ __device__ __forceinline__ void level_perm(const LevelTask& t, int idx) {
     for (; b < e1; b += 512) run(b, std::integral_constant<int, 2>{});
 }
 
-// C (+)= alpha A (n = 0), or C += the sum of n arrays; whole pairs, then the last one
+// C (+)= alpha A, or C += the sum of n arrays; whole pairs, then the last one.
+// (IOC: the stored type of an add's C, of the arrays of a sum, whose C is IO)
 template <typename IO, typename IOC>
 __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
   const GemmArgs& g = t.g;
@@ -833,12 +834,13 @@ __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
   auto one = [&](int64_t e) {
     double s = add ? g.alpha * ldg<IO>(g.A, e) : 0.0;
     if (!add) {
-      s = ldg<IOC>(g.C, e);
-      for (int k = 0; k < t.nsrc; ++k) s += ldg<double>(t.src[k], e);
+      s = ldg<IO>(g.C, e);
+      for (int k = 0; k < t.nsrc; ++k) s += ldg<IOC>(t.src[k], e);
     } else if (g.accumulate) {
       s = ldg<IOC>(g.C, e) + s;
     }
-    stg<IOC>(g.C, e, s);
+    if (add) stg<IOC>(g.C, e, s);
+    else stg<IO>(g.C, e, s);
   };
   auto pairs = [&](int64_t e, auto count) {   // count pairs a thread, 512 elements apart
     constexpr int J = decltype(count)::value;
@@ -856,12 +858,12 @@ __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
     } else {
       d2 v[kMaxLevelSrc - 1][J];
 #pragma unroll
-      for (int j = 0; j < J; ++j) s[j] = ldg2<IOC>(g.C, e + 512 * j);
+      for (int j = 0; j < J; ++j) s[j] = ldg2<IO>(g.C, e + 512 * j);
 #pragma unroll
       for (int k = 0; k < kMaxLevelSrc - 1; ++k)
         if (k < t.nsrc)
 #pragma unroll
-          for (int j = 0; j < J; ++j) v[k][j] = ldg2<double>(t.src[k], e + 512 * j);
+          for (int j = 0; j < J; ++j) v[k][j] = ldg2<IOC>(t.src[k], e + 512 * j);
 #pragma unroll
       for (int k = 0; k < kMaxLevelSrc - 1; ++k)
         if (k < t.nsrc)
@@ -869,7 +871,9 @@ __device__ __forceinline__ void level_flat(const LevelTask& t, int idx) {
           for (int j = 0; j < J; ++j) s[j] += v[k][j];
     }
 #pragma unroll
-    for (int j = 0; j < J; ++j) stg2<IOC>(g.C, e + 512 * j, s[j]);
+    for (int j = 0; j < J; ++j)
+      if (add) stg2<IOC>(g.C, e + 512 * j, s[j]);
+      else stg2<IO>(g.C, e + 512 * j, s[j]);
   };
   int64_t e = e0 + 2 * threadIdx.x;
   for (; e - 2 * threadIdx.x + 1024 <= e1; e += 1024) pairs(e, std::integral_constant<int, 2>{});

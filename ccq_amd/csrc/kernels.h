@@ -53,8 +53,8 @@ struct GemmArgs {
   // LDS-tiled kernel: 2 = two 4-wave groups share a 32x32 tile and split its K
   // slabs, 1 = one group
   int ksplit = 1;
-  // C holds FP64 whatever the storage (level launches: the partial
-  // accumulators of an FP32-storage sweep)
+  // C holds FP64 whatever the storage (level launches: partial accumulators of an
+  // FP32-storage sweep; kLvSum: the arrays it adds hold FP64)
   int c64 = 0;
   // split-K workspace of at least gemm_ws_need doubles
   double* ws = nullptr;
@@ -218,7 +218,7 @@ struct LevelTask {
   int pshift;    // kLvReduce: 2^pshift threads share an element
   int nsrc;
   GemmArgs g;
-  const double* src[kMaxLevelSrc];   // FP64 in either storage
+  const double* src[kMaxLevelSrc];
 };
 struct LevelItem {
   int task, idx;   // task < 0: nothing
