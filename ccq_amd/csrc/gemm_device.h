@@ -413,8 +413,8 @@ struct TabLds {
 // sums.  The rounding of an FP32 accumulator grows with its length, so a bound of
 // the kernel's own keeps it independent of tiles and K splits, which levels
 // choose longer than a launch per product would.  The FP64 sums take 32 registers
-// in a 64 x 64 tile (some spill in the table modes: FP32-storage sweeps of CCSD 61
-// orbitals 362 -> 375 us, CCSDT 31 1131 -> 1160); two workgroups a CU without
+// in a 64 x 64 tile, and some spill in the table modes (FP32-storage sweeps of CCSD
+// 61 orbitals 362 -> 375 us, CCSDT 31 1131 -> 1160); two workgroups a CU without
 // spills are slower (428, 1282), sums of runs in FP32 too (394, 1198), and runs
 // of 128 no faster.
 constexpr int kF32Run = 64;
@@ -567,7 +567,8 @@ __device__ __forceinline__ void tile_run(const GemmArgs& g, int64_t m0, int64_t 
   }
 }
 
-template <typename T, typename IO, int BM, int BN, int BK, int KS>
+// FEW: k-contiguous tables and tables only, whatever the operands
+template <typename T, typename IO, int BM, int BN, int BK, int KS, bool FEW = false>
 __device__ __forceinline__ void tile_mma(const GemmArgs& g, int64_t m0, int64_t n0, int64_t kbeg, int64_t kend,
                                          unsigned char* smem, d4 (&acc)[BM / 32][BN / 32]) {
   // 0 contiguous, 1 strided, 2 pairs, 3 k-contiguous table, 4 table
@@ -578,6 +579,8 @@ __device__ __forceinline__ void tile_mma(const GemmArgs& g, int64_t m0, int64_t 
   const bool pa = ma == 0 || (ma == 2 && even), pb = mb == 0 || (mb == 2 && even);
 #define CCQ_RUN(a, b) tile_run<T, IO, BM, BN, BK, KS, KMode::a, KMode::b>(g, m0, n0, kbeg, kend, smem, acc)
   if (g.wide) CCQ_RUN(Wide, Wide);
+  else if (FEW && g.a_kfast && g.b_kfast) CCQ_RUN(TabK, TabK);
+  else if (FEW) CCQ_RUN(Tab, Tab);
   else if (ma < 2 && mb < 2) {
     if (ma == 0 && mb == 0) CCQ_RUN(Vec, Vec);
     else if (ma == 0) CCQ_RUN(Vec, Aff);
@@ -591,7 +594,7 @@ __device__ __forceinline__ void tile_mma(const GemmArgs& g, int64_t m0, int64_t 
 #undef CCQ_RUN
 }
 
-template <typename T, typename IO, int BM, int BN, int BK, int KS>
+template <typename T, typename IO, int BM, int BN, int BK, int KS, bool FEW = false>
 __device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty, int tz, unsigned char* smem) {
   constexpr int WM = BM / 2, WN = BN / 2;
   constexpr int TM = WM / 16, TN = WN / 16;
@@ -612,7 +615,7 @@ __device__ __forceinline__ void gemm_tab_tile(const GemmArgs& g, int tx, int ty,
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = d4{0, 0, 0, 0};
-  tile_mma<T, IO, BM, BN, BK, KS>(g, m0, n0, kbeg, kend, smem, acc);
+  tile_mma<T, IO, BM, BN, BK, KS, FEW>(g, m0, n0, kbeg, kend, smem, acc);
 
   if (KS > 1) {
     // group 1 hands its accumulators to group 0 (slab order: group 0's sum
@@ -947,31 +950,23 @@ __global__ __launch_bounds__(256, kTileWaves<1>) void level_kernel(const LevelTa
   const int tz = idx / per_z;
   int tx, ty;
   tile_in_group(idx - tz * per_z, tm, tn, g.group, tx, ty);
-  const int tile = (t.kind - kLvTile6464) & 3;
-#define CCQ_LV(A, BM, BN, TY) gemm_tab_tile<A, IO, BM, BN, tile_bk(BM, BN), 1>(g, tx, TY, tz, smem)
+#define CCQ_LV(A, FEW)                                                                         \
+  switch ((t.kind - kLvTile6464) & 3) {                                                        \
+    case 0: gemm_tab_tile<A, IO, 64, 64, tile_bk(64, 64), 1, FEW>(g, tx, ty, tz, smem); break; \
+    case 1: gemm_tab_tile<A, IO, 64, 32, tile_bk(64, 32), 1, FEW>(g, tx, ty, tz, smem); break; \
+    case 2: gemm_tab_tile<A, IO, 32, 64, tile_bk(32, 64), 1, FEW>(g, tx, ty, tz, smem); break; \
+    default: gemm_tab_tile<A, IO, 32, 32, tile_bk(32, 32), 1, FEW>(g, tx, ty, tz, smem);       \
+  }
+  // FP64 products of the FP32 modes are small or bound by memory; on FP32 storage
+  // three operand modes for them are faster than nine (CCSDTQ 14 orbitals 2534 ->
+  // 2389 us a sweep, CCSDT 40 2298 -> 2276), on FP64 storage slower (2500 -> 2515)
   if constexpr (sizeof(T) == 4) {
     if (t.kind >= kLvTileF64) {
-      // a 64 x 64 tile as two of 64 x 32, whose registers fit beside the FP32 forms'
-      if (tile == 0) {
-        CCQ_LV(double, 64, 32, 2 * ty);
-        __syncthreads();
-        CCQ_LV(double, 64, 32, 2 * ty + 1);
-      } else if (tile == 1) {
-        CCQ_LV(double, 64, 32, ty);
-      } else if (tile == 2) {
-        CCQ_LV(double, 32, 64, ty);
-      } else {
-        CCQ_LV(double, 32, 32, ty);
-      }
+      CCQ_LV(double, sizeof(IO) == 4)
       return;
     }
   }
-  switch (tile) {
-    case 0: CCQ_LV(T, 64, 64, ty); break;
-    case 1: CCQ_LV(T, 64, 32, ty); break;
-    case 2: CCQ_LV(T, 32, 64, ty); break;
-    default: CCQ_LV(T, 32, 32, ty); break;
-  }
+  CCQ_LV(T, false)
 #undef CCQ_LV
 }
 
