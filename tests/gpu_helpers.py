@@ -100,10 +100,13 @@ class Case:
 def leave_free(nbytes):
     """Tensors that take the device's memory but for about nbytes (what the driver
     reports as free is not all there after one large allocation)."""
+    import gc
     import torch
+    gc.collect()   # engines that earlier tests dropped give theirs back now, not later
     blocks = []
-    while len(blocks) < 8 and torch.cuda.mem_get_info()[0] > nbytes + (32 << 20):
+    while len(blocks) < 64 and torch.cuda.mem_get_info()[0] > nbytes + (32 << 20):
         blocks.append(torch.empty(torch.cuda.mem_get_info()[0] - nbytes, dtype=torch.uint8, device="cuda"))
+    assert torch.cuda.mem_get_info()[0] <= nbytes + (32 << 20)
     return blocks
 
 
