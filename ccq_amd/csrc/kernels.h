@@ -48,7 +48,8 @@ struct GemmArgs {
   int64_t kchunk = 0;
   int group = 1;           // tile rows per group of the XCD-aware tile order
   // arithmetic of the LDS-tiled kernel: 0 FP64 MFMA; 1 FP32 MFMA (operands
-  // rounded to FP32 when staged into LDS, FP32 accumulation, FP64 epilogue)
+  // rounded to FP32 when staged into LDS, FP32 sums of 64 summed indices added
+  // in FP64)
   int prec = 0;
   // LDS-tiled kernel: 2 = two 4-wave groups share a 32x32 tile and split its K
   // slabs, 1 = one group
