@@ -1967,7 +1967,7 @@ struct ccq_hip_ctx {
       int64_t own = 1;
       for (const auto& sec : sections)
         for (const auto& op : sec.ops)
-          if (op.gemm && own_launch(op))
+          if (op.gemm && (own_launch(op) || tensors[op.out].kind == TKind::Amp))
             own = std::max({own, ccqk::gemm_ws_need(op.plan), op.has_plan32 ? ccqk::gemm_ws_need(op.plan32) : 0});
       ws.alloc(own);
       cur_ws = ws.p;
@@ -2654,7 +2654,7 @@ struct ccq_hip_ctx {
     const int acc = op.assign ? 0 : 1;
     if (op.gemm) {
       ccqk::GemmArgs g = gemm_args(op);
-      if (run_prec && g.kind == 0 && op.K > 0 && ccqk::fp64_in_mixed(op.M, op.N, op.K)) ccqk::gemm_plan_reg(g, ws_sections.n);
+      if (run_prec && g.kind == 0 && op.K > 0 && ccqk::fp64_in_mixed(op.M, op.N, op.K)) ccqk::gemm_plan_reg(g, cur_ws == ws.p ? ws.n : ws_sections.n);
       HIPCHK(ccqk::launch_gemm(stream, g));
     } else {
       if (amp_in_fp64(1, [&](size_t) { return op.out; }, [&] { run_op(op); })) return;
