@@ -4027,6 +4027,9 @@ int ccq_hip_create(const ccq_hip_dims* dims, const ccq_hip_opts* opts, ccq_hip_c
 int ccq_hip_set_ints(ccq_hip_ctx* ctx, const double* f_a, const double* f_b, const double* v_aa,
                      const double* v_ab, const double* v_bb) {
   return guarded(ctx, [&] {
+    // the copies below do not wait for the context's stream, whose sweeps read the
+    // orbital energies
+    HIPCHK(hipStreamSynchronize(ctx->stream));
     const int64_t nc = ctx->nc, n3 = ctx->orbs, n0 = ctx->froz;
     const int64_t nc4 = nc * nc * nc * nc;
     // Fortran v(p,q,r,s) column-major -> C order [p][q][r][s]: full axis reversal
