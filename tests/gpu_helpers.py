@@ -98,7 +98,7 @@ class Case:
 
 
 def leave_free(nbytes):
-    """Tensors that take the device's memory but for about nbytes (what the driver
+    """Tensors that take the device's memory but for about nbytes (what the runtime
     reports as free is not all there after one large allocation)."""
     import gc
     import torch
